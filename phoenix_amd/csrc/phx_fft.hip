@@ -10,10 +10,10 @@
  *                           inverse FFT -- all without leaving LDS;
  *   3. fft_rows<inverse>  : inverse row FFTs.
  * Each kernel reads and writes the grid once (6 passes over N_c N_r complex).
- * Lengths 256, 512 and 1024 on both axes take the four-step kernels instead (fft4_rows,
+ * Lengths 256, 512 and 1024 take the four-step kernels instead (fft4_rows,
  * fft4_cols: N = N1 N2, sub-transforms in registers, one LDS transpose per transform, two
  * lanes per sub-sequence); other powers of two the Stockham kernels below, other even
- * lengths direct DFTs.
+ * lengths the mixed-radix kernels of phx_fft_mixed.hip.
  *
  * The transforms are unnormalised DFTs with the forward sign e^{-2 pi i jk/N}
  * (cuFFT/FFTW convention).  Algorithm: Stockham autosort, radix 4 with a final
@@ -30,22 +30,13 @@
 
 #include "custom_rhs.h"
 #include "phx_device.h"
+#include "phx_fft_cx.h"
+#include "phx_fft_mixed.h"
 #include "phx_kernels.h"
 
 namespace phx {
 
 constexpr int kFftThreads = 256;
-
-/* aligned to its full size, so an element moves with one 64-bit (FP32) / 128-bit (FP64) LDS access */
-template <typename real>
-struct alignas(2 * sizeof(real)) Cx {
-    real r, i;
-};
-
-template <typename real>
-__device__ __forceinline__ Cx<real> cmul(Cx<real> a, Cx<real> w) {
-    return {phx_fma(a.r, w.r, -(a.i * w.i)), phx_fma(a.r, w.i, a.i * w.r)};
-}
 
 /* LDS slot of element i: one spare slot after every 32 elements (PAD), so that the strided
    Stockham writes of the early passes spread over all banks instead of a few. */
@@ -169,16 +160,8 @@ __global__ __launch_bounds__(kFftThreads) void fft_rows(typename Vec2<real>::typ
     }
 }
 
-/* Column groups are handed out XCD by XCD (block b runs on XCD b % 8): consecutive
-   groups share cache lines, so they go to the same L2. */
-__device__ __forceinline__ int fft_xcd_group(int b, int nblocks) {
-    const int q = nblocks >> 3, r = nblocks & 7;
-    const int x = b & 7;
-    return x * q + (x < r ? x : r) + (b >> 3);
-}
-
 /* What the column pass does in k-space. */
-enum { kColFilter = 0, kColPropagate = 1, kColForward = 2 };
+enum { kColFilter = kFftFilter, kColPropagate = kFftPropagate, kColForward = kFftForward };
 
 /* CB adjacent columns: forward FFT along the column, a pointwise factor in k-space, inverse FFT.
    MODE kColFilter:    F <- F / (N_c N_r) * mask[shifted] (the k-space filter); with spec != nullptr
@@ -239,7 +222,8 @@ __global__ __launch_bounds__(kFftThreads) void fft_cols_filter(typename Vec2<rea
             const int i = min((int)threadIdx.x + k * kFftThreads, cnt - 1);
             const int r = i / CB, j = i - r * CB;
             const int rs = (r + (Nr >> 1)) & (Nr - 1);
-            const int cs = (c0 + j + (Nc >> 1)) & (Nc - 1);
+            int cs = c0 + j + (Nc >> 1); /* Nc need not be a power of two */
+            if (cs >= Nc) cs -= Nc;
             mk[k] = mask[(size_t)rs * Nc + cs];
         }
 #pragma unroll
@@ -479,7 +463,8 @@ __global__ __launch_bounds__(2 * CB *(N1 > N2 ? N1 : N2)) void fft4_cols(typenam
 #pragma unroll
             for (int m = 0; m < H2; m++) y[m] = cmul(cmul(y[m], cf), rowf[t + N1 * (m + p * H2)]);
         } else {
-            const int cs = (col + (Nc >> 1)) & (Nc - 1);
+            int cs = col + (Nc >> 1); /* Nc need not be a power of two */
+            if (cs >= Nc) cs -= Nc;
             real mk[H2];
 #pragma unroll
             for (int m = 0; m < H2; m++) mk[m] = mask[(size_t)(((t + N1 * (m + p * H2)) + (N >> 1)) & (N - 1)) * Nc + cs];
@@ -595,132 +580,6 @@ static hipError_t launch_fft4_cols(typename Vec2<real>::type* psi, const void* t
     }
 }
 
-/* ------------------------------------------------------------------------------------------
-   Direct DFT for lengths that are not powers of two (any even N; the reference validates even
-   grid sizes, system_validate_input.cpp:19-56): out[k] = sum_j x[j] w^((j k) mod N) with
-   w = e^(-+2 pi i / N) from the twiddle table, one output per thread and pass, the sequence in
-   LDS.  O(N) multiply-adds per output value instead of O(log N): a general-size path next to the
-   radix-4 Stockham kernels, which stay the fast path for powers of two. */
-template <typename real, int SIGN>
-__device__ __forceinline__ Cx<real> dft_one(const Cx<real>* x, int stride, const Cx<real>* __restrict__ tw, int N, int k) {
-    real sr = 0, si = 0;
-    int idx = 0;
-    for (int j = 0; j < N; j++) {
-        Cx<real> w = tw[idx];
-        if (SIGN > 0) w.i = -w.i;
-        const Cx<real> v = x[j * stride];
-        sr = phx_fma(v.r, w.r, phx_fma(-v.i, w.i, sr));
-        si = phx_fma(v.r, w.i, phx_fma(v.i, w.r, si));
-        idx += k; /* (j k) mod N, incrementally: idx + k < 2 N */
-        if (idx >= N) idx -= N;
-    }
-    return {sr, si};
-}
-
-template <typename real, int SIGN>
-__global__ __launch_bounds__(kFftThreads) void dft_rows(typename Vec2<real>::type* data, const Cx<real>* __restrict__ tw, int N) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    Cx<real>* A = reinterpret_cast<Cx<real>*>(lds_raw);
-    typename Vec2<real>::type* row = data + (size_t)blockIdx.x * (size_t)N;
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const auto v = row[i];
-        A[i] = {v.x, v.y};
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < N; k += blockDim.x) {
-        const Cx<real> f = dft_one<real, SIGN>(A, 1, tw, N, k);
-        typename Vec2<real>::type v;
-        v.x = f.r;
-        v.y = f.i;
-        row[k] = v;
-    }
-}
-
-/* CB adjacent columns: forward DFT along the column, the k-space factor (MODE as fft_cols_filter, with
-   the same optional spectrum output), inverse DFT; two LDS buffers (the transforms are out of place). */
-template <typename real, int CB, int MODE>
-__global__ __launch_bounds__(kFftThreads) void dft_cols_filter(typename Vec2<real>::type* data, const Cx<real>* __restrict__ tw,
-                                                              const real* __restrict__ mask, const Cx<real>* __restrict__ rowf,
-                                                              const Cx<real>* __restrict__ colf, int Nc, int Nr, real Ntot,
-                                                              typename Vec2<real>::type* spec) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    Cx<real>* A = reinterpret_cast<Cx<real>*>(lds_raw);
-    Cx<real>* B = A + CB * Nr;
-    const int c0 = fft_xcd_group(blockIdx.x, gridDim.x) * CB;
-    for (int i = threadIdx.x; i < CB * Nr; i += blockDim.x) {
-        const int r = i / CB, j = i - r * CB;
-        const auto v = data[(size_t)r * Nc + c0 + j];
-        A[j * Nr + r] = {v.x, v.y};
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < CB * Nr; i += blockDim.x) {
-        const int k = i / CB, j = i - k * CB;
-        Cx<real> f = dft_one<real, -1>(A + j * Nr, 1, tw, Nr, k);
-        if constexpr (MODE == kColForward) {
-            typename Vec2<real>::type o;
-            o.x = f.r;
-            o.y = f.i;
-            data[(size_t)k * Nc + c0 + j] = o; /* A holds the columns: the in-place store is safe */
-            continue;
-        } else if constexpr (MODE == kColPropagate) {
-            f = cmul(cmul(f, colf[c0 + j]), rowf[k]);
-        } else {
-            /* mask of the quadrant-swapped grid (fft_shift_2D, kernel_fft.cuh:15-32) */
-            int rs = k + (Nr >> 1), cs = c0 + j + (Nc >> 1);
-            if (rs >= Nr) rs -= Nr;
-            if (cs >= Nc) cs -= Nc;
-            const real m = mask[(size_t)rs * Nc + cs];
-            f.r = f.r / Ntot * m;
-            f.i = f.i / Ntot * m;
-            if (spec) {
-                typename Vec2<real>::type o;
-                o.x = f.r;
-                o.y = f.i;
-                spec[(size_t)k * Nc + c0 + j] = o;
-            }
-        }
-        B[j * Nr + k] = f;
-    }
-    if constexpr (MODE == kColForward) return;
-    __syncthreads();
-    for (int i = threadIdx.x; i < CB * Nr; i += blockDim.x) {
-        const int r = i / CB, j = i - r * CB;
-        const Cx<real> f = dft_one<real, +1>(B + j * Nr, 1, tw, Nr, r);
-        typename Vec2<real>::type v;
-        v.x = f.r;
-        v.y = f.i;
-        data[(size_t)r * Nc + c0 + j] = v;
-    }
-}
-
-/* sizes the direct DFT takes: even, and two column buffers of one column in 64 KiB */
-static bool dft_supported(int N, size_t real_size) { return N >= 2 && N % 2 == 0 && (size_t)N * 4 * real_size <= 65536; }
-
-template <typename real, int MODE>
-static hipError_t dft_roundtrip(typename Vec2<real>::type* psi, const void* tw_c, const void* tw_r, const real* mask, const void* rowf,
-                                const void* colf, int Nc, int Nr, hipStream_t s, typename Vec2<real>::type* spec = nullptr) {
-    const auto* twc = (const Cx<real>*)tw_c;
-    const auto* twr = (const Cx<real>*)tw_r;
-    const auto* rf = (const Cx<real>*)rowf;
-    const auto* cf = (const Cx<real>*)colf;
-    const real ntot = (real)((double)Nc * (double)Nr);
-    hipLaunchKernelGGL((dft_rows<real, -1>), dim3(Nr), dim3(kFftThreads), (size_t)Nc * sizeof(Cx<real>), s, psi, twc, Nc);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const size_t per_col = 2 * (size_t)Nr * sizeof(Cx<real>);
-    auto fits = [&](int cb) { return per_col * cb <= 65536 && Nc % cb == 0; };
-    if (fits(4))
-        hipLaunchKernelGGL((dft_cols_filter<real, 4, MODE>), dim3(Nc / 4), dim3(kFftThreads), 4 * per_col, s, psi, twr, mask, rf, cf, Nc, Nr, ntot, spec);
-    else if (fits(2))
-        hipLaunchKernelGGL((dft_cols_filter<real, 2, MODE>), dim3(Nc / 2), dim3(kFftThreads), 2 * per_col, s, psi, twr, mask, rf, cf, Nc, Nr, ntot, spec);
-    else
-        hipLaunchKernelGGL((dft_cols_filter<real, 1, MODE>), dim3(Nc), dim3(kFftThreads), per_col, s, psi, twr, mask, rf, cf, Nc, Nr, ntot, spec);
-    e = hipGetLastError();
-    if (e != hipSuccess || MODE == kColForward) return e;
-    hipLaunchKernelGGL((dft_rows<real, +1>), dim3(Nr), dim3(kFftThreads), (size_t)Nc * sizeof(Cx<real>), s, psi, twc, Nc);
-    return hipGetLastError();
-}
-
 static int ilog2(int n) {
     int l = 0;
     while ((1 << l) < n) l++;
@@ -735,7 +594,7 @@ static bool stockham_supported(int N, size_t real_size) {
     return (size_t)N * 2 * real_size <= 65536 && N / 4 <= mb * kFftThreads;
 }
 
-bool fft_supported(int N, size_t real_size) { return stockham_supported(N, real_size) || dft_supported(N, real_size); }
+bool fft_supported(int N, size_t real_size) { return stockham_supported(N, real_size) || fft_mixed_supported(N, real_size); }
 
 /* smallest power of two KB with butterflies <= KB * threads */
 static int bfly_bound(int butterflies) {
@@ -808,24 +667,11 @@ static hipError_t launch_cols(typename Vec2<real>::type* psi, const void* tw_r, 
     return launch_cols_p<real, CB, MODE, false>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
 }
 
-/* rows forward -> columns (forward, k-space factor, inverse) -> rows inverse; kColForward stops
-   after the forward column transform */
+/* columns by the Stockham kernel: as wide a block as LDS and registers allow, but no wider than
+   keeps 512 workgroups in flight (the machine has 256 CUs) */
 template <typename real, int MODE>
-static hipError_t fft_roundtrip(typename Vec2<real>::type* psi, const void* tw_c, const void* tw_r, const real* mask, const void* rowf,
-                                const void* colf, int Nc, int Nr, hipStream_t s, typename Vec2<real>::type* spec = nullptr) {
-    int n1, n2;
-    if (fft4_enabled() && fft4_split(Nc, n1, n2) && fft4_split(Nr, n1, n2) && Nc % (kFft4Threads / 32) == 0) {
-        /* both row kernels leave each row transformed in natural order, in place */
-        const bool rows4 = fft4_rows_enabled();
-        hipError_t e = rows4 ? launch_fft4_rows<real, -1>(psi, tw_c, Nc, Nr, s) : launch_rows<real, -1>(psi, tw_c, Nc, Nr, s);
-        if (e == hipSuccess) e = launch_fft4_cols<real, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-        if (e != hipSuccess || MODE == kColForward) return e;
-        return rows4 ? launch_fft4_rows<real, +1>(psi, tw_c, Nc, Nr, s) : launch_rows<real, +1>(psi, tw_c, Nc, Nr, s);
-    }
-    hipError_t e = launch_rows<real, -1>(psi, tw_c, Nc, Nr, s);
-    if (e != hipSuccess) return e;
-    /* column block width: as wide as LDS and registers allow, but no wider than keeps
-       512 workgroups in flight (the machine has 256 CUs) */
+static hipError_t launch_stockham_cols(typename Vec2<real>::type* psi, const void* tw, const real* mask, const void* rowf,
+                                       const void* colf, int Nc, int Nr, hipStream_t s, typename Vec2<real>::type* spec) {
     const size_t per_col = (size_t)Nr * sizeof(Cx<real>);
     auto fits = [&](int cb) {
         return per_col * cb <= 65536 && Nc % cb == 0 && cb * (Nr / 4) <= max_bfly<real>() * kFftThreads && (cb == 1 || Nc / cb >= 512);
@@ -835,57 +681,74 @@ static hipError_t fft_roundtrip(typename Vec2<real>::type* psi, const void* tw_c
     auto fits_env = [&](int cb) {
         return cb_env == cb && per_col * cb <= 65536 && Nc % cb == 0 && cb * (Nr / 4) <= max_bfly<real>() * kFftThreads;
     };
-    if (fits_env(8))
-        e = launch_cols<real, 8, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    else if (fits_env(4))
-        e = launch_cols<real, 4, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    else if (fits_env(1))
-        e = launch_cols<real, 1, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    else if (fits(8))
-        e = launch_cols<real, 8, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    else if (fits(4))
-        e = launch_cols<real, 4, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    else if (fits(2))
-        e = launch_cols<real, 2, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    else
-        e = launch_cols<real, 1, MODE>(psi, tw_r, mask, rowf, colf, Nc, Nr, s, spec);
-    if (e != hipSuccess || MODE == kColForward) return e;
-    return launch_rows<real, +1>(psi, tw_c, Nc, Nr, s);
+    if (fits_env(8)) return launch_cols<real, 8, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
+    if (fits_env(4)) return launch_cols<real, 4, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
+    if (fits_env(1)) return launch_cols<real, 1, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
+    if (fits(8)) return launch_cols<real, 8, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
+    if (fits(4)) return launch_cols<real, 4, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
+    if (fits(2)) return launch_cols<real, 2, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
+    return launch_cols<real, 1, MODE>(psi, tw, mask, rowf, colf, Nc, Nr, s, spec);
 }
 
-/* powers of two on both axes: Stockham kernels; otherwise the direct DFT kernels for both axes */
+/* one pass over the rows or the columns, each axis by the kernel of its own length: four-step for 256,
+   512 and 1024 (columns: where a whole number of column blocks fits the row), Stockham for the other
+   powers of two, mixed radix for the rest and for FP32 columns of 2048 points and more (a filter of 2048^2
+   FP32: 87 us instead of 117, 1024 x 2048 55 / 61, 512 x 8192 136 / 163, 4096^2 479 / 481; FP64 columns are
+   no faster there: 2048^2 145 / 135) */
+template <typename real, int SIGN>
+static hipError_t rows_pass(typename Vec2<real>::type* psi, const FftAxis& c, int Nr, hipStream_t s) {
+    int n1, n2;
+    if (fft4_enabled() && fft4_rows_enabled() && fft4_split(c.N, n1, n2)) return launch_fft4_rows<real, SIGN>(psi, c.table, c.N, Nr, s);
+    if (stockham_supported(c.N, sizeof(real))) return launch_rows<real, SIGN>(psi, c.table, c.N, Nr, s);
+    return launch_mixed_rows<real>(psi, c, Nr, SIGN > 0, s);
+}
+
+template <typename real, int MODE>
+static hipError_t cols_pass(typename Vec2<real>::type* psi, const FftAxis& r, int Nc, const real* mask, const void* rowf,
+                            const void* colf, hipStream_t s, typename Vec2<real>::type* spec) {
+    int n1, n2;
+    if (fft4_enabled() && fft4_split(r.N, n1, n2) && Nc % (kFft4Threads / (2 * (n1 > n2 ? n1 : n2))) == 0)
+        return launch_fft4_cols<real, MODE>(psi, r.table, mask, rowf, colf, Nc, r.N, s, spec);
+    if (stockham_supported(r.N, sizeof(real)) && (sizeof(real) == 8 || r.N < 2048))
+        return launch_stockham_cols<real, MODE>(psi, r.table, mask, rowf, colf, Nc, r.N, s, spec);
+    return launch_mixed_cols<real>(psi, r, Nc, MODE, mask, rowf, colf, spec, s);
+}
+
+/* rows forward -> columns (forward, k-space factor, inverse) -> rows inverse; kColForward stops
+   after the forward column transform */
+template <typename real, int MODE>
+static hipError_t fft_roundtrip(typename Vec2<real>::type* psi, const FftAxis& c, const FftAxis& r, const real* mask, const void* rowf,
+                                const void* colf, hipStream_t s, typename Vec2<real>::type* spec = nullptr) {
+    if (!fft_supported(c.N, sizeof(real)) || !fft_supported(r.N, sizeof(real))) return hipErrorInvalidValue;
+    hipError_t e = rows_pass<real, -1>(psi, c, r.N, s);
+    if (e == hipSuccess) e = cols_pass<real, MODE>(psi, r, c.N, mask, rowf, colf, s, spec);
+    if (e != hipSuccess || MODE == kColForward) return e;
+    return rows_pass<real, +1>(psi, c, r.N, s);
+}
+
 template <typename real>
-hipError_t launch_fft_filter(typename Vec2<real>::type* psi, const void* tw_c, const void* tw_r, const real* mask, int Nc, int Nr,
-                             hipStream_t s, typename Vec2<real>::type* spec) {
-    if (stockham_supported(Nc, sizeof(real)) && stockham_supported(Nr, sizeof(real)))
-        return fft_roundtrip<real, kColFilter>(psi, tw_c, tw_r, mask, nullptr, nullptr, Nc, Nr, s, spec);
-    if (!fft_supported(Nc, sizeof(real)) || !fft_supported(Nr, sizeof(real))) return hipErrorInvalidValue;
-    return dft_roundtrip<real, kColFilter>(psi, tw_c, tw_r, mask, nullptr, nullptr, Nc, Nr, s, spec);
+hipError_t launch_fft_filter(typename Vec2<real>::type* psi, const FftAxis& c, const FftAxis& r, const real* mask, hipStream_t s,
+                             typename Vec2<real>::type* spec) {
+    return fft_roundtrip<real, kColFilter>(psi, c, r, mask, nullptr, nullptr, s, spec);
 }
 
 /* the unnormalised forward 2D transform of the grid, in place */
 template <typename real>
-hipError_t launch_fft_forward(typename Vec2<real>::type* data, const void* tw_c, const void* tw_r, int Nc, int Nr, hipStream_t s) {
-    if (stockham_supported(Nc, sizeof(real)) && stockham_supported(Nr, sizeof(real)))
-        return fft_roundtrip<real, kColForward>(data, tw_c, tw_r, nullptr, nullptr, nullptr, Nc, Nr, s);
-    if (!fft_supported(Nc, sizeof(real)) || !fft_supported(Nr, sizeof(real))) return hipErrorInvalidValue;
-    return dft_roundtrip<real, kColForward>(data, tw_c, tw_r, nullptr, nullptr, nullptr, Nc, Nr, s);
+hipError_t launch_fft_forward(typename Vec2<real>::type* data, const FftAxis& c, const FftAxis& r, hipStream_t s) {
+    return fft_roundtrip<real, kColForward>(data, c, r, nullptr, nullptr, nullptr, s);
 }
 
 template <typename real>
-hipError_t launch_fft_propagate(typename Vec2<real>::type* psi, const void* tw_c, const void* tw_r, const void* rowf, const void* colf,
-                                int Nc, int Nr, hipStream_t s) {
-    if (stockham_supported(Nc, sizeof(real)) && stockham_supported(Nr, sizeof(real)))
-        return fft_roundtrip<real, kColPropagate>(psi, tw_c, tw_r, nullptr, rowf, colf, Nc, Nr, s);
-    if (!fft_supported(Nc, sizeof(real)) || !fft_supported(Nr, sizeof(real))) return hipErrorInvalidValue;
-    return dft_roundtrip<real, kColPropagate>(psi, tw_c, tw_r, nullptr, rowf, colf, Nc, Nr, s);
+hipError_t launch_fft_propagate(typename Vec2<real>::type* psi, const FftAxis& c, const FftAxis& r, const void* rowf, const void* colf,
+                                hipStream_t s) {
+    return fft_roundtrip<real, kColPropagate>(psi, c, r, nullptr, rowf, colf, s);
 }
 
-template hipError_t launch_fft_propagate<float>(float2*, const void*, const void*, const void*, const void*, int, int, hipStream_t);
-template hipError_t launch_fft_propagate<double>(double2*, const void*, const void*, const void*, const void*, int, int, hipStream_t);
-template hipError_t launch_fft_filter<float>(float2*, const void*, const void*, const float*, int, int, hipStream_t, float2*);
-template hipError_t launch_fft_filter<double>(double2*, const void*, const void*, const double*, int, int, hipStream_t, double2*);
-template hipError_t launch_fft_forward<float>(float2*, const void*, const void*, int, int, hipStream_t);
-template hipError_t launch_fft_forward<double>(double2*, const void*, const void*, int, int, hipStream_t);
+template hipError_t launch_fft_propagate<float>(float2*, const FftAxis&, const FftAxis&, const void*, const void*, hipStream_t);
+template hipError_t launch_fft_propagate<double>(double2*, const FftAxis&, const FftAxis&, const void*, const void*, hipStream_t);
+template hipError_t launch_fft_filter<float>(float2*, const FftAxis&, const FftAxis&, const float*, hipStream_t, float2*);
+template hipError_t launch_fft_filter<double>(double2*, const FftAxis&, const FftAxis&, const double*, hipStream_t, double2*);
+template hipError_t launch_fft_forward<float>(float2*, const FftAxis&, const FftAxis&, hipStream_t);
+template hipError_t launch_fft_forward<double>(double2*, const FftAxis&, const FftAxis&, hipStream_t);
 
 } // namespace phx

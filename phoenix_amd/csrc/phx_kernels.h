@@ -278,21 +278,21 @@ inline int rk_generic_waves(RkTableau tab, int Nc, int Nr, int ty = kRkGenMinTil
 }
 
 /* k-space filter psi <- IDFT(DFT(psi) / (N_c N_r) * fftshift(mask)), in place.
-   tw_c / tw_r: forward twiddle tables exp(-2 pi i k / N) for k < N (complex, real
-   precision) of the row length N_c and column length N_r. */
+   c / r: the row axis (length N_c) and the column axis (length N_r), phx_fft_mixed.h. */
+struct FftAxis;
 template <typename real>
-hipError_t launch_fft_filter(typename Vec2<real>::type* psi, const void* tw_c, const void* tw_r, const real* mask, int Nc, int Nr,
-                             hipStream_t s, typename Vec2<real>::type* spec = nullptr);
+hipError_t launch_fft_filter(typename Vec2<real>::type* psi, const FftAxis& c, const FftAxis& r, const real* mask, hipStream_t s,
+                             typename Vec2<real>::type* spec = nullptr);
 /* The filter above also stores the filtered spectrum DFT(psi) / (N_c N_r) * fftshift(mask) in spec
    (row-major, k = 0 first) when spec != nullptr.  launch_fft_forward: DFT(data) in place. */
 template <typename real>
-hipError_t launch_fft_forward(typename Vec2<real>::type* data, const void* tw_c, const void* tw_r, int Nc, int Nr, hipStream_t s);
+hipError_t launch_fft_forward(typename Vec2<real>::type* data, const FftAxis& c, const FftAxis& r, hipStream_t s);
 
 /* Split-step linear propagator in place: psi <- IDFT(DFT(psi) * colf[c] * rowf[r]), with the
    separable complex factors rowf (N_r), colf (N_c) computed on the host (they carry 1/(N_c N_r)). */
 template <typename real>
-hipError_t launch_fft_propagate(typename Vec2<real>::type* psi, const void* tw_c, const void* tw_r, const void* rowf, const void* colf,
-                                int Nc, int Nr, hipStream_t s);
+hipError_t launch_fft_propagate(typename Vec2<real>::type* psi, const FftAxis& c, const FftAxis& r, const void* rowf, const void* colf,
+                                hipStream_t s);
 
 /* Pointwise parts of the split-step Fourier iterator (phx_ssfm.hip).  Index 0 = plus, 1 = minus. */
 template <typename real>
@@ -321,7 +321,7 @@ hipError_t launch_ssfm_nonlinear(const SsfmArgs<real>& a, hipStream_t s);
 template <typename real>
 hipError_t launch_ssfm_independent(const SsfmArgs<real>& a, hipStream_t s);
 
-/* Power of two in [4, 4096] whose two LDS row buffers fit in 64 KiB. */
+/* Lengths the transforms take: powers of two up to 8192 (FP32) / 4096 (FP64), other even lengths up to half that. */
 bool fft_supported(int N, size_t real_size);
 
 } // namespace phx

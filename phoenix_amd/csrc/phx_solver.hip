@@ -24,6 +24,7 @@
 
 #include "../../include/phx.h"
 #include "phx_config.hpp"
+#include "phx_fft_mixed.h"
 #include "phx_kernels.h"
 
 namespace {
@@ -72,8 +73,7 @@ struct phx_solver {
     void* pump[2] = {nullptr, nullptr};
     void* pot[2] = {nullptr, nullptr};
     void* mask[2] = {nullptr, nullptr};
-    void* tw_c = nullptr; /* forward FFT twiddles of the row length N_c */
-    void* tw_r = nullptr; /* ... and of the column length N_r */
+    phx::FftAxis fft_c, fft_r; /* transforms along the rows (length N_c) and the columns (length N_r) */
     void* noise = nullptr;      /* noise field of the current step (complex, real precision) */
     double* norm_partials = nullptr; /* imaginary-time normalisation: per-block sums, reduced sums */
     double* norm_sums = nullptr;
@@ -290,13 +290,11 @@ int initialize_t(phx_solver* s) {
         if (int r = dev_alloc(s, &s->ssfm_colf, 2 * (size_t)c.N_c * sizeof(real))) return r;
     }
     if (c.use_fft_mask || s->ssfm || s->spec[0]) {
-        for (int d = 0; d < 2; d++) {
-            const int L = d == 0 ? c.N_c : c.N_r;
-            std::vector<std::complex<double>> w(L);
-            for (int k = 0; k < L; k++) w[k] = std::polar(1.0, -2.0 * M_PI * (double)k / (double)L);
-            void** slot = d == 0 ? &s->tw_c : &s->tw_r;
-            if (int r = dev_alloc(s, slot, 2 * L * sizeof(real))) return r;
-            if (int r = upload_complex<real>(s, *slot, w)) return r;
+        for (phx::FftAxis* ax : {&s->fft_c, &s->fft_r}) {
+            *ax = phx::fft_axis(ax == &s->fft_c ? c.N_c : c.N_r);
+            const auto table = phx::fft_axis_table(*ax);
+            if (int r = dev_alloc(s, &ax->table, 2 * table.size() * sizeof(real))) return r;
+            if (int r = upload_complex<real>(s, ax->table, table)) return r;
         }
     }
 
@@ -587,11 +585,11 @@ int rk_attempt(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
 template <typename real>
 int fft_filter_t(phx_solver* s) {
     auto& c = s->cfg;
-    if (!s->tw_c || !s->tw_r) return fail(PHX_ERR_STATE, "no FFT mask in this configuration");
+    if (!s->fft_c.table || !s->fft_r.table) return fail(PHX_ERR_STATE, "no FFT mask in this configuration");
     using v2 = typename phx::Vec2<real>::type;
     for (int k = 0; k < (c.tetm ? 2 : 1); k++)
-        PHX_HIP(phx::launch_fft_filter<real>((v2*)s->psi[k][s->cur], s->tw_c, s->tw_r, (const real*)s->mask[k], c.N_c, c.N_r,
-                                             s->stream, (v2*)s->spec[k]));
+        PHX_HIP(phx::launch_fft_filter<real>((v2*)s->psi[k][s->cur], s->fft_c, s->fft_r, (const real*)s->mask[k], s->stream,
+                                             (v2*)s->spec[k]));
     s->spec_raw = false;
     return PHX_OK;
 }
@@ -612,7 +610,7 @@ int spectrum_ready_t(phx_solver* s) {
     if (!s->spec_raw) return PHX_OK;
     using v2 = typename phx::Vec2<real>::type;
     for (int k = 0; k < 2; k++)
-        if (s->spec[k]) PHX_HIP(phx::launch_fft_forward<real>((v2*)s->spec[k], s->tw_c, s->tw_r, s->cfg.N_c, s->cfg.N_r, s->stream));
+        if (s->spec[k]) PHX_HIP(phx::launch_fft_forward<real>((v2*)s->spec[k], s->fft_c, s->fft_r, s->stream));
     s->spec_raw = false;
     return PHX_OK;
 }
@@ -692,10 +690,10 @@ int ssfm_step(phx_solver* s, double t_pre) {
     a.dt = (real)s->dt;
     a.ph = phys_of<real>(s);
     for (int k = 0; k < ncomp; k++)
-        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->tw_c, s->tw_r, s->ssfm_rowf, s->ssfm_colf, c.N_c, c.N_r, s->stream));
+        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->fft_c, s->fft_r, s->ssfm_rowf, s->ssfm_colf, s->stream));
     PHX_HIP(phx::launch_ssfm_nonlinear<real>(a, s->stream));
     for (int k = 0; k < ncomp; k++)
-        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->tw_c, s->tw_r, s->ssfm_rowf, s->ssfm_colf, c.N_c, c.N_r, s->stream));
+        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->fft_c, s->fft_r, s->ssfm_rowf, s->ssfm_colf, s->stream));
     PHX_HIP(phx::launch_ssfm_independent<real>(a, s->stream));
     return PHX_OK;
 }
