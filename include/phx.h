@@ -79,8 +79,10 @@ typedef struct {
     int64_t rejected;           /* rejected adaptive attempts so far */
     int32_t tile_rows;          /* output rows per wavefront tile of the fused RK4 kernel (0 before the first step) */
     int32_t prefetch_rows;      /* rows it loads ahead of use */
-    int32_t staged;             /* 1: the stage-by-stage path runs the step (K's in HBM: pulses, several
-                                   non-constant temporal groups, complex potential envelopes, DP85, NSRK78) */
+    int32_t staged;             /* 1: a step that the plain fused kernels do not take (pulses, several
+                                   non-constant temporal groups, complex potential envelopes, DP85, NSRK78): run
+                                   stage by stage with the K's in HBM, or, for RK4 under sources of at most two
+                                   temporal groups, by the fused chain kernel */
     int64_t multi_step_steps;   /* fixed RK4 steps taken by the multi-step kernel (phx_step and
                                    phx_run_interval run constant-source stretches that way, up to 500 steps
                                    per launch; PHX_RK4_FLOW=0: never) */

@@ -177,6 +177,25 @@ struct RkGenArgs {
 
 template <typename real>
 hipError_t launch_rk_generic(const RkGenArgs<real>& a, RkTableau tab, hipStream_t s);
+
+/* Sources of the chain kernel (phx_rk_chain.hip): RK4 under chains of at most kChainGroups temporal groups
+   per source.  Group g of a source is the full-grid field at g N; its amplitude at stage s is
+   a_g(t)(1 - c_s) + c_s a_g(t + dt), the potential's and the pulse's divided by hbar.  The pumps and
+   potentials are RkGenArgs::pump / pot, the other members of which keep their meaning. */
+constexpr int kChainGroups = 2, kChainStages = 4;
+template <typename real>
+struct RkChainArgs {
+    using v2 = typename Vec2<real>::type;
+    const v2* pulse[2];
+    int npump, npot, npulse;
+    real pump_amp[kChainStages][kChainGroups];
+    v2 pot_amp_h[kChainStages][kChainGroups];
+    v2 pulse_amp_h[kChainStages][kChainGroups];
+};
+/* whether the chain kernel takes a grid with that many groups of its largest source */
+bool rk_chain_supported(int Nc, int Nr, int groups, size_t real_size);
+template <typename real>
+hipError_t launch_rk_chain(const RkGenArgs<real>& a, const RkChainArgs<real>& ch, hipStream_t s);
 /* groups of tableaux instantiated in their own translation units (1-3, 3-4 and 6 stages) */
 template <typename real>
 hipError_t launch_rk_tab3(const RkGenArgs<real>& a, RkTableau tab, hipStream_t s);
@@ -186,6 +205,10 @@ template <typename real>
 hipError_t launch_rk_tab6(const RkGenArgs<real>& a, RkTableau tab, hipStream_t s);
 template <typename real>
 hipError_t launch_rk_tab6f(const RkGenArgs<real>& a, RkTableau tab, hipStream_t s);
+/* RK4 with noise or TE-TM (phx_rk_tab4.hip), and its tile height for a grid */
+template <typename real>
+hipError_t launch_rk4_generic(const RkGenArgs<real>& a, hipStream_t s);
+int rk4_generic_tile_rows(int Nc, int Nr);
 /* adaptive DP45, TE-TM, FP32, tile height 32 (phx_rk_dp45t.hip) */
 hipError_t launch_dp45_tetm_tall(const RkGenArgs<float>& a, int ty, hipStream_t s);
 /* tile height of the adaptive DP45 kernel for a grid: the height among the compiled ones that

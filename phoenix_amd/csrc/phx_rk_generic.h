@@ -26,6 +26,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "custom_rhs.h"
 #include "phx_device.h"
 #include "phx_kernels.h"
@@ -48,9 +50,12 @@ hipError_t launch_reduce_partials(const double* partials, int nwaves, double* su
    branches: halo lanes, lanes and rows outside a zero-BC domain load through out-of-range
    offsets (0) and store through them (dropped); rows past the last grid row skip their store
    with a wave-uniform branch. */
-/* POT = false: no potential (the potential's loads and descriptors compiled out; a.pot must be null) */
-template <typename real, typename TAB, int TY, bool TETM, bool RES, bool STOCH, bool POT = true>
-__global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
+/* POT = false: no potential (the potential's loads and descriptors compiled out; a.pot must be null).
+   NG > 0: sources are chains of up to NG temporal groups each (RkChainArgs): real pumps, potentials with a
+   complex amplitude and complex pulses; group g of a source is one full-grid field after the other, a
+   group that a source does not have reads 0 beyond its descriptor. */
+template <typename real, typename TAB, int TY, bool TETM, bool RES, bool STOCH, bool POT, int NG>
+__device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const RkChainArgs<real>& ch) {
     using v2 = typename Vec2<real>::type;
     constexpr int S = TAB::S;
     constexpr int H = S;          /* halo = number of K evaluations */
@@ -85,14 +90,16 @@ __global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
     const uint32_t row_c = (uint32_t)Nc * (uint32_t)sizeof(v2);
     const uint32_t all_r = row_r * (uint32_t)Nr, all_c = row_c * (uint32_t)Nr;
     rsrc_t d_psi[NC], d_n[NC], d_p[NC], d_v[NC], o_psi[NC], o_n[NC];
+    rsrc_t d_f[NC];
     const rsrc_t d_xi = row_rsrc(a.noise, STOCH ? all_c : 0u);
     const RowWrap wrap = make_row_wrap(Nr, H);
 #pragma unroll
     for (int k = 0; k < NC; k++) {
         d_psi[k] = row_rsrc(a.psi_in[k], all_c);
         d_n[k] = row_rsrc(a.n_in[k], RES ? all_r : 0u);
-        d_p[k] = row_rsrc(a.pump[k], a.pump[k] ? all_r : 0u);
-        d_v[k] = row_rsrc(a.pot[k], a.pot[k] ? all_r : 0u);
+        d_p[k] = row_rsrc(a.pump[k], a.pump[k] ? (NG ? (uint32_t)ch.npump : 1u) * all_r : 0u);
+        d_v[k] = row_rsrc(a.pot[k], a.pot[k] ? (NG ? (uint32_t)ch.npot : 1u) * all_r : 0u);
+        if constexpr (NG > 0) d_f[k] = row_rsrc(ch.pulse[k], ch.pulse[k] ? (uint32_t)ch.npulse * all_c : 0u);
         o_psi[k] = row_rsrc(a.psi_out[k], all_c);
         o_n[k] = row_rsrc(a.n_out[k], RES ? all_r : 0u);
     }
@@ -107,7 +114,9 @@ __global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
     const real dti = a.imag ? -dt : real(0);
 
     /* per component, per extended row */
-    real p0r[NC][E], p0i[NC][E], n0[NC][E], pp[NC][E], vv[NC][E];
+    constexpr int G = NG > 0 ? NG : 1;
+    real p0r[NC][E], p0i[NC][E], n0[NC][E], pp[NC][G][E], vv[NC][G][E];
+    real fr[NC][G][E], fi[NC][G][E]; /* pulse fields (NG > 0) */
     real Kr[NC][S][E], Ki[NC][S][E], Kn[NC][S][E];
     real Yr[NC][S][E], Yi[NC][S][E], Yn[NC][S][E]; /* Y[s] = input of stage s+1, s = 0..S-2 */
     real xr[E], xi[E], sg[E];                      /* noise xi and its amplitude sqrt((R n0 + gc)/(4 dV)) */
@@ -124,8 +133,17 @@ __global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
             p0r[k][r] = v.x;
             p0i[k][r] = v.y;
             n0[k][r] = RES ? load_real_s<real>(d_n[k], vr, 0u) : real(0);
-            pp[k][r] = load_real_s<real>(d_p[k], vr, 0u);
-            vv[k][r] = POT ? load_real_s<real>(d_v[k], vr, 0u) : real(0);
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                /* group g's field follows the earlier ones; kOutOfRange plus it stays out of range */
+                pp[k][g][r] = load_real_s<real>(d_p[k], vr + (uint32_t)g * all_r, 0u);
+                vv[k][g][r] = POT ? load_real_s<real>(d_v[k], vr + (uint32_t)g * all_r, 0u) : real(0);
+                if constexpr (NG > 0) {
+                    const v2 f = load_cplx_s<real>(d_f[k], vc + (uint32_t)g * all_c, 0u);
+                    fr[k][g][r] = f.x;
+                    fi[k][g][r] = f.y;
+                }
+            }
         }
         if (STOCH) {
             /* this step's noise field (launch_noise_field); 0 outside a zero-BC domain */
@@ -162,8 +180,22 @@ __global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
 #pragma unroll
         for (int k = 0; k < NC; k++) {
             const real nv = RES ? in_n(k, s, e) : real(0);
-            const real pmp = pp[k][e] * pamp;
-            const real poth = POT ? vv[k][e] * vamp_h : real(0);
+            real pmp, poth, vih = 0, sr_ = 0, si_ = 0;
+            if constexpr (NG > 0) {
+                pmp = poth = real(0);
+#pragma unroll
+                for (int g = 0; g < NG; g++) {
+                    pmp = phx_fma(pp[k][g][e], ch.pump_amp[s][g], pmp);
+                    poth = phx_fma(vv[k][g][e], ch.pot_amp_h[s][g].x, poth);
+                    vih = phx_fma(vv[k][g][e], ch.pot_amp_h[s][g].y, vih);
+                    const v2 am = ch.pulse_amp_h[s][g];
+                    sr_ = phx_fma(fr[k][g][e], am.x, phx_fma(-fi[k][g][e], am.y, sr_));
+                    si_ = phx_fma(fr[k][g][e], am.y, phx_fma(fi[k][g][e], am.x, si_));
+                }
+            } else {
+                pmp = pp[k][0][e] * pamp;
+                poth = POT ? vv[k][0][e] * vamp_h : real(0);
+            }
             real kr, ki, kn;
             if constexpr (TETM) {
                 /* cross term of the other component o (kernel_gp_compute.cuh:123-130):
@@ -185,6 +217,12 @@ __global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
                 const real tr = phx_fma(ph.kin_x, ewr[k], ph.kin_y * nsr[k]);
                 const real ti = phx_fma(ph.kin_x, ewi[k], ph.kin_y * nsi[k]);
                 phx_rhs_scalar<real>(ph, cr_[k], ci_[k], tr, ti, nv, pmp, poth, kr, ki, kn);
+            }
+            if constexpr (NG > 0) {
+                /* imaginary part of a complex potential, (1/hbar)(i V_im)(-i psi) = V_im/hbar psi, and the pulse
+                   + (1/hbar) sum_g F_g a_g(w) (kernel_gp_compute.cuh:89-100) */
+                kr = phx_fma(vih, cr_[k], kr) + sr_;
+                ki = phx_fma(vih, ci_[k], ki) + si_;
             }
             if (STOCH) {
                 /* stochastic corrections of the RHS (kernel_gp_compute.cuh:83-85,106-108):
@@ -317,6 +355,11 @@ __global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
             a.partials[2 * gw + 1] = ns;
         }
     }
+}
+
+template <typename real, typename TAB, int TY, bool TETM, bool RES, bool STOCH, bool POT = true>
+__global__ __launch_bounds__(256) void rk_generic_fused(RkGenArgs<real> a) {
+    rk_generic_tile<real, TAB, TY, TETM, RES, STOCH, POT, 0>(a, RkChainArgs<real>{});
 }
 
 /* ---------------------------------------------------------------- launch */

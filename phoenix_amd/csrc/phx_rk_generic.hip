@@ -138,17 +138,41 @@ hipError_t launch_noise_field(typename Vec2<real>::type* xi, int Nc, int Nr, uin
 template hipError_t launch_noise_field<float>(float2*, int, int, uint64_t, uint64_t, float, hipStream_t);
 template hipError_t launch_noise_field<double>(double2*, int, int, uint64_t, uint64_t, double, hipStream_t);
 
-int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr) {
-    if (!(tetm && fp32)) return kRkGenMinTileRows; /* the tall tiles exist for the FP32 spinor kernel */
-    const char* e = std::getenv("PHX_GEN_TY"); /* read at every launch: tests switch it within a process */
-    const int env_ty = e ? std::atoi(e) : 0;
-    if (env_ty == 16 || env_ty == 32) return env_ty;
+static int device_simds() {
     static const int simds = [] {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             cus = 256;
         return 4 * std::max(cus, 1);
     }();
+    return simds;
+}
+
+int rk4_generic_tile_rows(int Nc, int Nr) {
+    if (const char* e = std::getenv("PHX_RK4G_TY")) return std::atoi(e); /* 4, 8 or 16 */
+    /* The model of dp45_adaptive_tile_rows for four stages: rounds of tiles over the SIMDs x row evaluations
+       of a tile.  A tile's rows are a serial chain, so a grid that does not fill the chip wants short tiles,
+       and a large one tall tiles, which recompute fewer halo rows.  TE-TM, us per step alone / with two other
+       grids in flight, 4, 8 and 16 rows (the rule's choice in brackets): 200^2 FP64 [12.5 / 4.4] 16 / 5.6
+       26 / 8.9; 480 x 640 FP64 24 / 16.7 [19 / 13.6] 29 / 13.5; 1200^2 FP64 75 / 85 64 / 66 [60 / 57];
+       one-component chain kernel at 512 x 384 FP32 [8.4 / 3.4] 8.8 / 3.5 12.1 / 4.7. */
+    constexpr int S = 4;
+    int best = 16;
+    long best_cost = -1;
+    for (int ty : {16, 8, 4}) {
+        const long waves = (long)((Nc + 55) / 56) * ((Nr + ty - 1) / ty);
+        const long cost = ((waves + device_simds() - 1) / device_simds()) * (long)(S * (ty + 2 * S) - S * (S + 1));
+        if (best_cost < 0 || cost < best_cost) best = ty, best_cost = cost;
+    }
+    return best;
+}
+
+int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr) {
+    if (!(tetm && fp32)) return kRkGenMinTileRows; /* the tall tiles exist for the FP32 spinor kernel */
+    const char* e = std::getenv("PHX_GEN_TY"); /* read at every launch: tests switch it within a process */
+    const int env_ty = e ? std::atoi(e) : 0;
+    if (env_ty == 16 || env_ty == 32) return env_ty;
+    const int simds = device_simds();
     /* One wave per SIMD at the kernel's register count (over 256 VGPRs + AGPRs at every height),
        and about the same VALU work per row evaluation at every height (145-148 instructions): a
        SIMD's time is its number of tiles (rounded up) times the row evaluations of one tile,
@@ -170,7 +194,7 @@ int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr) {
 template <typename real>
 hipError_t launch_rk_generic(const RkGenArgs<real>& a, RkTableau tab, hipStream_t s) {
     switch (tab) {
-        case RkTableau::RK4: return launch_tab<real, TabRK4>(a, s);
+        case RkTableau::RK4: return launch_rk4_generic<real>(a, s);
         case RkTableau::DP45_FIXED: return launch_tab<real, TabDP45Fixed>(a, s);
         case RkTableau::DP45_ADAPTIVE: {
             const int ty = dp45_adaptive_tile_rows(a.tetm, sizeof(real) == 4, a.Nc, a.Nr);

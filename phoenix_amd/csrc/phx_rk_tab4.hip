@@ -1,10 +1,22 @@
 /*
  * phx_rk_tab4.hip -- instantiations of the fused Runge-Kutta kernel (phx_rk_generic.h) for the
- * three- and four-stage iterators (Fehlberg 2(1) fixed and adaptive, Ralston4, Rule38, Bogacki-Shampine 3(2) fixed and adaptive).
+ * three- and four-stage iterators (RK4 with noise or TE-TM, Fehlberg 2(1) fixed and adaptive, Ralston4, Rule38, Bogacki-Shampine 3(2) fixed and adaptive).
  */
 #include "phx_rk_generic.h"
 
 namespace phx {
+
+template <typename real>
+hipError_t launch_rk4_generic(const RkGenArgs<real>& a, hipStream_t s) {
+    switch (rk4_generic_tile_rows(a.Nc, a.Nr)) {
+        case 4: return dispatch_flags<real, TabRK4, 4>(a, s);
+        case 8: return dispatch_flags<real, TabRK4, 8>(a, s);
+        default: return launch_tab<real, TabRK4>(a, s);
+    }
+}
+
+template hipError_t launch_rk4_generic<float>(const RkGenArgs<float>&, hipStream_t);
+template hipError_t launch_rk4_generic<double>(const RkGenArgs<double>&, hipStream_t);
 
 template <typename real>
 hipError_t launch_rk_tab4(const RkGenArgs<real>& a, RkTableau tab, hipStream_t s) {

@@ -108,6 +108,7 @@ struct phx_solver {
     bool flow_off = false;
     /* staged path (phx_staged.hip): padded stage input and K slots, per-group source fields */
     bool staged = false;
+    bool chain = false;   /* ... with the chain kernel in place of the stages in HBM (phx_rk_chain.hip) */
     bool grouped = false; /* one source field per temporal group (staged path, SSFM with chains or pulses) */
     /* k-space spectra kept for output (the reference's fft_plus / fft_minus): the filtered spectrum
        of the last filter application, or, without a mask, a copy of psi at the last FFT time whose
@@ -226,6 +227,11 @@ int initialize_t(phx_solver* s) {
     s->staged = !s->ssfm && (s->grouped || c.complex_reservoir ||
                              (s->iter && (!phx::rk_tableau_fused(s->iter->fixed) || !phx::rk_tableau_fused(s->iter->adaptive))));
     if (s->staged) s->grouped = true;
+    /* RK4 under chains of few groups takes the chain kernel: no K slots in HBM */
+    const int groups = std::max(std::max(c.use_pumps ? c.pump.groupSize() : 0, c.use_potentials ? c.potential.groupSize() : 0),
+                                c.use_pulses ? c.pulse.groupSize() : 0);
+    s->chain = s->staged && !c.complex_reservoir && s->iter && s->iter->fixed == phx::RkTableau::RK4 &&
+               phx::rk_chain_supported(c.N_c, c.N_r, groups, sizeof(real));
 
     for (int k = 0; k < ncomp; k++) {
         for (int b = 0; b < 2; b++) {
@@ -261,7 +267,7 @@ int initialize_t(phx_solver* s) {
         if (want)
             if (int r = dev_alloc(s, &s->spec[k], 2 * N * sizeof(real))) return r;
     }
-    if (s->staged) {
+    if (s->staged && !s->chain) {
         const int H = std::max(phx::rk_tableau_stages(s->iter->fixed), phx::rk_tableau_stages(s->iter->adaptive));
         s->staged_H = H;
         s->staged_padN = (size_t)(c.N_c + 2 * H) * (size_t)(c.N_r + 2 * H);
@@ -432,9 +438,10 @@ bool adapt_dt(double err, double norm, double tol, double dt, double dt_min, dou
     return fe < tol;
 }
 
-/* One fused generic-tableau step from the current buffers into the other ones. */
+/* Arguments of the fused generic kernel from the current buffers into the other ones, without the
+   temporal amplitudes. */
 template <typename real>
-int generic_launch(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
+phx::RkGenArgs<real> generic_args(phx_solver* s, double dt) {
     auto& c = s->cfg;
     using v2 = typename phx::Vec2<real>::type;
     phx::RkGenArgs<real> a{};
@@ -455,6 +462,18 @@ int generic_launch(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
     a.stochastic = c.use_stochastic;
     a.imag = c.imag_time_amplitude != 0.0;
     a.dt = (real)dt;
+    a.noise = (const v2*)s->noise;
+    a.partials = s->partials;
+    a.sums = s->sums;
+    a.ph = phys_of<real>(s);
+    return a;
+}
+
+/* One fused generic-tableau step from the current buffers into the other ones. */
+template <typename real>
+int generic_launch(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
+    auto& c = s->cfg;
+    phx::RkGenArgs<real> a = generic_args<real>(s, dt);
     static const double w01[2] = {0.0, 1.0};
     real pa[2], va[2];
     stage_amps<real>(c.pump, t_k, dt, w01, 2, pa);
@@ -463,19 +482,67 @@ int generic_launch(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
     a.amp_next_pump = pa[1];
     a.amp_pot_h = (real)((double)va[0] * c.one_over_h_bar_s);
     a.amp_next_pot_h = (real)((double)va[1] * c.one_over_h_bar_s);
-    a.noise = (const v2*)s->noise;
-    a.partials = s->partials;
-    a.sums = s->sums;
-    a.ph = phys_of<real>(s);
     PHX_HIP(phx::launch_rk_generic<real>(a, tab, s->stream));
+    return PHX_OK;
+}
+
+/* Temporal amplitudes of every group of the three sources (pump, potential, pulse) at t and at t + dt, in
+   the build's precision; at a stage of weight w a group enters with a_g(t)(1 - w) + w a_g(t + dt)
+   (kernel_gp_compute.cuh:79,93,98). */
+template <typename real>
+struct GroupAmps {
+    std::complex<real> a0[3][phx::kStagedMaxGroups], a1[3][phx::kStagedMaxGroups];
+    GroupAmps(phx_solver* s, double t, double dt) {
+        const auto& c = s->cfg;
+        const phx::Envelope* env[3] = {&c.pump, &c.potential, &c.pulse};
+        const int ng[3] = {s->st_npump, s->st_npot, s->st_npulse};
+        for (int q = 0; q < 3; q++)
+            for (int g = 0; g < ng[q]; g++) {
+                a0[q][g] = std::complex<real>(env[q]->temporal(g, t));
+                a1[q][g] = std::complex<real>(env[q]->temporal(g, s->rnd(t + dt)));
+            }
+    }
+    typename phx::Vec2<real>::type at(int q, int g, real w) const {
+        typename phx::Vec2<real>::type z;
+        z.x = a0[q][g].real() * (real(1) - w) + w * a1[q][g].real();
+        z.y = a0[q][g].imag() * (real(1) - w) + w * a1[q][g].imag();
+        return z;
+    }
+};
+
+/* One RK4 step under source chains by the chain kernel (phx_rk_chain.hip). */
+template <typename real>
+int chain_launch(phx_solver* s, double t_k, double dt) {
+    auto& c = s->cfg;
+    phx::RkGenArgs<real> a = generic_args<real>(s, dt);
+    phx::RkChainArgs<real> ch{};
+    for (int k = 0; k < (c.tetm ? 2 : 1); k++) ch.pulse[k] = (const typename phx::Vec2<real>::type*)s->st_pulse[k];
+    ch.npump = s->st_npump;
+    ch.npot = s->st_npot;
+    ch.npulse = s->st_npulse;
+    const GroupAmps<real> amps(s, t_k, dt);
+    const real h = phys_of<real>(s).one_over_h_bar_s;
+    static const double w[phx::kChainStages] = {0.0, 0.5, 0.5, 1.0};
+    for (int st = 0; st < phx::kChainStages; st++) {
+        for (int g = 0; g < ch.npump; g++) ch.pump_amp[st][g] = amps.at(0, g, (real)w[st]).x;
+        for (int g = 0; g < ch.npot; g++) {
+            ch.pot_amp_h[st][g] = amps.at(1, g, (real)w[st]);
+            ch.pot_amp_h[st][g].x *= h;
+            ch.pot_amp_h[st][g].y *= h;
+        }
+        for (int g = 0; g < ch.npulse; g++) {
+            ch.pulse_amp_h[st][g] = amps.at(2, g, (real)w[st]);
+            ch.pulse_amp_h[st][g].x *= h;
+            ch.pulse_amp_h[st][g].y *= h;
+        }
+    }
+    PHX_HIP(phx::launch_rk_chain<real>(a, ch, s->stream));
     return PHX_OK;
 }
 
 /* One staged step attempt (phx_staged.hip) from the current buffers into the other ones:
    the reference's CALCULATE_K / INTERMEDIATE_SUM_K sequence on shrinking extents, then the
-   final sum (and, for an adaptive tableau, the reduced error and norm in s->sums).  Each
-   temporal group g of a source enters stage s with a_g(t)(1 - c_s) + c_s a_g(t + dt)
-   (kernel_gp_compute.cuh:79,93,98). */
+   final sum (and, for an adaptive tableau, the reduced error and norm in s->sums). */
 template <typename real>
 int staged_attempt(phx_solver* s, phx::RkTableau tab_id, double t_k, double dt) {
     auto& c = s->cfg;
@@ -520,27 +587,14 @@ int staged_attempt(phx_solver* s, phx::RkTableau tab_id, double t_k, double dt) 
     a.dti = imag ? -(real)dt : real(0);
     a.partials = s->st_partials;
     a.ph = phys_of<real>(s);
-    /* temporal amplitudes of every group at t and t + dt, in the build's precision */
-    std::complex<real> amp0[3][phx::kStagedMaxGroups], amp1[3][phx::kStagedMaxGroups];
-    const phx::Envelope* env[3] = {&c.pump, &c.potential, &c.pulse};
-    const int ng[3] = {a.npump, a.npot, a.npulse};
-    for (int q = 0; q < 3; q++)
-        for (int g = 0; g < ng[q]; g++) {
-            amp0[q][g] = std::complex<real>(env[q]->temporal(g, t_k));
-            amp1[q][g] = std::complex<real>(env[q]->temporal(g, s->rnd(t_k + dt)));
-        }
+    const GroupAmps<real> amps(s, t_k, dt);
     auto set_amps = [&](real w) {
-        for (int q = 0; q < 3; q++)
-            for (int g = 0; g < ng[q]; g++) {
-                const real re = amp0[q][g].real() * (real(1) - w) + w * amp1[q][g].real();
-                const real im = amp0[q][g].imag() * (real(1) - w) + w * amp1[q][g].imag();
-                if (q == 0) a.pump_amp[g] = re, a.pump_amp_im[g] = im;
-                v2 z;
-                z.x = re;
-                z.y = im;
-                if (q == 1) a.pot_amp[g] = z;
-                if (q == 2) a.pulse_amp[g] = z;
-            }
+        for (int g = 0; g < a.npump; g++) {
+            a.pump_amp[g] = amps.at(0, g, w).x;
+            a.pump_amp_im[g] = amps.at(0, g, w).y;
+        }
+        for (int g = 0; g < a.npot; g++) a.pot_amp[g] = amps.at(1, g, w);
+        for (int g = 0; g < a.npulse; g++) a.pulse_amp[g] = amps.at(2, g, w);
     };
     /* weights of a sum: the nonzero a[s][j] (or b, e) with their slots */
     auto set_weights = [&](const double* wts, int n, int* slot, real* w, int& count, real* wsum) {
@@ -575,9 +629,10 @@ int staged_attempt(phx_solver* s, phx::RkTableau tab_id, double t_k, double dt) 
     return PHX_OK;
 }
 
-/* one step attempt of the configured iterator: fused generic kernel or staged path */
+/* one step attempt of the configured iterator: fused generic kernel, chain kernel or staged path */
 template <typename real>
 int rk_attempt(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
+    if (s->chain) return chain_launch<real>(s, t_k, dt);
     return s->staged ? staged_attempt<real>(s, tab, t_k, dt) : generic_launch<real>(s, tab, t_k, dt);
 }
 
