@@ -532,19 +532,17 @@ FftPlan make_plan(int len, const int* radix, int passes) {
 /* e^{-2 pi i k / n}, k reduced exactly */
 std::complex<double> root(long long k, long long n) { return std::polar(1.0, -2.0 * M_PI * (double)(k % n) / (double)n); }
 
-/* forward DFT by decimation in time over the prime factors of the length */
-std::vector<std::complex<double>> host_fft(const std::vector<std::complex<double>>& x) {
-    const long long n = (long long)x.size();
-    if (n == 1) return x;
-    long long p = 2;
+/* forward DFT of every step-th value from x, by decimation in time over the prime factors of the length n;
+   w holds the roots of the whole transform, of n * step points */
+std::vector<std::complex<double>> host_fft(const std::complex<double>* x, size_t n, size_t step, const std::vector<std::complex<double>>& w) {
+    if (n == 1) return {x[0]};
+    size_t p = 2;
     while (n % p) p++;
-    const long long m = n / p;
+    const size_t m = n / p;
     std::vector<std::complex<double>> out(n);
-    for (long long j = 0; j < p; j++) {
-        std::vector<std::complex<double>> sub(m);
-        for (long long i = 0; i < m; i++) sub[i] = x[i * p + j];
-        sub = host_fft(sub);
-        for (long long k = 0; k < n; k++) out[k] += root(j * k, n) * sub[k % m];
+    for (size_t j = 0; j < p; j++) {
+        const auto sub = host_fft(x + j * step, m, step * p, w);
+        for (size_t k = 0; k < n; k++) out[k] += w[j * k % n * step] * sub[k % m];
     }
     return out;
 }
@@ -589,7 +587,8 @@ std::vector<std::complex<double>> fft_axis_table(const FftAxis& a) {
     std::vector<std::complex<double>> t;
     for (int k = 0; k < a.N; k++) t.push_back(root(k, a.N));
     if (!a.M) return t;
-    for (int k = 0; k < a.M; k++) t.push_back(root(k, a.M));
+    std::vector<std::complex<double>> w(a.M);
+    for (int k = 0; k < a.M; k++) t.push_back(w[k] = root(k, a.M));
     std::vector<std::complex<double>> b(a.M);
     for (long long j = 0; j < a.N; j++) {
         const auto c = root(j * j % (2 * a.N), 2 * a.N);
@@ -597,7 +596,7 @@ std::vector<std::complex<double>> fft_axis_table(const FftAxis& a) {
         b[j] = std::conj(c);
         if (j) b[a.M - j] = std::conj(c);
     }
-    for (const auto& z : host_fft(b)) t.push_back(z / (double)a.M);
+    for (const auto& z : host_fft(b.data(), a.M, 1, w)) t.push_back(z / (double)a.M);
     return t;
 }
 

@@ -50,12 +50,17 @@ inline int rk4_alt_rows() {
 }
 
 /* Launch shape of the fused RK4 kernel.
-   ty: output rows per wavefront tile (8, 10, 12, 16, 20, 24);
+   ty: output rows per wavefront tile (2, 4, 8, 10, 12, 16, 20, 24);
    ew, pf: kept for the tuning interface; the kernel uses DPP wave shifts for
    east/west and loads rows 2 ahead of first use. */
 struct Rk4Tune {
     int ty = 16, ew = 1, pf = 2;
 };
+
+/* SIMDs of the device (four a CU) */
+int rk4_simds();
+/* tile height of an untimed launch (phx_rk_generic.hip) */
+Rk4Tune rk4_default_tune(int Nc, int Nr, size_t real_size);
 
 template <typename real>
 hipError_t launch_rk4_scalar(const Rk4Args<real>& a, const Rk4Tune& t, hipStream_t s);

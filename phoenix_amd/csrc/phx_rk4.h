@@ -216,18 +216,31 @@ __global__ __launch_bounds__(256) void rk4_scalar_fused(Rk4Args<real> a) {
     rk4_tile<real, TY, ISO, PF, RES, PUMP, POT, PERY>(a, strip, band);
 }
 
+/* Tile d (-2 .. 2) places away along one axis of n tiles of w cells (the last: the rest of N): its index, and
+   `ok` cleared where it does not exist or the kHalo cells next to tile i do not reach it. */
+__device__ __forceinline__ int flow_reach(int i, int d, int n, int w, int N, bool periodic, bool& ok) {
+    int j = i + d;
+    if (j < 0 || j >= n) {
+        if (!periodic) ok = false;
+        j = (j + 2 * n) % n;
+    }
+    if (d == 2 || d == -2) { /* cells of the tile in between */
+        const int m = (i + d / 2 + n) % n;
+        if ((m == n - 1 ? N - m * w : w) >= kHalo) ok = false;
+    }
+    return j;
+}
+
 /* Many steps in one launch, one resident wavefront per tile.  Before step k a tile waits
-   until the eight tiles whose cells its 4-cell halo covers have finished step k-1 (their
-   step counters reach base + k): their outputs of step k-1 are its inputs, and their reads
+   until the tiles whose cells its 4-cell halo covers (eight of them, more next to a narrow
+   last strip or band) have finished step k-1 (their step counters reach base + k): their outputs of step k-1 are its inputs, and their reads
    of step k-1, which covered its cells in the buffer it is about to overwrite, are done.
    psi and n go through device-scope loads and stores (no stale line of another XCD's
    write is used); a counter moves only after all stores of the step have completed.  Each
    counter has a 128-byte line of its own: packed 32 to a line, the polls of neighbouring
    tiles contended for the same lines and a step took 21 instead of 8 us at 1024^2.  A
    wait longer than spin_limit polls sets *error and ends the wave (its neighbours then
-   time out too, so every wave exits); the state is then undefined.  Tiles of the last
-   band and strip must be at least kHalo cells deep/wide, so that a halo never reaches
-   past the neighbouring tile (rk4_flow_shape_ok). */
+   time out too, so every wave exits); the state is then undefined. */
 template <typename real, int TY, bool ISO, int PF, bool RES, bool PUMP, bool POT, bool PERY, bool CAMP = false>
 __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow f) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -237,24 +250,14 @@ __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow 
     const int band = (tile / a.nstrips) * kWavesPerBlock + wave;
     if (band >= a.nbands) return; /* no tile: nobody watches this wave's counter */
     const int me = band * a.nstrips + strip;
-    /* lanes 0..7 watch the neighbours (d = 0..8 without the centre 4) */
+    /* lanes 0..24 watch the tiles up to two strips and two bands away that the halo reaches: the next one
+       on each side, and the one behind it where the next is a last strip or band of fewer than kHalo cells */
     int watch = -1;
-    if (lane < 8) {
-        const int d = lane + (lane >= 4 ? 1 : 0);
-        int ns = strip + d % 3 - 1, nb = band + d / 3 - 1;
-        bool ok = true;
-        if (ns < 0 || ns >= a.nstrips) {
-            if (a.periodic_x)
-                ns = (ns + a.nstrips) % a.nstrips;
-            else
-                ok = false;
-        }
-        if (nb < 0 || nb >= a.nbands) {
-            if (PERY)
-                nb = (nb + a.nbands) % a.nbands;
-            else
-                ok = false;
-        }
+    if (lane < 25) {
+        const int ds = lane % 5 - 2, db = lane / 5 - 2;
+        bool ok = lane != 12;
+        const int ns = flow_reach(strip, ds, a.nstrips, kOutW, a.Nc, a.periodic_x, ok);
+        const int nb = flow_reach(band, db, a.nbands, TY, a.Nr, PERY, ok);
         if (ok) watch = nb * a.nstrips + ns;
     }
     int* const mine = f.counters + (size_t)me * kFlowCounterStride;
@@ -351,10 +354,12 @@ inline hipError_t launch_ty(const Rk4Args<real>& a0, hipStream_t s) {
     return hipGetLastError();
 }
 
-/* Tile height TY in {8, 10, 12, 16, 20, 24} (others: 16). */
+/* Tile height TY in {2, 4, 8, 10, 12, 16, 20, 24} (others: 16). */
 template <typename real, bool ISO, int PF, bool RES, bool PUMP, bool POT>
 inline hipError_t launch_tys(const Rk4Args<real>& a, const Rk4Tune& t, hipStream_t s) {
     switch (t.ty) {
+        case 2: return launch_ty<real, 2, ISO, PF, RES, PUMP, POT>(a, s);
+        case 4: return launch_ty<real, 4, ISO, PF, RES, PUMP, POT>(a, s);
         case 8: return launch_ty<real, 8, ISO, PF, RES, PUMP, POT>(a, s);
         case 10: return launch_ty<real, 10, ISO, PF, RES, PUMP, POT>(a, s);
         case 12: return launch_ty<real, 12, ISO, PF, RES, PUMP, POT>(a, s);
@@ -390,10 +395,9 @@ hipError_t launch_rk4_scalar(const Rk4Args<real>& a, const Rk4Tune& t, hipStream
 }
 
 /* ---------------------------------------------------------------- many steps per launch */
-inline bool rk4_flow_shape_ok(int Nc, int Nr, int ty) {
-    const int last_rows = Nr - ((Nr - 1) / ty) * ty, last_cols = Nc - ((Nc - 1) / kOutW) * kOutW;
-    return Nr >= ty && Nc >= kOutW && last_rows >= kHalo && last_cols >= kHalo;
-}
+/* At least one whole tile along each axis: every tile but the last is then ty (>= kHalo) rows and kOutW columns,
+   and no halo reaches further than flow_reach looks. */
+inline bool rk4_flow_shape_ok(int Nc, int Nr, int ty) { return ty >= kHalo && Nr >= ty && Nc >= kOutW; }
 
 template <typename real, int TY, bool ISO, int PF, bool RES, bool PUMP, bool POT, bool CAMP = false>
 inline hipError_t launch_flow_ty(const Rk4Args<real>& a0, const Rk4Flow& f, hipStream_t s) {
@@ -418,6 +422,7 @@ inline hipError_t launch_flow_ty(const Rk4Args<real>& a0, const Rk4Flow& f, hipS
 template <typename real, bool ISO, int PF, bool RES, bool PUMP, bool POT, bool CAMP = false>
 inline hipError_t launch_flow_tys(const Rk4Args<real>& a, const Rk4Tune& t, const Rk4Flow& f, hipStream_t s) {
     switch (t.ty) {
+        case 4: return launch_flow_ty<real, 4, ISO, PF, RES, PUMP, POT, CAMP>(a, f, s);
         case 8: return launch_flow_ty<real, 8, ISO, PF, RES, PUMP, POT, CAMP>(a, f, s);
         case 10: return launch_flow_ty<real, 10, ISO, PF, RES, PUMP, POT, CAMP>(a, f, s);
         case 12: return launch_flow_ty<real, 12, ISO, PF, RES, PUMP, POT, CAMP>(a, f, s);
@@ -476,6 +481,7 @@ inline hipError_t launch_batch_ty(const Rk4BatchArgs<real>& b, hipStream_t s) {
 template <typename real, bool ISO, bool RES, bool PUMP, bool POT>
 inline hipError_t launch_batch_tys(const Rk4BatchArgs<real>& b, int ty, hipStream_t s) {
     switch (ty) {
+        case 4: return launch_batch_ty<real, 4, ISO, RES, PUMP, POT>(b, s);
         case 8: return launch_batch_ty<real, 8, ISO, RES, PUMP, POT>(b, s);
         case 10: return launch_batch_ty<real, 10, ISO, RES, PUMP, POT>(b, s);
         case 16: return launch_batch_ty<real, 16, ISO, RES, PUMP, POT>(b, s);

@@ -138,7 +138,7 @@ hipError_t launch_noise_field(typename Vec2<real>::type* xi, int Nc, int Nr, uin
 template hipError_t launch_noise_field<float>(float2*, int, int, uint64_t, uint64_t, float, hipStream_t);
 template hipError_t launch_noise_field<double>(double2*, int, int, uint64_t, uint64_t, double, hipStream_t);
 
-static int device_simds() {
+int rk4_simds() {
     static const int simds = [] {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -146,6 +146,24 @@ static int device_simds() {
         return 4 * std::max(cus, 1);
     }();
     return simds;
+}
+
+Rk4Tune rk4_default_tune(int Nc, int Nr, size_t real_size) {
+    /* The rows of a tile are a serial chain: a grid that fits the SIMDs in one round takes the shortest tile
+       that does.  Up to two rounds FP32 runs best at 10 rows (two waves a SIMD cover each other's waits);
+       FP64, whose waves issue twice the work a row, at one round of 20; larger grids are within 5 % of their
+       best at 16.  us per launch at 16 rows and by this rule: 200 x 150 FP32 7.3 and 3.7, FP64 8.7 and 4.4;
+       400^2 7.7 / 4.5, 9.2 / 5.4; 512^2 7.7 / 5.5, 9.4 / 6.8; 768^2 8.4 / 7.1, 10.4 / 8.8; 1024^2 11.2 / 9.2,
+       16.0 / 13.5; 1500^2 16.0, 25.0. */
+    Rk4Tune t;
+    for (int ty : {2, 4, 8, 12})
+        if (rk4_tiles(Nc, Nr, ty) <= rk4_simds()) {
+            t.ty = ty;
+            return t;
+        }
+    if (real_size == 4 && rk4_tiles(Nc, Nr, 10) <= 2 * rk4_simds()) t.ty = 10;
+    if (real_size == 8 && rk4_tiles(Nc, Nr, 20) <= rk4_simds()) t.ty = 20;
+    return t;
 }
 
 int rk4_generic_tile_rows(int Nc, int Nr) {
@@ -161,7 +179,7 @@ int rk4_generic_tile_rows(int Nc, int Nr) {
     long best_cost = -1;
     for (int ty : {16, 8, 4}) {
         const long waves = (long)((Nc + 55) / 56) * ((Nr + ty - 1) / ty);
-        const long cost = ((waves + device_simds() - 1) / device_simds()) * (long)(S * (ty + 2 * S) - S * (S + 1));
+        const long cost = ((waves + rk4_simds() - 1) / rk4_simds()) * (long)(S * (ty + 2 * S) - S * (S + 1));
         if (best_cost < 0 || cost < best_cost) best = ty, best_cost = cost;
     }
     return best;
@@ -172,7 +190,7 @@ int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr) {
     const char* e = std::getenv("PHX_GEN_TY"); /* read at every launch: tests switch it within a process */
     const int env_ty = e ? std::atoi(e) : 0;
     if (env_ty == 16 || env_ty == 32) return env_ty;
-    const int simds = device_simds();
+    const int simds = rk4_simds();
     /* One wave per SIMD at the kernel's register count (over 256 VGPRs + AGPRs at every height),
        and about the same VALU work per row evaluation at every height (145-148 instructions): a
        SIMD's time is its number of tiles (rounded up) times the row evaluations of one tile,

@@ -91,14 +91,16 @@ struct phx_solver {
     double t = 0, dt = 0, fft_cached_t = 0;
     int64_t iteration = 0, rejected = 0;
     int64_t out_iter = 1; /* output intervals started (main.cu:64, out_every_iterations) */
-    phx::Rk4Tune tune; /* launch shape of the fused RK4 kernel */
+    phx::Rk4Tune tune;      /* launch shape of the fused RK4 kernel */
+    phx::Rk4Tune flow_tune; /* ... and of its multi-step form */
     bool tuned = false;
-    /* captured run of kGraphSteps fused RK4 launches (replayed while nothing changes between steps) */
+    /* captured run of graph_steps fused RK4 launches (replayed while nothing changes between steps) */
     hipGraphExec_t graph = nullptr;
-    int graph_parity = -1;
+    int graph_parity = -1, graph_steps = 0;
     double graph_dt = 0;
     hipStream_t graph_stream = nullptr;
     bool graph_off = false;
+    int64_t direct_steps = 0; /* steps of such runs launched one by one so far */
     /* the same runs as one launch of rk4_scalar_flow: per-tile step counters (all equal to
        flow_base between launches) and the kernel's error word */
     int* flow_counters = nullptr;
@@ -375,7 +377,7 @@ int initialize_t(phx_solver* s) {
     s->fft_cached_t = 0.0;
     s->cur = 0;
     s->initialized = true;
-    s->tune = rk4_tune_from_env(s->tune);
+    s->tune = s->flow_tune = rk4_tune_from_env(s->tune);
     return PHX_OK;
 }
 
@@ -773,18 +775,19 @@ int autotune_rk4(phx_solver* s) {
     hipEvent_t e0, e1;
     PHX_HIP(hipEventCreate(&e0));
     PHX_HIP(hipEventCreate(&e1));
-    const int cands[] = {8, 10, 12, 16, 20, 24};
+    const int cands[] = {8, 10, 12, 16, 20, 24, 4, 2};
+    constexpr int ncand = 8;
     /* deeper row prefetch exists for the pumped reservoir model */
     const int pfs[] = {2, 3, 4, 6, 8};
     const int npf = (c.use_reservoir && c.use_pumps && !c.use_potentials) ? 5 : 1;
     /* three round-robin passes over the candidates, each candidate's fastest pass counts: a
        single pass in a fixed order would time the first candidates while the clocks ramp up */
-    std::vector<float> cand_ms(6 * npf, 1e30f);
+    std::vector<float> cand_ms(ncand * npf, 1e30f);
     for (int pass = 0; pass < 3; pass++) {
-        for (int cand = 0; cand < 6 * npf; cand++) {
+        for (int cand = 0; cand < ncand * npf; cand++) {
             phx::Rk4Tune t = s->tune;
-            t.ty = cands[cand % 6];
-            t.pf = pfs[cand / 6];
+            t.ty = cands[cand % ncand];
+            t.pf = pfs[cand / ncand];
             const phx::Rk4Tune keep = s->tune;
             s->tune = t;
             int rc = PHX_OK;
@@ -802,11 +805,11 @@ int autotune_rk4(phx_solver* s) {
         }
     }
     int best = 0;
-    for (int cand = 1; cand < 6 * npf; cand++)
+    for (int cand = 1; cand < ncand * npf; cand++)
         if (cand_ms[cand] < cand_ms[best]) best = cand;
     phx::Rk4Tune best_t = s->tune;
-    best_t.ty = cands[best % 6];
-    best_t.pf = pfs[best / 6];
+    best_t.ty = cands[best % ncand];
+    best_t.pf = pfs[best / ncand];
     PHX_HIP(hipEventDestroy(e0));
     PHX_HIP(hipEventDestroy(e1));
     s->tune = best_t;
@@ -913,7 +916,9 @@ int iterate(phx_solver* s, bool force_fixed) {
     return s->precision == PHX_FP32 ? iterate_t<float>(s, force_fixed) : iterate_t<double>(s, force_fixed);
 }
 
-constexpr int kGraphSteps = 50; /* graph replay: even, so the buffer parity returns */
+/* graph replay: at most kGraphSteps launches, an even number, so the buffer parity returns */
+constexpr int kGraphSteps = 50, kGraphMinSteps = 10;
+constexpr int64_t kGraphAfter = 400;
 
 /* One launch of rk4_scalar_flow for `steps` (even) steps of the same run; returns 1 when the
    kernel cannot take this grid or launch shape (the caller falls back to the graph). */
@@ -946,23 +951,36 @@ phx::Rk4Args<real> rk4_args(phx_solver* s, void* psi_in, void* n_in, void* psi_o
     return a;
 }
 
+/* Whether a run of n steps goes to the multi-step kernel.  PHX_RK4_FLOW=0: never, 1: from 2 steps on.
+   Otherwise from 10 steps on, on grids whose 4-row tiles fill the SIMDs.  A cooperative launch costs about
+   15 us before its first step and no two of them run at once on a device, so short runs and small grids
+   are launched step by step (from a graph once they repeat), which leaves room for the kernels of other
+   handles.  us per run, one handle alone / three in turn, launches and multi-step (FP64 unless noted):
+   256^2 5 steps 32 / 25 and 43 / 34, 50 steps 199 / 95 and 212 / 208; 400^2 5 steps 37 / 27 and 45 / 36,
+   50 steps 252 / 137 and 234 / 226; 640^2 5 steps 48 / 24 and 50 / 43, 50 steps 349 / 269 and 288 / 307;
+   1024^2 10 steps 140 / 102 and 126 / 127, 50 steps 643 / 514 and 525 / 587, FP32 439 / 326 and 369 / 390. */
+constexpr int64_t kFlowMinSteps = 10, kFlowMaxSteps = 500;
+
+bool flow_wanted(phx_solver* s, int64_t n) {
+    if (const char* e = std::getenv("PHX_RK4_FLOW")) return std::atoi(e) != 0 && n >= 2;
+    return n >= kFlowMinSteps && phx::rk4_tiles(s->cfg.N_c, s->cfg.N_r, 4) > phx::rk4_simds();
+}
+
 /* Counters of the multi-step kernel, allocated on first use once the kernel is known to take
-   this grid with the handle's tile shape.  Returns 1 when it does not (or PHX_RK4_FLOW=0). */
+   this grid with the handle's tile shape.  Returns 1 when it does not. */
 template <typename real>
 int flow_ready(phx_solver* s) {
     if (s->flow_off) return 1;
-    if (const char* e = std::getenv("PHX_RK4_FLOW"))
-        if (std::atoi(e) == 0) return 1; /* PHX_RK4_FLOW=0: one launch per step */
     auto& c = s->cfg;
-    const size_t counters = (size_t)((c.N_c + 55) / 56) * (size_t)((c.N_r + 7) / 8) * phx::kFlowCounterStride;
+    const size_t counters = (size_t)((c.N_c + 55) / 56) * (size_t)((c.N_r + 3) / 4) * phx::kFlowCounterStride;
     if (!s->flow_counters) {
         const phx::Rk4Args<real> a = rk4_args<real>(s, s->psi[0][s->cur], s->n[0][s->cur], s->psi[0][s->cur ^ 1], s->n[0][s->cur ^ 1]);
-        if (phx::launch_rk4_flow<real>(a, s->tune, phx::Rk4Flow{nullptr, nullptr, 0, 2, 0}, s->stream) != hipSuccess) {
+        if (phx::launch_rk4_flow<real>(a, s->flow_tune, phx::Rk4Flow{nullptr, nullptr, 0, 2, 0}, s->stream) != hipSuccess) {
             (void)hipGetLastError();
             s->flow_off = true;
             return 1;
         }
-        if (int r = dev_alloc(s, (void**)&s->flow_counters, counters * sizeof(int))) return r; /* any tile height >= 8 */
+        if (int r = dev_alloc(s, (void**)&s->flow_counters, counters * sizeof(int))) return r; /* any tile height >= 4 */
         if (int r = dev_alloc(s, (void**)&s->flow_error, sizeof(int))) return r;
         s->flow_base = 0;
     }
@@ -993,9 +1011,9 @@ hipError_t flow_launch(phx_solver* s, const phx::Rk4Tune& tune, void* psi_in, vo
 template <typename real>
 int flow_block_t(phx_solver* s, int steps) {
     if (int r = flow_ready<real>(s)) return r;
-    if (flow_launch<real>(s, s->tune, s->psi[0][s->cur], s->n[0][s->cur], s->psi[0][s->cur ^ 1], s->n[0][s->cur ^ 1], steps) !=
+    if (flow_launch<real>(s, s->flow_tune, s->psi[0][s->cur], s->n[0][s->cur], s->psi[0][s->cur ^ 1], s->n[0][s->cur ^ 1], steps) !=
         hipSuccess) {
-        s->flow_off = true; /* nothing ran: step by graph from now on */
+        s->flow_off = true; /* nothing ran: step by launches from now on */
         return 1;
     }
     s->flow_steps += steps;
@@ -1006,16 +1024,18 @@ int flow_block_t(phx_solver* s, int steps) {
 /* Tile shape of the multi-step kernel, timed on that kernel: every candidate runs kFlowTuneSteps
    steps from the second buffer through a temporary one and back (an even count), so the state in
    the current buffer is not touched.  Two passes, each candidate's faster one counts; shapes the
-   kernel does not take are skipped.  The winner replaces the one-step tuning's choice. */
+   kernel does not take are skipped. */
 constexpr int kFlowTuneSteps = 40;
 
 template <typename real>
 int autotune_flow(phx_solver* s) {
     static std::map<std::string, phx::Rk4Tune> cache;
     auto& c = s->cfg;
+    s->flow_tune = s->tune;
     if (std::getenv("PHX_RK4_TY")) return PHX_OK;
     if (const char* e = std::getenv("PHX_AUTOTUNE"))
         if (std::atoi(e) == 0) return PHX_OK;
+    if (!flow_wanted(s, kFlowMaxSteps)) return PHX_OK;
     const auto constant = [](const phx::Envelope& e) { return e.groupSize() != 1 || e.allConstant(); };
     if (s->staged || c.iterator != "RK4" || c.tetm || c.use_stochastic || c.imag_time_amplitude != 0.0 || !constant(c.pump) ||
         !constant(c.potential))
@@ -1024,14 +1044,14 @@ int autotune_flow(phx_solver* s) {
                             std::to_string(c.use_reservoir) + std::to_string(c.use_pumps) + std::to_string(c.use_potentials) +
                             std::to_string(c.periodic_x) + std::to_string(c.periodic_y);
     if (auto it = cache.find(key); it != cache.end()) {
-        s->tune = it->second;
+        s->flow_tune = it->second;
         return PHX_OK;
     }
     const phx::Rk4Tune one_step = s->tune;
-    s->tune.ty = 10; /* a shape the kernel has, for the availability check */
-    s->tune.pf = 2;
+    s->flow_tune.ty = 10; /* a shape the kernel has, for the availability check */
+    s->flow_tune.pf = 2;
     const int fr = flow_ready<real>(s);
-    s->tune = one_step;
+    s->flow_tune = one_step;
     if (fr) return fr < 0 ? fr : PHX_OK;
     const size_t N = s->cells();
     void *tmp_psi = nullptr, *tmp_n = nullptr;
@@ -1043,18 +1063,19 @@ int autotune_flow(phx_solver* s) {
     hipEvent_t e0, e1;
     PHX_HIP(hipEventCreate(&e0));
     PHX_HIP(hipEventCreate(&e1));
-    const int tys[] = {8, 10, 12, 16, 20};
+    const int tys[] = {8, 10, 12, 16, 20, 4};
+    constexpr int nty = 6;
     const int pfs[] = {2, 3, 4, 6, 8};
     const int npf = (c.use_reservoir && c.use_pumps && !c.use_potentials) ? 5 : 1;
-    std::vector<float> ms(5 * npf, 1e30f);
+    std::vector<float> ms(nty * npf, 1e30f);
     void* psi2 = s->psi[0][s->cur ^ 1];
     void* n2 = s->n[0][s->cur ^ 1];
     int rc = PHX_OK;
     for (int pass = 0; pass < 2 && !rc; pass++) {
-        for (int cand = 0; cand < 5 * npf && !rc; cand++) {
+        for (int cand = 0; cand < nty * npf && !rc; cand++) {
             phx::Rk4Tune t = one_step;
-            t.ty = tys[cand % 5];
-            t.pf = pfs[cand / 5];
+            t.ty = tys[cand % nty];
+            t.pf = pfs[cand / nty];
             if (hipEventRecord(e0, s->stream) != hipSuccess) rc = fail(PHX_ERR_HIP, "hipEventRecord");
             if (!rc && flow_launch<real>(s, t, psi2, n2, tmp_psi, tmp_n, kFlowTuneSteps) != hipSuccess) continue;
             float m = 0;
@@ -1072,15 +1093,15 @@ int autotune_flow(phx_solver* s) {
     if (rc) return rc;
     if (int r = flow_check(s)) return r;
     int best = -1;
-    for (int cand = 0; cand < 5 * npf; cand++)
+    for (int cand = 0; cand < nty * npf; cand++)
         if (ms[cand] < 1e29f && (best < 0 || ms[cand] < ms[best])) best = cand;
     if (best < 0) {
         s->flow_off = true;
         return PHX_OK;
     }
-    s->tune.ty = tys[best % 5];
-    s->tune.pf = pfs[best / 5];
-    cache[key] = s->tune;
+    s->flow_tune.ty = tys[best % nty];
+    s->flow_tune.pf = pfs[best / nty];
+    cache[key] = s->flow_tune;
     return PHX_OK;
 }
 
@@ -1099,14 +1120,13 @@ int flow_check(phx_solver* s) {
 }
 
 /* Runs of fixed RK4 steps of the scalar model whose kernel arguments do not change from step
-   to step (constant temporal amplitudes, no noise) leave the one-launch-per-step path: up to
-   kFlowMaxSteps of them as one launch of the multi-step kernel, or, where that kernel does not
-   take the grid, kGraphSteps of them replayed from a captured hipGraph.  A run stops before the
+   to step (constant temporal amplitudes, no noise) go to the device together: up to
+   kFlowMaxSteps of them as one launch of the multi-step kernel (flow_wanted), otherwise launch by launch,
+   up to kGraphSteps of them replayed from a captured hipGraph once the handle has launched kGraphAfter steps
+   one by one (a replayed step takes 0.8 to 1.3 us less than a launched one, a capture of 50 about 300 us).  A run stops before the
    step that reaches t_max, that fires the k-space filter, or that would pass t_stop (the
    caller shortens that one); the host advances t and the FFT guard exactly as iterate()
    would.  *taken: the steps run (0: not eligible, the caller iterates). */
-constexpr int64_t kFlowMaxSteps = 500;
-
 template <typename real>
 int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     auto& c = s->cfg;
@@ -1115,66 +1135,77 @@ int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     if (!s->tuned || s->staged || c.iterator != "RK4" || c.tetm || c.use_stochastic || c.imag_time_amplitude != 0.0 ||
         !constant(c.pump) || !constant(c.potential))
         return PHX_OK;
-    double t = s->t, fc = s->fft_cached_t, t_graph = 0, fc_graph = 0;
-    int64_t m = 0;
-    const int64_t lim = std::min(max_steps, kFlowMaxSteps);
-    while (m < lim) {
-        if (t >= c.t_max || t >= t_stop) break;
-        const double tn = s->rnd(t + s->dt);
-        if (tn > t_stop) break;
-        double fcn = fc;
-        if (!(s->rnd(tn - fc) < c.fft_every)) {
-            if (c.use_fft_mask || s->spec[0]) break;
-            fcn = tn;
+    /* time and FFT guard after up to `lim` steps that neither reach t_max, pass t_stop nor fire the filter */
+    auto advance = [&](int64_t lim, double& t, double& fc) {
+        t = s->t;
+        fc = s->fft_cached_t;
+        int64_t m = 0;
+        for (; m < lim && t < c.t_max && t < t_stop; m++) {
+            const double tn = s->rnd(t + s->dt);
+            if (tn > t_stop) break;
+            if (!(s->rnd(tn - fc) < c.fft_every)) {
+                if (c.use_fft_mask || s->spec[0]) break;
+                fc = tn;
+            }
+            t = tn;
         }
-        t = tn;
-        fc = fcn;
-        if (++m == kGraphSteps) t_graph = t, fc_graph = fc;
-    }
-    if (m >= 2) {
+        return m;
+    };
+    double t, fc;
+    int64_t m = advance(std::min(max_steps, kFlowMaxSteps), t, fc);
+    auto took = [&](int64_t n) {
+        s->t = t;
+        s->fft_cached_t = fc;
+        s->iteration += n;
+        *taken = n;
+        return PHX_OK;
+    };
+    if (flow_wanted(s, m)) {
         const int fr = flow_block_t<real>(s, (int)m);
         if (fr < 0) return fr;
         if (fr == PHX_OK) {
             if (m & 1) s->cur ^= 1; /* an odd run leaves the result in the other buffer */
-            s->t = t;
-            s->fft_cached_t = fc;
-            s->iteration += m;
-            *taken = m;
-            return PHX_OK;
+            return took(m);
         }
     }
-    if (m < kGraphSteps || s->graph_off) return PHX_OK;
-    if (const char* e = std::getenv("PHX_GRAPH"))
-        if (std::atoi(e) == 0) return PHX_OK; /* PHX_GRAPH=0: launch by launch */
-    if (!s->graph || s->graph_parity != s->cur || s->graph_dt != s->dt || s->graph_stream != s->stream) {
+    if (m < 2) return PHX_OK;
+    const char* ge = std::getenv("PHX_GRAPH"); /* PHX_GRAPH=0: launch by launch */
+    const bool graphs = !s->graph_off && !(ge && std::atoi(ge) == 0);
+    const bool same = s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream;
+    if (graphs && s->direct_steps >= kGraphAfter && m >= kGraphMinSteps && !(same && s->graph_steps <= m)) {
+        const int cur = s->cur, steps = (int)std::min<int64_t>(m, kGraphSteps) & ~1;
+        s->direct_steps = 0;
         if (s->graph) PHX_HIP(hipGraphExecDestroy(s->graph));
         s->graph = nullptr;
-        const int cur = s->cur;
         if (hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
             (void)hipGetLastError();
-            s->graph_off = true; /* e.g. the legacy default stream: step launch by launch */
-            return PHX_OK;
+            s->graph_off = true; /* a stream that cannot be captured: launch by launch from now on */
+        } else {
+            int rc = PHX_OK;
+            for (int k = 0; k < steps && !rc; k++) rc = rk4_launch<real>(s, s->t, s->dt);
+            hipGraph_t g = nullptr;
+            const hipError_t ce = hipStreamEndCapture(s->stream, &g);
+            s->cur = cur;
+            if (rc) return rc;
+            PHX_HIP(ce);
+            const hipError_t ie = hipGraphInstantiate(&s->graph, g, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(g);
+            PHX_HIP(ie);
+            s->graph_parity = cur;
+            s->graph_dt = s->dt;
+            s->graph_stream = s->stream;
+            s->graph_steps = steps;
         }
-        int rc = PHX_OK;
-        for (int k = 0; k < kGraphSteps && !rc; k++) rc = rk4_launch<real>(s, s->t, s->dt);
-        hipGraph_t g = nullptr;
-        const hipError_t ce = hipStreamEndCapture(s->stream, &g);
-        s->cur = cur;
-        if (rc) return rc;
-        PHX_HIP(ce);
-        const hipError_t ie = hipGraphInstantiate(&s->graph, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        PHX_HIP(ie);
-        s->graph_parity = cur;
-        s->graph_dt = s->dt;
-        s->graph_stream = s->stream;
     }
-    PHX_HIP(hipGraphLaunch(s->graph, s->stream));
-    s->t = t_graph;
-    s->fft_cached_t = fc_graph;
-    s->iteration += kGraphSteps;
-    *taken = kGraphSteps;
-    return PHX_OK;
+    if (graphs && s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream && s->graph_parity == s->cur && s->graph_steps <= m) {
+        PHX_HIP(hipGraphLaunch(s->graph, s->stream));
+        return took(advance(s->graph_steps, t, fc));
+    }
+    /* (a run that starts in the other buffer than the captured one is launched too, not captured anew) */
+    for (int64_t k = 0; k < m; k++)
+        if (int r = rk4_launch<real>(s, s->t, s->dt)) return r;
+    s->direct_steps += m;
+    return took(m);
 }
 
 int field_info(phx_solver* s, int field, void*** slot, size_t* elems) {
@@ -1515,8 +1546,9 @@ int phx_get_info(phx_solver* s, phx_info* info) {
     info->dt_max = c.dt_max;
     info->iteration = s->iteration;
     info->rejected = s->rejected;
-    info->tile_rows = s->tuned ? s->tune.ty : 0;
-    info->prefetch_rows = s->tuned ? s->tune.pf : 0;
+    const phx::Rk4Tune& shape = s->flow_launches ? s->flow_tune : s->tune;
+    info->tile_rows = s->tuned ? shape.ty : 0;
+    info->prefetch_rows = s->tuned ? shape.pf : 0;
     info->staged = s->staged;
     info->multi_step_steps = s->flow_steps;
     info->multi_step_launches = s->flow_launches;
@@ -1610,7 +1642,7 @@ static int rk4_device_t(const phx_physics* ph, int N_c, int N_r, int px, int py,
     a.ph = phx::make_phys<real>(c);
     a.pump = (const real*)pump;
     a.pot = (const real*)pot;
-    const phx::Rk4Tune tune = rk4_tune_from_env(phx::Rk4Tune{});
+    const phx::Rk4Tune tune = rk4_tune_from_env(phx::rk4_default_tune(N_c, N_r, sizeof(real)));
     for (int64_t k = 0; k < n_steps; k++) {
         const bool even = (k % 2) == 0;
         a.psi_in = (const v2*)(even ? psi_a : psi_b);
