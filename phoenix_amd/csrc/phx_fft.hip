@@ -744,6 +744,21 @@ hipError_t launch_fft_propagate(typename Vec2<real>::type* psi, const FftAxis& c
     return fft_roundtrip<real, kColPropagate>(psi, c, r, nullptr, rowf, colf, s);
 }
 
+/* the passes of the propagator one by one */
+template <typename real>
+hipError_t launch_fft_rows(typename Vec2<real>::type* psi, const FftAxis& c, int Nr, bool inverse, hipStream_t s) {
+    return inverse ? rows_pass<real, +1>(psi, c, Nr, s) : rows_pass<real, -1>(psi, c, Nr, s);
+}
+template <typename real>
+hipError_t launch_fft_propagate_cols(typename Vec2<real>::type* psi, const FftAxis& r, int Nc, const void* rowf, const void* colf,
+                                     hipStream_t s) {
+    return cols_pass<real, kColPropagate>(psi, r, Nc, nullptr, rowf, colf, s, nullptr);
+}
+
+template hipError_t launch_fft_rows<float>(float2*, const FftAxis&, int, bool, hipStream_t);
+template hipError_t launch_fft_rows<double>(double2*, const FftAxis&, int, bool, hipStream_t);
+template hipError_t launch_fft_propagate_cols<float>(float2*, const FftAxis&, int, const void*, const void*, hipStream_t);
+template hipError_t launch_fft_propagate_cols<double>(double2*, const FftAxis&, int, const void*, const void*, hipStream_t);
 template hipError_t launch_fft_propagate<float>(float2*, const FftAxis&, const FftAxis&, const void*, const void*, hipStream_t);
 template hipError_t launch_fft_propagate<double>(double2*, const FftAxis&, const FftAxis&, const void*, const void*, hipStream_t);
 template hipError_t launch_fft_filter<float>(float2*, const FftAxis&, const FftAxis&, const float*, hipStream_t, float2*);

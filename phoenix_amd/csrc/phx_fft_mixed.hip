@@ -18,327 +18,14 @@
  * registers and the turn costs no LDS trip.  Two LDS buffers take turns, one barrier a pass.
  * Column groups keep their CB columns adjacent in LDS and in the lanes.
  */
-#include "phx_fft_mixed.h"
-
 #include <algorithm>
 #include <cmath>
-#include <cstdlib>
-#include <type_traits>
 
-#include "custom_rhs.h"
-#include "phx_fft_cx.h"
+#include "phx_fft_engine.h"
 
 namespace phx {
 
-/* ------------------------------------------------------------------ transforms in registers */
 namespace {
-
-/* cos and sin of 2 pi k / R at compile time: Taylor series after reduction to |x| <= pi / 4 */
-constexpr double kPi = 3.14159265358979323846264338327950288;
-constexpr double taylor_sin(double x) {
-    double t = x, s = 0;
-    for (int n = 1; n < 24; n += 2) {
-        s += t;
-        t *= -x * x / ((n + 1) * (n + 2));
-    }
-    return s;
-}
-constexpr double taylor_cos(double x) {
-    double t = 1, s = 0;
-    for (int n = 0; n < 24; n += 2) {
-        s += t;
-        t *= -x * x / ((n + 1) * (n + 2));
-    }
-    return s;
-}
-/* cos(2 pi k / R) for 0 <= k: eighths of a turn, exact reduction in integers */
-constexpr double cos_turn(int k, int R) {
-    k %= R;
-    if (2 * k > R) k = R - k;                        /* cos is even: k / R <= 1/2 */
-    if (4 * k > R) return -cos_turn(R - 2 * k, 2 * R); /* cos(pi - x) = -cos x */
-    if (8 * k > R) return taylor_sin(kPi * (R - 4 * k) / (2.0 * R)); /* sin(pi/2 - x) */
-    return taylor_cos(2.0 * kPi * k / R);
-}
-constexpr double sin_turn(int k, int R) { return cos_turn(4 * k + 3 * R, 4 * R); } /* sin x = cos(x - pi/2) */
-
-template <int R>
-struct Roots {
-    double c[R] = {}, s[R] = {};
-    constexpr Roots() {
-        for (int k = 0; k < R; k++) {
-            c[k] = cos_turn(k, R);
-            s[k] = sin_turn(k, R);
-        }
-    }
-};
-template <int R>
-struct RootTable {
-    static constexpr Roots<R> v{};
-};
-
-/* factor of a composite radix that is transformed first */
-constexpr int first_factor(int R) { return R % 4 == 0 && R > 4 ? 4 : R % 2 == 0 ? 2 : R % 3 == 0 ? 3 : R; }
-
-/* forward DFT of R values in registers */
-template <typename real, int R>
-__device__ __forceinline__ void dft(Cx<real> (&x)[R]) {
-    if constexpr (R == 2) {
-        const Cx<real> a = x[0], b = x[1];
-        x[0] = {a.r + b.r, a.i + b.i};
-        x[1] = {a.r - b.r, a.i - b.i};
-    } else if constexpr (R == 4) {
-        const Cx<real> s02 = {x[0].r + x[2].r, x[0].i + x[2].i}, d02 = {x[0].r - x[2].r, x[0].i - x[2].i};
-        const Cx<real> s13 = {x[1].r + x[3].r, x[1].i + x[3].i}, d13 = {x[1].r - x[3].r, x[1].i - x[3].i};
-        x[0] = {s02.r + s13.r, s02.i + s13.i};
-        x[1] = {d02.r + d13.i, d02.i - d13.r};
-        x[2] = {s02.r - s13.r, s02.i - s13.i};
-        x[3] = {d02.r - d13.i, d02.i + d13.r};
-    } else if constexpr (first_factor(R) != R) {
-        /* R = R1 R2: n = R2 n1 + n2, k = k1 + R1 k2 */
-        constexpr int R1 = first_factor(R), R2 = R / R1;
-        Cx<real> y[R2][R1];
-#pragma unroll
-        for (int n2 = 0; n2 < R2; n2++) {
-            Cx<real> t[R1];
-#pragma unroll
-            for (int n1 = 0; n1 < R1; n1++) t[n1] = x[R2 * n1 + n2];
-            dft<real, R1>(t);
-#pragma unroll
-            for (int k1 = 0; k1 < R1; k1++) {
-                const int m = (n2 * k1) % R;
-                y[n2][k1] = m == 0 ? t[k1] : cmul(t[k1], Cx<real>{(real)RootTable<R>::v.c[m], (real)-RootTable<R>::v.s[m]});
-            }
-        }
-#pragma unroll
-        for (int k1 = 0; k1 < R1; k1++) {
-            Cx<real> t[R2];
-#pragma unroll
-            for (int n2 = 0; n2 < R2; n2++) t[n2] = y[n2][k1];
-            dft<real, R2>(t);
-#pragma unroll
-            for (int k2 = 0; k2 < R2; k2++) x[k1 + R1 * k2] = t[k2];
-        }
-    } else {
-        /* odd prime: sums and differences of the pairs k, R - k */
-        constexpr int P = (R - 1) / 2;
-        Cx<real> t[P], u[P];
-        Cx<real> z = x[0];
-#pragma unroll
-        for (int k = 0; k < P; k++) {
-            t[k] = {x[k + 1].r + x[R - 1 - k].r, x[k + 1].i + x[R - 1 - k].i};
-            u[k] = {x[k + 1].r - x[R - 1 - k].r, x[k + 1].i - x[R - 1 - k].i};
-            z.r += t[k].r;
-            z.i += t[k].i;
-        }
-        const Cx<real> x0 = x[0];
-        x[0] = z;
-#pragma unroll
-        for (int j = 1; j <= P; j++) {
-            Cx<real> a = x0, b = {real(0), real(0)};
-#pragma unroll
-            for (int k = 0; k < P; k++) {
-                const int m = (j * (k + 1)) % R;
-                const real c = (real)RootTable<R>::v.c[m], s = (real)RootTable<R>::v.s[m];
-                a.r = phx_fma(c, t[k].r, a.r);
-                a.i = phx_fma(c, t[k].i, a.i);
-                b.r = phx_fma(s, u[k].r, b.r);
-                b.i = phx_fma(s, u[k].i, b.i);
-            }
-            x[j] = {a.r + b.i, a.i - b.r};
-            x[R - j] = {a.r - b.i, a.i + b.r};
-        }
-    }
-}
-
-template <typename real>
-__device__ __forceinline__ Cx<real> swapped(Cx<real> v) {
-    return {v.i, v.r};
-}
-
-/* ------------------------------------------------------------------------------ the passes */
-
-/* Butterfly b of a group of sequences -> (sequence, butterfly of the sequence), and the LDS slot of
-   an element.  Rows: one sequence after the other; columns: the CB columns adjacent. */
-template <int CB>
-struct Lay {
-    static __device__ __forceinline__ void split(int b, int nb, uint32_t m_nb, int& seq, int& bb) {
-        if constexpr (CB > 0) {
-            seq = b % CB;
-            bb = b / CB;
-        } else {
-            seq = nb == 1 ? b : (int)__umulhi((uint32_t)b, m_nb);
-            bb = b - seq * nb;
-        }
-    }
-    static __device__ __forceinline__ int slot(int seq, int idx, int len) {
-        if constexpr (CB > 0)
-            return idx * CB + seq;
-        else
-            return seq * len + idx;
-    }
-};
-
-/* the workgroup's LDS; the two buffers are kept as offsets into it, not as pointers (a pointer that is
-   exchanged in a loop loses its address space, and every access becomes a flat one) */
-template <typename real>
-__device__ __forceinline__ Cx<real>* lds() {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    return reinterpret_cast<Cx<real>*>(lds_raw);
-}
-
-/* entry i of a plan array by selects: the plan is a kernel argument, and an indexed read of it would be a
-   scalar load in the middle of the kernel instead of one of those at its start */
-template <typename T>
-__device__ __forceinline__ T pick(const T (&v)[kFftMaxPasses], int i) {
-    T r = v[0];
-#pragma unroll
-    for (int k = 1; k < kFftMaxPasses; k++) r = i == k ? v[k] : r;
-    return r;
-}
-
-/* One pass of radix R.  Inputs come from rd(seq, idx) when `first`, else from A; outputs go to
-   wr(seq, idx, value) when `last`, else to B (element offsets in LDS). */
-template <typename real, int R, int CB, class RD, class WR>
-__device__ __forceinline__ void one_pass(const FftPlan& pl, int i, int count, bool first, bool last, int A, int B,
-                                         const Cx<real>* __restrict__ tw, RD rd, WR wr) {
-    const int nb = pl.len / R, s = pick(pl.s, i), total = nb * count;
-    const uint32_t m_nb = pick(pl.m_nb, i), m_s = pick(pl.m_s, i);
-    Cx<real>* const L = lds<real>();
-    for (int b = threadIdx.x; b < total; b += blockDim.x) {
-        int seq, bb;
-        Lay<CB>::split(b, nb, m_nb, seq, bb);
-        const int p = s == 1 ? bb : (int)__umulhi((uint32_t)bb, m_s), ps = p * s, q = bb - ps;
-        Cx<real> x[R], w[R];
-#pragma unroll
-        for (int j = 1; j < R; j++) w[j] = tw[last ? 0 : j * ps];
-        if (first) {
-#pragma unroll
-            for (int j = 0; j < R; j++) x[j] = rd(seq, bb + j * nb);
-        } else {
-#pragma unroll
-            for (int j = 0; j < R; j++) x[j] = L[A + Lay<CB>::slot(seq, bb + j * nb, pl.len)];
-        }
-        dft<real, R>(x);
-        if (last) {
-#pragma unroll
-            for (int j = 0; j < R; j++) wr(seq, bb + j * s, x[j]);
-        } else {
-            const int o = q + R * ps;
-            L[B + Lay<CB>::slot(seq, o, pl.len)] = x[0];
-#pragma unroll
-            for (int j = 1; j < R; j++) L[B + Lay<CB>::slot(seq, o + s * j, pl.len)] = cmul(x[j], w[j]);
-        }
-    }
-}
-
-/* The turn of a convolution: the last forward pass, the factor, and the first pass of the inverse
-   (radices reversed, real and imaginary parts swapped), which takes the same elements. */
-template <typename real, int R, int CB, class RD, class FA, class WR>
-__device__ __forceinline__ void turn_pass(const FftPlan& pl, int i, int count, bool first, int A, int B,
-                                          const Cx<real>* __restrict__ tw, RD rd, FA factor, WR wr) {
-    const int nb = pl.len / R, total = nb * count;
-    const uint32_t m_nb = pick(pl.m_nb, i);
-    Cx<real>* const L = lds<real>();
-    for (int b = threadIdx.x; b < total; b += blockDim.x) {
-        int seq, bb;
-        Lay<CB>::split(b, nb, m_nb, seq, bb);
-        Cx<real> x[R], w[R];
-#pragma unroll
-        for (int j = 1; j < R; j++) w[j] = tw[j * bb];
-        if (first) {
-#pragma unroll
-            for (int j = 0; j < R; j++) x[j] = rd(seq, bb + j * nb);
-        } else {
-#pragma unroll
-            for (int j = 0; j < R; j++) x[j] = L[A + Lay<CB>::slot(seq, bb + j * nb, pl.len)];
-        }
-        dft<real, R>(x);
-        factor(seq, bb, nb, x);
-#pragma unroll
-        for (int j = 0; j < R; j++) x[j] = swapped(x[j]);
-        dft<real, R>(x);
-        if (first) { /* a single pass: the whole transform */
-#pragma unroll
-            for (int j = 0; j < R; j++) wr(seq, bb + j, x[j]);
-        } else {
-            L[B + Lay<CB>::slot(seq, R * bb, pl.len)] = x[0];
-#pragma unroll
-            for (int j = 1; j < R; j++) L[B + Lay<CB>::slot(seq, R * bb + j, pl.len)] = cmul(x[j], w[j]);
-        }
-    }
-}
-
-/* run `f` with the radix as a compile-time constant, out of a family of radices: 0 the powers of two,
-   1 with 3, 5, 9 and 10, 2 with 7, 11 and 13 too.  Every pass of a kernel holds the code of its whole
-   family, and the instruction cache is 64 KiB for two CUs: a filter of 646 x 646 (Bluestein, 2048
-   points) takes 100 us FP64 / 60 us FP32 with family 0 and 122 / 77 with family 1. */
-template <int FAM, class F>
-__device__ __forceinline__ void with_radix(int r, F f) {
-    switch (r) {
-        case 2: f(std::integral_constant<int, 2>{}); return;
-        case 4: f(std::integral_constant<int, 4>{}); return;
-        case 8: f(std::integral_constant<int, 8>{}); return;
-        case 16: f(std::integral_constant<int, 16>{}); return;
-        default: break;
-    }
-    if constexpr (FAM >= 1) {
-        switch (r) {
-            case 3: f(std::integral_constant<int, 3>{}); return;
-            case 5: f(std::integral_constant<int, 5>{}); return;
-            case 9: f(std::integral_constant<int, 9>{}); return;
-            case 10: f(std::integral_constant<int, 10>{}); return;
-            default: break;
-        }
-    }
-    if constexpr (FAM >= 2) {
-        switch (r) {
-            case 7: f(std::integral_constant<int, 7>{}); return;
-            case 11: f(std::integral_constant<int, 11>{}); return;
-            case 13: f(std::integral_constant<int, 13>{}); return;
-            default: break;
-        }
-    }
-}
-
-/* forward transform of `count` sequences: rd -> wr */
-template <typename real, int CB, int FAM, class RD, class WR>
-__device__ __forceinline__ void transform(const FftPlan& pl, int count, int A, int B, const Cx<real>* __restrict__ tw,
-                                          RD rd, WR wr) {
-    for (int i = 0; i < pl.passes; i++) {
-        const bool last = i == pl.passes - 1;
-        with_radix<FAM>(pick(pl.radix, i), [&](auto R) { one_pass<real, decltype(R)::value, CB>(pl, i, count, i == 0, last, A, B, tw, rd, wr); });
-        if (!last) __syncthreads();
-        const int t = A;
-        A = B;
-        B = t;
-    }
-}
-
-/* forward, factor, inverse (its real and imaginary parts still swapped when they reach wr).  The
-   last pass reads the buffer that is returned as the second one: the first is free for wr. */
-template <typename real, int CB, int FAM, class RD, class FA, class WR>
-__device__ __forceinline__ void convolve(const FftPlan& fwd, const FftPlan& inv, int count, int& A, int& B,
-                                         const Cx<real>* __restrict__ tw, RD rd, FA factor, WR wr) {
-    const int last_fwd = fwd.passes - 1;
-    auto flip = [&] {
-        const int t = A;
-        A = B;
-        B = t;
-    };
-    for (int i = 0; i < last_fwd; i++) {
-        with_radix<FAM>(pick(fwd.radix, i), [&](auto R) { one_pass<real, decltype(R)::value, CB>(fwd, i, count, i == 0, false, A, B, tw, rd, wr); });
-        __syncthreads();
-        flip();
-    }
-    with_radix<FAM>(pick(fwd.radix, last_fwd),
-                     [&](auto R) { turn_pass<real, decltype(R)::value, CB>(fwd, last_fwd, count, last_fwd == 0, A, B, tw, rd, factor, wr); });
-    for (int i = 1; i <= last_fwd; i++) {
-        __syncthreads();
-        flip();
-        const bool last = i == last_fwd;
-        with_radix<FAM>(pick(inv.radix, i), [&](auto R) { one_pass<real, decltype(R)::value, CB>(inv, i, count, false, last, A, B, tw, rd, wr); });
-    }
-}
 
 /* k-space factor of the column pass at column c, row k of the spectrum (k = 0 first) */
 template <typename real>
@@ -368,8 +55,6 @@ struct ColFactor {
         return f;
     }
 };
-
-constexpr int kMixThreads = 256;
 
 } // namespace
 
@@ -474,15 +159,6 @@ __global__ __launch_bounds__(kMixThreads) void mixed_cols(typename Vec2<real>::t
 
 /* ------------------------------------------------------------------------------- host side */
 namespace {
-
-constexpr size_t kMixLdsMax = 128 * 1024; /* of the 160 KiB a gfx950 workgroup may hold */
-
-int largest_prime(int n) {
-    int big = 1;
-    for (int p = 2; p * p <= n; p++)
-        while (n % p == 0) big = p, n /= p;
-    return n > 1 ? std::max(big, n) : big;
-}
 
 constexpr int kRadices[] = {2, 3, 4, 5, 7, 8, 9, 10, 11, 13, 16};
 
@@ -600,36 +276,12 @@ std::vector<std::complex<double>> fft_axis_table(const FftAxis& a) {
     return t;
 }
 
-/* family of radices (with_radix) that splits a length */
-static int family(int len) {
-    const int p = largest_prime(len);
-    return p <= 2 ? 0 : p <= 5 ? 1 : 2;
-}
-
-/* threads of a workgroup with `work` butterflies in its widest pass */
-static int mixed_threads(int work) { return std::min(kMixThreads, (work + 63) / 64 * 64); }
-
-static int smallest_radix(const FftPlan& p) {
-    int r = p.radix[0];
-    for (int i = 1; i < p.passes; i++) r = std::min(r, p.radix[i]);
-    return r;
-}
-
-template <typename K>
-static hipError_t allow_lds(K kernel, size_t lds) {
-    return lds > 65536 ? hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMixLdsMax) : hipSuccess;
-}
-
 template <typename real>
 hipError_t launch_mixed_rows(typename Vec2<real>::type* data, const FftAxis& c, int Nr, bool inverse, hipStream_t s) {
     const int len = c.fwd.len;
     const size_t per = 2 * (size_t)len * sizeof(Cx<real>);
     if (!c.fwd.passes || per > kMixLdsMax) return hipErrorInvalidValue;
-    const int wide = len / smallest_radix(c.fwd); /* butterflies of a row in the widest pass */
-    /* as few rows per workgroup as fill its waves: the transforms wait on LDS and L2, and more, smaller
-       workgroups spread the waits (400 x 400 FP64: 1 row 23.2 us a filter, 3 rows 23.3; 1500 x 1500 FP32
-       67.0 / 69.4; 138 x 158 FP64, Bluestein, 27.3 / 30.9 for 1 and 4 rows) */
-    const int rpb = std::max(1, 64 / wide);
+    const int wide = widest_pass(c.fwd), rpb = rows_per_block(c.fwd);
     const dim3 grid((Nr + rpb - 1) / rpb), blk(mixed_threads(wide * rpb));
     const auto* t = (const Cx<real>*)c.table;
     auto go = [&](auto kernel) {
@@ -638,14 +290,14 @@ hipError_t launch_mixed_rows(typename Vec2<real>::type* data, const FftAxis& c, 
         hipLaunchKernelGGL(kernel, grid, blk, per * rpb, s, data, c.fwd, c.inv, c.N, Nr, rpb, (int)inverse, t);
         return hipGetLastError();
     };
-    if (c.M) return family(len) == 0 ? go(&mixed_rows<real, true, 0>) : go(&mixed_rows<real, true, 1>);
-    return family(len) < 2 ? go(&mixed_rows<real, false, 1>) : go(&mixed_rows<real, false, 2>);
+    if (c.M) return radix_family(len) == 0 ? go(&mixed_rows<real, true, 0>) : go(&mixed_rows<real, true, 1>);
+    return radix_family(len) < 2 ? go(&mixed_rows<real, false, 1>) : go(&mixed_rows<real, false, 2>);
 }
 
 template <typename real, int CB, bool BLUE, int FAM>
 static hipError_t cols_cb(typename Vec2<real>::type* data, const FftAxis& r, const ColFactor<real>& f, hipStream_t s) {
     const size_t lds = 2 * (size_t)CB * r.fwd.len * sizeof(Cx<real>);
-    const dim3 grid((f.Nc + CB - 1) / CB), blk(mixed_threads(CB * (r.fwd.len / smallest_radix(r.fwd))));
+    const dim3 grid((f.Nc + CB - 1) / CB), blk(mixed_threads(CB * widest_pass(r.fwd)));
     auto go = [&](auto kernel) {
         const hipError_t e = allow_lds(kernel, lds);
         if (e != hipSuccess) return e;
@@ -665,7 +317,7 @@ hipError_t launch_mixed_cols(typename Vec2<real>::type* data, const FftAxis& r, 
        each 128-byte line (600 x 600 FP64: 39.5 us a filter with one, 32.9 with two, 36.5 with four; 1500 x
        1500 FP64, 96 KiB for two, 104 / 120).  Bluestein's lengths take one: their buffers are twice to four
        times as long (1030 x 1030 FP32: 185 / 223) */
-    const int fam = family(r.fwd.len);
+    const int fam = radix_family(r.fwd.len);
     if (r.M) return fam == 0 ? cols_cb<real, 1, true, 0>(data, r, f, s) : cols_cb<real, 1, true, 1>(data, r, f, s);
     if (2 * per <= 65536 && Nc > 1)
         return fam < 2 ? cols_cb<real, 2, false, 1>(data, r, f, s) : cols_cb<real, 2, false, 2>(data, r, f, s);

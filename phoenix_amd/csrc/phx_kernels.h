@@ -322,6 +322,13 @@ template <typename real>
 hipError_t launch_fft_propagate(typename Vec2<real>::type* psi, const FftAxis& c, const FftAxis& r, const void* rowf, const void* colf,
                                 hipStream_t s);
 
+/* its passes: the row transforms, and the columns' forward transform, factor and inverse */
+template <typename real>
+hipError_t launch_fft_rows(typename Vec2<real>::type* psi, const FftAxis& c, int Nr, bool inverse, hipStream_t s);
+template <typename real>
+hipError_t launch_fft_propagate_cols(typename Vec2<real>::type* psi, const FftAxis& r, int Nc, const void* rowf, const void* colf,
+                                     hipStream_t s);
+
 /* Pointwise parts of the split-step Fourier iterator (phx_ssfm.hip).  Index 0 = plus, 1 = minus. */
 template <typename real>
 struct SsfmArgs {
@@ -346,6 +353,10 @@ struct SsfmArgs {
 };
 template <typename real>
 hipError_t launch_ssfm_nonlinear(const SsfmArgs<real>& a, hipStream_t s);
+/* inverse row transform, the nonlinear step (or the pulse), forward row transform (phx_ssfm_rows.hip): scalar
+   model, real reservoir; n_nxt may be n_cur */
+template <typename real>
+hipError_t launch_ssfm_rows(const SsfmArgs<real>& a, const FftAxis& c, int Nr, bool pulse, hipStream_t s);
 template <typename real>
 hipError_t launch_ssfm_independent(const SsfmArgs<real>& a, hipStream_t s);
 

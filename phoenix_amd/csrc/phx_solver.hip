@@ -82,8 +82,10 @@ struct phx_solver {
     double* sums_host = nullptr; /* pinned host copy */
     const phx::IteratorInfo* iter = nullptr; /* registry entry of cfg.iterator (nullptr for SSFM) */
     bool ssfm = false;                        /* split-step Fourier iterator */
-    void* ssfm_rowf = nullptr;                /* linear half-step factors along rows (N_r) and columns (N_c) */
-    void* ssfm_colf = nullptr;
+    /* linear factors along rows (N_r) and columns (N_c): of a half step, and of the two half steps that meet
+       between the nonlinear steps of a run */
+    void* ssfm_rowf[2] = {nullptr, nullptr};
+    void* ssfm_colf[2] = {nullptr, nullptr};
     double ssfm_dt = -1.0;                    /* dt the factors were made for */
     int max_rejections = 10000;
     double last_error = 0; /* E of the last adaptive attempt */
@@ -294,8 +296,10 @@ int initialize_t(phx_solver* s) {
         if (int r = dev_alloc(s, (void**)&s->norm_sums, 2 * sizeof(double))) return r;
     }
     if (s->ssfm) {
-        if (int r = dev_alloc(s, &s->ssfm_rowf, 2 * (size_t)c.N_r * sizeof(real))) return r;
-        if (int r = dev_alloc(s, &s->ssfm_colf, 2 * (size_t)c.N_c * sizeof(real))) return r;
+        for (int w = 0; w < 2; w++) {
+            if (int r = dev_alloc(s, &s->ssfm_rowf[w], 2 * (size_t)c.N_r * sizeof(real))) return r;
+            if (int r = dev_alloc(s, &s->ssfm_colf[w], 2 * (size_t)c.N_c * sizeof(real))) return r;
+        }
     }
     if (c.use_fft_mask || s->ssfm || s->spec[0]) {
         for (phx::FftAxis* ax : {&s->fft_c, &s->fft_r}) {
@@ -679,24 +683,32 @@ int spectrum_ready_t(phx_solver* s) {
    and kept as a row table and a column table, remade when dt changes.  psi is updated in
    place; the reservoir goes through the spare buffer. */
 template <typename real>
-int ssfm_step(phx_solver* s, double t_pre) {
+int ssfm_tables(phx_solver* s) {
     auto& c = s->cfg;
-    using v2 = typename phx::Vec2<real>::type;
-    if (s->ssfm_dt != s->dt) {
-        const double dt = s->dt, lin = c.h_bar_s / 2.0 / c.m_eff;
+    if (s->ssfm_dt == s->dt) return PHX_OK;
+    const double dt = s->dt, lin = c.h_bar_s / 2.0 / c.m_eff;
+    for (int w = 0; w < 2; w++) { /* one half step, two half steps */
         std::vector<std::complex<double>> rowf(c.N_r), colf(c.N_c);
         for (int r = 0; r < c.N_r; r++) {
             const double ky = 2.0 * 3.1415926535 * (double)(r <= c.N_r / 2 ? r : r - c.N_r) / c.L_y;
-            rowf[r] = std::polar(1.0, -lin * ky * ky * dt / 2.0) / ((double)c.N_c * (double)c.N_r);
+            rowf[r] = std::polar(1.0, (w + 1) * (-lin * ky * ky * dt / 2.0)) / ((double)c.N_c * (double)c.N_r);
         }
         for (int col = 0; col < c.N_c; col++) {
             const double kx = 2.0 * 3.1415926535 * (double)(col <= c.N_c / 2 ? col : col - c.N_c) / c.L_x;
-            colf[col] = std::polar(1.0, -lin * kx * kx * dt / 2.0);
+            colf[col] = std::polar(1.0, (w + 1) * (-lin * kx * kx * dt / 2.0));
         }
-        if (int r = upload_complex<real>(s, s->ssfm_rowf, rowf)) return r;
-        if (int r = upload_complex<real>(s, s->ssfm_colf, colf)) return r;
-        s->ssfm_dt = s->dt;
+        if (int r = upload_complex<real>(s, s->ssfm_rowf[w], rowf)) return r;
+        if (int r = upload_complex<real>(s, s->ssfm_colf[w], colf)) return r;
     }
+    s->ssfm_dt = s->dt;
+    return PHX_OK;
+}
+
+/* arguments of the pointwise parts of the step that starts at t_pre */
+template <typename real>
+phx::SsfmArgs<real> ssfm_args(phx_solver* s, double t_pre) {
+    auto& c = s->cfg;
+    using v2 = typename phx::Vec2<real>::type;
     const int ncomp = c.tetm ? 2 : 1;
     phx::SsfmArgs<real> a{};
     const size_t N = s->cells();
@@ -746,12 +758,96 @@ int ssfm_step(phx_solver* s, double t_pre) {
     a.cres = c.complex_reservoir;
     a.dt = (real)s->dt;
     a.ph = phys_of<real>(s);
+    /* the real reservoir of the scalar model without noise is updated in place */
+    if (!c.tetm && !c.complex_reservoir && !c.use_stochastic) a.n_nxt[0] = a.n_cur[0];
+    return a;
+}
+
+template <typename real>
+int ssfm_step(phx_solver* s, double t_pre) {
+    auto& c = s->cfg;
+    if (int r = ssfm_tables<real>(s)) return r;
+    const phx::SsfmArgs<real> a = ssfm_args<real>(s, t_pre);
+    if (!c.tetm && !c.complex_reservoir) {
+        PHX_HIP(phx::launch_fft_rows<real>(a.psi[0], s->fft_c, c.N_r, false, s->stream));
+        PHX_HIP(phx::launch_fft_propagate_cols<real>(a.psi[0], s->fft_r, c.N_c, s->ssfm_rowf[0], s->ssfm_colf[0], s->stream));
+        PHX_HIP(phx::launch_ssfm_rows<real>(a, s->fft_c, c.N_r, false, s->stream));
+        PHX_HIP(phx::launch_fft_propagate_cols<real>(a.psi[0], s->fft_r, c.N_c, s->ssfm_rowf[0], s->ssfm_colf[0], s->stream));
+        PHX_HIP(phx::launch_fft_rows<real>(a.psi[0], s->fft_c, c.N_r, true, s->stream));
+        if (a.npulse || a.stochastic) PHX_HIP(phx::launch_ssfm_independent<real>(a, s->stream));
+        return PHX_OK;
+    }
+    const int ncomp = c.tetm ? 2 : 1;
     for (int k = 0; k < ncomp; k++)
-        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->fft_c, s->fft_r, s->ssfm_rowf, s->ssfm_colf, s->stream));
+        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->fft_c, s->fft_r, s->ssfm_rowf[0], s->ssfm_colf[0], s->stream));
     PHX_HIP(phx::launch_ssfm_nonlinear<real>(a, s->stream));
     for (int k = 0; k < ncomp; k++)
-        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->fft_c, s->fft_r, s->ssfm_rowf, s->ssfm_colf, s->stream));
+        PHX_HIP(phx::launch_fft_propagate<real>(a.psi[k], s->fft_c, s->fft_r, s->ssfm_rowf[0], s->ssfm_colf[0], s->stream));
     PHX_HIP(phx::launch_ssfm_independent<real>(a, s->stream));
+    return PHX_OK;
+}
+
+/* Time and FFT guard after up to `lim` steps that neither reach t_max, pass t_stop (the caller shortens that
+   one) nor fire the k-space filter, as iterate() would advance them; returns the steps. */
+int64_t advance_steps(const phx_solver* s, int64_t lim, double t_stop, double& t, double& fc) {
+    const auto& c = s->cfg;
+    t = s->t;
+    fc = s->fft_cached_t;
+    int64_t m = 0;
+    for (; m < lim && t < c.t_max && t < t_stop; m++) {
+        const double tn = s->rnd(t + s->dt);
+        if (tn > t_stop) break;
+        if (!(s->rnd(tn - fc) < c.fft_every)) {
+            if (c.use_fft_mask || s->spec[0]) break;
+            fc = tn;
+        }
+        t = tn;
+    }
+    return m;
+}
+
+/* A run of split steps of the scalar model without noise and filter: the linear half steps that end one step
+   and begin the next are one column pass with both factors, and without a pulse between them the row
+   transforms there cancel.  A step is then two passes over psi instead of eight.  Pulses enter in the row
+   pass between the half steps.  *taken: the steps run (0: not eligible). */
+constexpr int64_t kSsfmMaxSteps = 500;
+
+template <typename real>
+int ssfm_block(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
+    auto& c = s->cfg;
+    *taken = 0;
+    if (c.tetm || c.complex_reservoir || c.use_stochastic || c.imag_time_amplitude != 0.0) return PHX_OK;
+    double t, fc;
+    const int64_t m = advance_steps(s, std::min(max_steps, kSsfmMaxSteps), t_stop, t, fc);
+    if (m < 2) return PHX_OK;
+    if (int r = ssfm_tables<real>(s)) return r;
+    double tk = s->t;
+    phx::SsfmArgs<real> a = ssfm_args<real>(s, tk);
+    auto cols = [&](int w) {
+        return phx::launch_fft_propagate_cols<real>(a.psi[0], s->fft_r, c.N_c, s->ssfm_rowf[w], s->ssfm_colf[w], s->stream);
+    };
+    PHX_HIP(phx::launch_fft_rows<real>(a.psi[0], s->fft_c, c.N_r, false, s->stream));
+    PHX_HIP(cols(0));
+    for (int64_t k = 0; k < m; k++) {
+        if (k > 0) a = ssfm_args<real>(s, tk);
+        PHX_HIP(phx::launch_ssfm_rows<real>(a, s->fft_c, c.N_r, false, s->stream));
+        if (k == m - 1) break;
+        if (a.npulse) {
+            PHX_HIP(cols(0));
+            PHX_HIP(phx::launch_ssfm_rows<real>(a, s->fft_c, c.N_r, true, s->stream));
+            PHX_HIP(cols(0));
+        } else {
+            PHX_HIP(cols(1));
+        }
+        tk = s->rnd(tk + s->dt);
+    }
+    PHX_HIP(cols(0));
+    PHX_HIP(phx::launch_fft_rows<real>(a.psi[0], s->fft_c, c.N_r, true, s->stream));
+    if (a.npulse) PHX_HIP(phx::launch_ssfm_independent<real>(a, s->stream));
+    s->t = t;
+    s->fft_cached_t = fc;
+    s->iteration += m;
+    *taken = m;
     return PHX_OK;
 }
 
@@ -1131,28 +1227,13 @@ template <typename real>
 int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     auto& c = s->cfg;
     *taken = 0;
+    if (s->ssfm) return ssfm_block<real>(s, max_steps, t_stop, taken);
     const auto constant = [](const phx::Envelope& e) { return e.groupSize() != 1 || e.allConstant(); };
     if (!s->tuned || s->staged || c.iterator != "RK4" || c.tetm || c.use_stochastic || c.imag_time_amplitude != 0.0 ||
         !constant(c.pump) || !constant(c.potential))
         return PHX_OK;
-    /* time and FFT guard after up to `lim` steps that neither reach t_max, pass t_stop nor fire the filter */
-    auto advance = [&](int64_t lim, double& t, double& fc) {
-        t = s->t;
-        fc = s->fft_cached_t;
-        int64_t m = 0;
-        for (; m < lim && t < c.t_max && t < t_stop; m++) {
-            const double tn = s->rnd(t + s->dt);
-            if (tn > t_stop) break;
-            if (!(s->rnd(tn - fc) < c.fft_every)) {
-                if (c.use_fft_mask || s->spec[0]) break;
-                fc = tn;
-            }
-            t = tn;
-        }
-        return m;
-    };
     double t, fc;
-    int64_t m = advance(std::min(max_steps, kFlowMaxSteps), t, fc);
+    const int64_t m = advance_steps(s, std::min(max_steps, kFlowMaxSteps), t_stop, t, fc);
     auto took = [&](int64_t n) {
         s->t = t;
         s->fft_cached_t = fc;
@@ -1199,7 +1280,7 @@ int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     }
     if (graphs && s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream && s->graph_parity == s->cur && s->graph_steps <= m) {
         PHX_HIP(hipGraphLaunch(s->graph, s->stream));
-        return took(advance(s->graph_steps, t, fc));
+        return took(advance_steps(s, s->graph_steps, t_stop, t, fc));
     }
     /* (a run that starts in the other buffer than the captured one is launched too, not captured anew) */
     for (int64_t k = 0; k < m; k++)

@@ -22,7 +22,9 @@
  * through the same formulas: the exponent gains dt g_r Im n / hbar in its real part and
  * dt R Im n / 2 in its phase, the reservoir step takes sum_g P_g a_g whole, and the noise
  * amplitude is the principal complex square root of (R n + gamma_c) / (4 dV).
- * One thread per cell, coalesced; the fields are the solver's full-grid arrays.
+ * One thread per cell, coalesced; the fields are the solver's full-grid arrays.  The nonlinear step of the
+ * scalar model with a real reservoir is part of the row pass between the two half steps
+ * (phx_ssfm_rows.hip).
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -30,15 +32,9 @@
 #include "custom_rhs.h"
 #include "phx_kernels.h"
 #include "phx_noise.h"
+#include "phx_ssfm_cell.h"
 
 namespace phx {
-
-namespace {
-__device__ __forceinline__ void phx_sincos_dev(float x, float& s, float& c) { sincosf(x, &s, &c); }
-__device__ __forceinline__ void phx_sincos_dev(double x, double& s, double& c) { sincos(x, &s, &c); }
-__device__ __forceinline__ float phx_exp_dev(float x) { return expf(x); }
-__device__ __forceinline__ double phx_exp_dev(double x) { return exp(x); }
-} // namespace
 
 template <typename real, bool TETM, bool CRES>
 __global__ __launch_bounds__(256) void ssfm_nonlinear(SsfmArgs<real> a) {
@@ -156,8 +152,9 @@ __global__ __launch_bounds__(256) void ssfm_independent(SsfmArgs<real> a) {
         p.y += di;
         a.psi[k][i] = p;
     }
-    /* scalar model: the new reservoir becomes current (TE-TM keeps the old one) */
-    if (!TETM && a.n_nxt[0]) {
+    /* scalar model: the new reservoir becomes current (TE-TM keeps the old one; without noise the real one
+       was updated in place) */
+    if (!TETM && a.n_nxt[0] && a.n_nxt[0] != a.n_cur[0]) {
         if constexpr (CRES)
             reinterpret_cast<v2*>(a.n_cur[0])[i] = reinterpret_cast<const v2*>(a.n_nxt[0])[i];
         else
@@ -168,15 +165,14 @@ __global__ __launch_bounds__(256) void ssfm_independent(SsfmArgs<real> a) {
 template <typename real>
 hipError_t launch_ssfm_nonlinear(const SsfmArgs<real>& a, hipStream_t s) {
     const dim3 grid((unsigned)((a.cells + 255) / 256));
+    if (!a.tetm && !a.cres) return hipErrorInvalidValue; /* launch_ssfm_rows */
     if (a.cres && !a.n_cur[0]) return hipErrorInvalidValue;
     if (a.tetm && a.cres)
         hipLaunchKernelGGL((ssfm_nonlinear<real, true, true>), grid, dim3(256), 0, s, a);
     else if (a.tetm)
         hipLaunchKernelGGL((ssfm_nonlinear<real, true, false>), grid, dim3(256), 0, s, a);
-    else if (a.cres)
-        hipLaunchKernelGGL((ssfm_nonlinear<real, false, true>), grid, dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL((ssfm_nonlinear<real, false, false>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((ssfm_nonlinear<real, false, true>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
