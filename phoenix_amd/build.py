@@ -37,14 +37,14 @@ HIP_FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-Wno-unuse
 # does the FP64 RK4 kernel at 24 rows with 8 prefetched rows (4 KiB of scratch per lane without it).
 _UNROLL = ["-mllvm", "-pragma-unroll-threshold=2000000"]
 HIP_FLAGS_FILE = {f: _UNROLL for f in ("phx_rk_generic.hip", "phx_rk_tab3.hip", "phx_rk_tab4.hip", "phx_rk_tab6.hip",
-                                     "phx_rk_tab6f.hip", "phx_rk_dp45t.hip", "phx_rk4_f64.hip", "phx_rk_chain.hip")}
+                                     "phx_rk_tab6f.hip", "phx_rk_dp45t.hip", "phx_rk_dp45.hip", "phx_rk4_f64.hip", "phx_rk4_batch_f64.hip", "phx_rk_chain.hip")}
 # The mixed-radix transforms hold every radix in one kernel: hoisting the roots of unity of all of them
 # out of the pass loop costs hundreds of scalar spills before the first pass.
 HIP_FLAGS_FILE["phx_fft_mixed.hip"] = HIP_FLAGS_FILE["phx_ssfm_rows.hip"] = ["-mllvm", "-disable-machine-licm"]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-I", os.path.join(ROOT, "include")]
 
 # longest compiles first: the thread pool then finishes them side by side
-HIP_SOURCES = ["phx_rk_generic.hip", "phx_rk_chain.hip", "phx_rk_dp45t.hip", "phx_rk4_f64.hip", "phx_rk4.hip", "phx_rk4_flow.hip", "phx_rk4_flow_f64.hip", "phx_rk_tab6.hip", "phx_rk_tab6f.hip", "phx_rk_tab4.hip",
+HIP_SOURCES = ["phx_rk_generic.hip", "phx_rk_chain.hip", "phx_rk_dp45t.hip", "phx_rk_dp45.hip", "phx_rk4_f64.hip", "phx_rk4_batch_f64.hip", "phx_rk4.hip", "phx_rk4_batch.hip", "phx_rk4_flow.hip", "phx_rk4_flow_f64.hip", "phx_rk_tab6.hip", "phx_rk_tab6f.hip", "phx_rk_tab4.hip",
                "phx_rk_tab3.hip", "phx_fft_mixed.hip", "phx_ssfm_rows.hip", "phx_fft.hip", "phx_solver.hip", "phx_ensemble.hip", "phx_adjoint.hip", "phx_ssfm.hip",
                "phx_staged.hip"]
 CXX_SOURCES = ["phx_config.cpp"]

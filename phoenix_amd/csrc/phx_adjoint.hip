@@ -24,7 +24,7 @@
  * i-6.  Every stage value lives in an 8-row register window indexed modulo 8,
  * so the row loop is unrolled 8 times whatever the tile height (a runtime
  * value): the code size does not grow with the tile.  Stages are evaluated on
- * every row of the loop, valid or not (only the store is guarded): a slot
+ * every row of the loop, valid or not (an invalid row's stores are out of range): a slot
  * that is written on every pass is dead between its last read and the next
  * write, which keeps the windows in about half the registers that
  * conditionally written slots would hold.  Rows where a stage is not valid
@@ -71,12 +71,6 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
     const int local = gw - item * a.tiles_per_item;
     const int strip = local % a.nstrips, band = local / a.nstrips;
     const size_t so = (size_t)item * a.item_stride, po = (size_t)item * a.param_stride;
-    const v2* psi = a.psi + so;
-    const real* nres = RES ? a.n + so : nullptr;
-    const v2* lpsi = a.lam_psi_in + so;
-    const real* lres = RES ? a.lam_n_in + so : nullptr;
-    const real* pump = PUMP ? a.pump + po : nullptr;
-    const real* pot = POT ? a.pot + po : nullptr;
 
     const int TY = a.ty;
     const int E = TY + 2 * kAdjHalo;
@@ -93,9 +87,25 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
     }
     const uint32_t off_r = col_in ? (uint32_t)gcol * (uint32_t)sizeof(real) : kOutOfRange;
     const uint32_t off_c = col_in ? (uint32_t)gcol * (uint32_t)sizeof(v2) : kOutOfRange;
+    /* halo lanes and lanes past the last column write nothing */
     const bool out_lane = lane >= kAdjHalo && lane < kWave - kAdjHalo && (x0 - kAdjHalo + lane) < Nc;
-    const uint32_t rbytes = (uint32_t)Nc * (uint32_t)sizeof(real);
-    const uint32_t cbytes = (uint32_t)Nc * (uint32_t)sizeof(v2);
+    const uint32_t so_r = out_lane ? (uint32_t)(x0 - kAdjHalo + lane) * (uint32_t)sizeof(real) : kOutOfRange;
+    const uint32_t so_c = out_lane ? (uint32_t)(x0 - kAdjHalo + lane) * (uint32_t)sizeof(v2) : kOutOfRange;
+    /* one descriptor per array of the item; the row is part of the lane offset, and what lies outside a
+       zero-boundary domain, the tile or the grid gets the out-of-range offset (reads 0, writes nothing).  An
+       array that is absent has no records. */
+    const uint32_t row_r = (uint32_t)Nc * (uint32_t)sizeof(real), row_c = (uint32_t)Nc * (uint32_t)sizeof(v2);
+    const uint32_t all_r = row_r * (uint32_t)Nr, all_c = row_c * (uint32_t)Nr;
+    const rsrc_t d_x = row_rsrc(a.psi + so, all_c), d_l = row_rsrc(a.lam_psi_in + so, all_c), d_o = row_rsrc(a.lam_psi_out + so, all_c);
+    const rsrc_t d_xn = row_rsrc(RES ? a.n + so : nullptr, RES ? all_r : 0u);
+    const rsrc_t d_ln = row_rsrc(RES ? a.lam_n_in + so : nullptr, RES ? all_r : 0u);
+    const rsrc_t d_on = row_rsrc(RES ? a.lam_n_out + so : nullptr, RES ? all_r : 0u);
+    const rsrc_t d_p = row_rsrc(PUMP ? a.pump + po : nullptr, PUMP ? all_r : 0u);
+    const rsrc_t d_v = row_rsrc(POT ? a.pot + po : nullptr, POT ? all_r : 0u);
+    const bool gp_on = RES && a.g_pump, gv_on = a.g_pot != nullptr;
+    const rsrc_t d_gp = row_rsrc(gp_on ? a.g_pump + so : nullptr, gp_on ? all_r : 0u);
+    const rsrc_t d_gv = row_rsrc(gv_on ? a.g_pot + so : nullptr, gv_on ? all_r : 0u);
+    const RowWrap wrap = make_row_wrap(Nr, kAdjHalo);
 
     PhxPhys<real> ph = a.ph;
     ph.mhalf_gamma_c = in_vgpr(ph.mhalf_gamma_c);
@@ -121,28 +131,31 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
     }
 
     auto load_row = [&](int r, int sl) {
-        int grow = y0 - kAdjHalo + r;
-        bool in = r < E; /* rows past the tile read as zero (no memory access) */
-        if (in && (grow < 0 || grow >= Nr)) {
-            if (a.periodic_y)
-                grow = ((grow % Nr) + Nr) % Nr;
-            else
-                in = false;
-        }
-        const size_t row = (size_t)(in ? grow : 0) * (size_t)Nc;
-        const v2 x = load_cplx<real>(row_rsrc(psi + row, in ? cbytes : 0u), off_c);
+        bool in;
+        const uint32_t grow = tile_row(y0 - kAdjHalo + r, wrap, a.periodic_y, in); /* wave-uniform */
+        in = in && r < E;                                                         /* rows past the tile read as zero */
+        const uint32_t vc = in ? off_c + grow * row_c : kOutOfRange;
+        const uint32_t vr = in ? off_r + grow * row_r : kOutOfRange;
+        const v2 x = load_cplx<real>(d_x, vc);
         xu[sl] = x.x;
         xv[sl] = x.y;
-        const v2 l = load_cplx<real>(row_rsrc(lpsi + row, in ? cbytes : 0u), off_c);
+        const v2 l = load_cplx<real>(d_l, vc);
         lu[sl] = l.x;
         lv[sl] = l.y;
         if (RES) {
-            xn[sl] = load_real<real>(row_rsrc(nres + row, in ? rbytes : 0u), off_r);
-            ln[sl] = load_real<real>(row_rsrc(lres + row, in ? rbytes : 0u), off_r);
+            xn[sl] = load_real<real>(d_xn, vr);
+            ln[sl] = load_real<real>(d_ln, vr);
         }
-        if (PUMP) pp[sl] = load_real<real>(row_rsrc(pump + row, in ? rbytes : 0u), off_r);
-        if (POT) vv[sl] = load_real<real>(row_rsrc(pot + row, in ? rbytes : 0u), off_r);
+        if (PUMP) pp[sl] = load_real<real>(d_p, vr);
+        if (POT) vv[sl] = load_real<real>(d_v, vr);
     };
+    /* the row written at tile row e: its offset, or out of range */
+    auto out_row = [&](int e, uint32_t lane_off, uint32_t row_bytes) {
+        const int grow = y0 + e - kAdjHalo;
+        return e >= kAdjHalo && e <= E - 1 - kAdjHalo && grow < Nr ? lane_off + (uint32_t)grow * row_bytes : kOutOfRange;
+    };
+    /* gradients accumulated so far at the row written next: read an iteration ahead */
+    real gp_old = load_real<real>(d_gp, out_row(-kPF - 6, so_r, row_r)), gv_old = load_real<real>(d_gv, out_row(-kPF - 6, so_r, row_r));
     /* neighbour part kin_x (W + (E + r (N+S))) of the stencil, r = kin_y / kin_x (the RHS
        hooks add the centre); for dx == dy r is 1 and its multiply is skipped */
     const real kin_yx = ph.kin_yx;
@@ -162,12 +175,15 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
         for (int j = 0; j < kWin; ++j) {
             const int it = base + j;
             load_row(it + kPF, slot(j, kPF));
+            const uint32_t g_next = out_row(it + 1 - 6, so_r, row_r);
+            const real gp_next = load_real<real>(d_gp, g_next), gv_next = load_real<real>(d_gv, g_next);
             /* ---- F1 at e = it-1: Y_2 = x + dt/2 f(x) */
             {
-                const int e = it - 1, s = slot(j, -1), sn = slot(j, -2), ss = slot(j, 0);
+                const int s = slot(j, -1), sn = slot(j, -2), ss = slot(j, 0);
                 {
                     real ku, kv, kn;
-                    rhs(xu[s], xv[s], xu[sn] + xu[ss], xv[sn] + xv[ss], xn[s], pp[s] * a.pamp[0], vv[s] * a.vamp_h[0], ku, kv, kn);
+                    if (POT) vv[s] *= a.vamp_h; /* V / hbar from here on */
+                    rhs(xu[s], xv[s], xu[sn] + xu[ss], xv[sn] + xv[ss], xn[s], pp[s], vv[s], ku, kv, kn);
                     y2u[s] = phx_fma(dth, ku, xu[s]);
                     y2v[s] = phx_fma(dth, kv, xv[s]);
                     if (RES) y2n[s] = phx_fma(dth, kn, xn[s]);
@@ -175,11 +191,11 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
             }
             /* ---- F2 at e = it-2: Y_3 = x + dt/2 f(Y_2) */
             {
-                const int e = it - 2, s = slot(j, -2), sn = slot(j, -3), ss = slot(j, -1);
+                const int s = slot(j, -2), sn = slot(j, -3), ss = slot(j, -1);
                 {
                     real ku, kv, kn;
-                    rhs(y2u[s], y2v[s], y2u[sn] + y2u[ss], y2v[sn] + y2v[ss], RES ? y2n[s] : real(0), pp[s] * a.pamp[1],
-                        vv[s] * a.vamp_h[1], ku, kv, kn);
+                    rhs(y2u[s], y2v[s], y2u[sn] + y2u[ss], y2v[sn] + y2v[ss], RES ? y2n[s] : real(0), pp[s],
+                        vv[s], ku, kv, kn);
                     y3u[s] = phx_fma(dth, ku, xu[s]);
                     y3v[s] = phx_fma(dth, kv, xv[s]);
                     if (RES) y3n[s] = phx_fma(dth, kn, xn[s]);
@@ -187,11 +203,11 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
             }
             /* ---- F3 + B4 at e = it-3: Y_4 = x + dt f(Y_3); c4 = dt/6 l', Yb4 = J(Y_4)^T c4, c3 */
             {
-                const int e = it - 3, s = slot(j, -3), sn = slot(j, -4), ss = slot(j, -2);
+                const int s = slot(j, -3), sn = slot(j, -4), ss = slot(j, -2);
                 {
                     real ku, kv, kn;
-                    rhs(y3u[s], y3v[s], y3u[sn] + y3u[ss], y3v[sn] + y3v[ss], RES ? y3n[s] : real(0), pp[s] * a.pamp[2],
-                        vv[s] * a.vamp_h[2], ku, kv, kn);
+                    rhs(y3u[s], y3v[s], y3u[sn] + y3u[ss], y3v[sn] + y3v[ss], RES ? y3n[s] : real(0), pp[s],
+                        vv[s], ku, kv, kn);
                     const real y4u = phx_fma(dt1, ku, xu[s]);
                     const real y4v = phx_fma(dt1, kv, xv[s]);
                     const real y4n = RES ? phx_fma(dt1, kn, xn[s]) : real(0);
@@ -199,7 +215,7 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
                     const real K4u = dt6 * nbr(lu[s], lu[sn] + lu[ss]);
                     const real K4v = dt6 * nbr(lv[s], lv[sn] + lv[ss]);
                     real bu, bv, bn;
-                    phx_rhs_scalar_vjp<real>(ph, y4u, y4v, y4n, POT ? vv[s] * a.vamp_h[3] : real(0), c4u, c4v, c4n, K4u, K4v, bu,
+                    phx_rhs_scalar_vjp<real>(ph, y4u, y4v, y4n, POT ? vv[s] : real(0), c4u, c4v, c4n, K4u, K4v, bu,
                                              bv, bn);
                     au[s] = bu;
                     av[s] = bv;
@@ -208,13 +224,13 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
                     c3u[s] = phx_fma(dt1, bu, d3u[s]);
                     c3v[s] = phx_fma(dt1, bv, d3v[s]);
                     real gp4, gv4, gp3, gv3;
-                    phx_rhs_scalar_param_vjp<real>(y4u, y4v, c4u, c4v, c4n, a.pamp[3], a.vamp_h[3], gp4, gv4);
+                    phx_rhs_scalar_param_vjp<real>(y4u, y4v, c4u, c4v, c4n, real(1), real(1), gp4, gv4);
                     if (RES) {
                         an[s] = bn;
                         d3n[s] = dt3 * ln[s];
                         c3n[s] = phx_fma(dt1, bn, d3n[s]);
                     }
-                    phx_rhs_scalar_param_vjp<real>(y3u[s], y3v[s], c3u[s], c3v[s], RES ? c3n[s] : real(0), a.pamp[2], a.vamp_h[2],
+                    phx_rhs_scalar_param_vjp<real>(y3u[s], y3v[s], c3u[s], c3v[s], RES ? c3n[s] : real(0), real(1), real(1),
                                                    gp3, gv3);
                     gpa[s] = gp4 + gp3;
                     gva[s] = gv4 + gv3;
@@ -222,12 +238,12 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
             }
             /* ---- B3 at e = it-4: Yb3 = J(Y_3)^T c3, c2 */
             {
-                const int e = it - 4, s = slot(j, -4), sn = slot(j, -5), ss = slot(j, -3);
+                const int s = slot(j, -4), sn = slot(j, -5), ss = slot(j, -3);
                 {
                     const real Ku = nbr(c3u[s], c3u[sn] + c3u[ss]);
                     const real Kv = nbr(c3v[s], c3v[sn] + c3v[ss]);
                     real bu, bv, bn;
-                    phx_rhs_scalar_vjp<real>(ph, y3u[s], y3v[s], RES ? y3n[s] : real(0), POT ? vv[s] * a.vamp_h[2] : real(0), c3u[s],
+                    phx_rhs_scalar_vjp<real>(ph, y3u[s], y3v[s], RES ? y3n[s] : real(0), POT ? vv[s] : real(0), c3u[s],
                                              c3v[s], RES ? c3n[s] : real(0), Ku, Kv, bu, bv, bn);
                     au[s] += bu;
                     av[s] += bv;
@@ -238,7 +254,7 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
                         c2n[s] = phx_fma(dth, bn, d3n[s]);
                     }
                     real gp2, gv2;
-                    phx_rhs_scalar_param_vjp<real>(y2u[s], y2v[s], c2u[s], c2v[s], RES ? c2n[s] : real(0), a.pamp[1], a.vamp_h[1],
+                    phx_rhs_scalar_param_vjp<real>(y2u[s], y2v[s], c2u[s], c2v[s], RES ? c2n[s] : real(0), real(1), real(1),
                                                    gp2, gv2);
                     gpa[s] += gp2;
                     gva[s] += gv2;
@@ -246,12 +262,12 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
             }
             /* ---- B2 at e = it-5: Yb2 = J(Y_2)^T c2, c1 */
             {
-                const int e = it - 5, s = slot(j, -5), sn = slot(j, -6), ss = slot(j, -4);
+                const int s = slot(j, -5), sn = slot(j, -6), ss = slot(j, -4);
                 {
                     const real Ku = nbr(c2u[s], c2u[sn] + c2u[ss]);
                     const real Kv = nbr(c2v[s], c2v[sn] + c2v[ss]);
                     real bu, bv, bn;
-                    phx_rhs_scalar_vjp<real>(ph, y2u[s], y2v[s], RES ? y2n[s] : real(0), POT ? vv[s] * a.vamp_h[1] : real(0), c2u[s],
+                    phx_rhs_scalar_vjp<real>(ph, y2u[s], y2v[s], RES ? y2n[s] : real(0), POT ? vv[s] : real(0), c2u[s],
                                              c2v[s], RES ? c2n[s] : real(0), Ku, Kv, bu, bv, bn);
                     au[s] += bu;
                     av[s] += bv;
@@ -262,7 +278,7 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
                         c1n[s] = phx_fma(dth, bn, dt6 * ln[s]);
                     }
                     real gp1, gv1;
-                    phx_rhs_scalar_param_vjp<real>(xu[s], xv[s], c1u[s], c1v[s], RES ? c1n[s] : real(0), a.pamp[0], a.vamp_h[0], gp1,
+                    phx_rhs_scalar_param_vjp<real>(xu[s], xv[s], c1u[s], c1v[s], RES ? c1n[s] : real(0), real(1), real(1), gp1,
                                                    gv1);
                     gpa[s] += gp1;
                     gva[s] += gv1;
@@ -271,25 +287,24 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
             /* ---- B1 at e = it-6: Yb1 = J(x)^T c1, l = l' + sum Yb; write row e */
             {
                 const int e = it - 6, s = slot(j, -6), sn = slot(j, -7), ss = slot(j, -5);
-                if (e >= 6 && e <= E - 7) {
-                    const real Ku = nbr(c1u[s], c1u[sn] + c1u[ss]);
-                    const real Kv = nbr(c1v[s], c1v[sn] + c1v[ss]);
-                    real bu, bv, bn;
-                    phx_rhs_scalar_vjp<real>(ph, xu[s], xv[s], RES ? xn[s] : real(0), POT ? vv[s] * a.vamp_h[0] : real(0), c1u[s],
-                                             c1v[s], RES ? c1n[s] : real(0), Ku, Kv, bu, bv, bn);
-                    const int grow = y0 + e - kAdjHalo;
-                    if (out_lane && grow < Nr) {
-                        const size_t idx = (size_t)grow * (size_t)Nc + (size_t)(x0 - kAdjHalo + lane);
-                        v2 o;
-                        o.x = lu[s] + (au[s] + bu);
-                        o.y = lv[s] + (av[s] + bv);
-                        a.lam_psi_out[so + idx] = o;
-                        if (RES) a.lam_n_out[so + idx] = ln[s] + (an[s] + bn);
-                        if (RES && a.g_pump) a.g_pump[so + idx] += gpa[s];
-                        if (a.g_pot) a.g_pot[so + idx] += gva[s];
-                    }
+                const real Ku = nbr(c1u[s], c1u[sn] + c1u[ss]);
+                const real Kv = nbr(c1v[s], c1v[sn] + c1v[ss]);
+                real bu, bv, bn;
+                phx_rhs_scalar_vjp<real>(ph, xu[s], xv[s], RES ? xn[s] : real(0), POT ? vv[s] : real(0), c1u[s], c1v[s],
+                                         RES ? c1n[s] : real(0), Ku, Kv, bu, bv, bn);
+                const uint32_t oc = out_row(e, so_c, row_c), orr = out_row(e, so_r, row_r);
+                v2 o;
+                o.x = lu[s] + (au[s] + bu);
+                o.y = lv[s] + (av[s] + bv);
+                store_cplx_s(d_o, oc, 0u, o);
+                if (RES) {
+                    store_real_s(d_on, orr, 0u, ln[s] + (an[s] + bn));
+                    store_real_s(d_gp, orr, 0u, gp_old + gpa[s]);
                 }
+                store_real_s(d_gv, orr, 0u, phx_fma(a.vamp_h, gva[s], gv_old));
             }
+            gp_old = gp_next;
+            gv_old = gv_next;
         }
     }
 }
@@ -368,7 +383,7 @@ struct phx_adjoint {
     const void* P = nullptr; /* parameters of the last forward call (caller-owned) */
     const void* V = nullptr;
     bool have_forward = false;
-    int ty_fwd = 12, ty_adj = 32;
+    int ty_fwd = 12, pf_fwd = 2, ty_adj = 32;
     bool tuned = false;
     hipStream_t own = nullptr, stream = nullptr;
 
@@ -429,7 +444,7 @@ int fwd_step(phx_adjoint* a, const void* psi_in, const void* n_in, void* psi_out
     }
     c.ph = adj_phys<real>(a);
     b.iso = c.ph.kin_yx == real(1);
-    ADJ_HIP(phx::launch_rk4_batched<real>(b, ty, a->res, a->pump, a->pot, st ? st : a->stream));
+    ADJ_HIP(phx::launch_rk4_batched<real>(b, ty, a->pf_fwd, a->res, a->pump, a->pot, st ? st : a->stream));
     return PHX_OK;
 }
 
@@ -475,10 +490,7 @@ int adj_step(phx_adjoint* a, void* state, int lin, int ty) {
     g.item_stride = a->N;
     g.param_stride = a->shared ? 0 : a->N;
     g.dt = (real)a->dt;
-    for (int k = 0; k < 4; k++) {
-        g.pamp[k] = 1;
-        g.vamp_h[k] = (real)a->ph.one_over_h_bar_s;
-    }
+    g.vamp_h = (real)a->ph.one_over_h_bar_s;
     g.ph = adj_phys<real>(a);
     ADJ_HIP(phx::launch_rk4_adjoint<real>(g, a->res, a->pump, a->pot, a->stream));
     return PHX_OK;
@@ -507,30 +519,38 @@ int autotune(phx_adjoint* a) {
         ADJ_HIP(hipEventElapsedTime(&ms, e0, e1));
         return PHX_OK;
     };
-    const int fwd_tys[] = {8, 10, 12, 16, 20};
+    const int fwd_tys[] = {8, 10, 12, 16, 20, 4};
+    const int fwd_pfs[] = {2, 4, 6};
     const int adj_tys[] = {16, 20, 24, 28, 32, 40, 48, 56, 64, 80};
-    float fwd_ms[5], adj_ms[10];
+    float fwd_ms[6], pf_ms[3], adj_ms[10];
     for (float& m : fwd_ms) m = 1e30f;
+    for (float& m : pf_ms) m = 1e30f;
     for (float& m : adj_ms) m = 1e30f;
     int rc = PHX_OK;
+    auto time_fwd = [&](int ty, int pf, float& best) {
+        float ms = 0;
+        a->pf_fwd = pf;
+        rc = timeit([&] { return fwd_step<real>(a, a->state_psi(a->ckpt_at(0)), a->state_n(a->ckpt_at(0)), a->state_psi(a->lam[1]),
+                                                a->state_n(a->lam[1]), ty); },
+                    ms);
+        if (!rc) best = std::min(best, ms);
+    };
     for (int pass = 0; pass < 3 && !rc; pass++) {
-        for (int i = 0; i < 5 && !rc; i++) {
-            float ms = 0;
-            rc = timeit([&] { return fwd_step<real>(a, a->state_psi(a->ckpt_at(0)), a->state_n(a->ckpt_at(0)), a->state_psi(a->lam[1]),
-                                                    a->state_n(a->lam[1]), fwd_tys[i]); },
-                        ms);
-            if (!rc) fwd_ms[i] = std::min(fwd_ms[i], ms);
-        }
+        for (int i = 0; i < 6 && !rc; i++) time_fwd(fwd_tys[i], 4, fwd_ms[i]);
         for (int i = 0; i < 10 && !rc; i++) {
             float ms = 0;
             rc = timeit([&] { return adj_step<real>(a, a->ckpt_at(0), 0, adj_tys[i]); }, ms);
             if (!rc) adj_ms[i] = std::min(adj_ms[i], ms);
         }
     }
+    const int ty_fwd = fwd_tys[std::min_element(fwd_ms, fwd_ms + 6) - fwd_ms];
+    for (int pass = 0; pass < 2; pass++) /* the forward kernel's prefetch depth at its best height */
+        for (int i = 0; i < 3 && !rc; i++) time_fwd(ty_fwd, fwd_pfs[i], pf_ms[i]);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    a->ty_fwd = fwd_tys[std::min_element(fwd_ms, fwd_ms + 5) - fwd_ms];
+    a->ty_fwd = ty_fwd;
+    a->pf_fwd = fwd_pfs[std::min_element(pf_ms, pf_ms + 3) - pf_ms];
     a->ty_adj = adj_tys[std::min_element(adj_ms, adj_ms + 10) - adj_ms];
     a->tuned = true;
     return PHX_OK;

@@ -34,6 +34,28 @@ __device__ __forceinline__ int xcd_contiguous(int b, int nblocks) {
     return start + (b >> 3);
 }
 
+/* Tile (strip, band) of a wave.  A block holds four vertically stacked bands of one strip, blocks go along
+   the strips; the bands left over below the last whole group of four are handed out four tiles to a block as
+   well, so that no wave is idle: a kernel that holds one wave a SIMD pays for every block in whole rounds
+   over the CUs (2048 x 2048 in 28-row tiles: 779 blocks with an idle wave in some, 759 without; a round of
+   256 CUs apart).  False: no tile. */
+__host__ __device__ inline int tile_blocks(int nstrips, int nbands) {
+    return (nbands / kWavesPerBlock) * nstrips + ((nbands % kWavesPerBlock) * nstrips + kWavesPerBlock - 1) / kWavesPerBlock;
+}
+__device__ __forceinline__ bool tile_of(int block, int wave, int nstrips, int nbands, int& strip, int& band) {
+    const int groups = nbands / kWavesPerBlock, rem = nbands % kWavesPerBlock, full = groups * nstrips;
+    if (block < full) {
+        strip = block % nstrips;
+        band = (block / nstrips) * kWavesPerBlock + wave;
+        return true;
+    }
+    const int t = (block - full) * kWavesPerBlock + wave;
+    if (t >= rem * nstrips) return false;
+    strip = t / rem;
+    band = groups * kWavesPerBlock + t % rem;
+    return true;
+}
+
 /* Periodic row wrap without branches, so that a fully unrolled row loop stays one
    basic block (a branch there splits it, and DPP moves then no longer fold into the
    adds that consume them).  x mod Nr for x = g + bias >= 0 is x - Nr * q with

@@ -48,8 +48,8 @@ struct phx_ensemble {
     /* per instance: offsets (bytes) of psi[2], n[2], pump, pot in the pool */
     std::vector<size_t> off_psi[2], off_n[2], off_pump, off_pot;
     int cur = 0;
-    int ty = 12;
-    bool ty_auto = true; /* tile height picked by timing at the first step */
+    int ty = 12, pf = 2; /* tile height, rows loaded ahead */
+    bool ty_auto = true; /* picked by timing at the first step */
     /* device tables for the two buffer parities and the tile list */
     void* entries[2] = {nullptr, nullptr};
     int* tile_inst = nullptr;
@@ -154,39 +154,47 @@ int launch_step(phx_ensemble* e, double dt, int parity) {
         b.common.vamp_h[k] = (real)e->ph.one_over_h_bar_s;
     }
     b.common.ph = phys_of<real>(e, 0);
-    ENS_HIP(phx::launch_rk4_batched<real>(b, e->ty, e->res, e->pump, e->pot, e->stream));
+    ENS_HIP(phx::launch_rk4_batched<real>(b, e->tables_ty, e->pf, e->res, e->pump, e->pot, e->stream));
     return PHX_OK;
 }
 
-/* Pick the tile height with the shortest step for this ensemble: every candidate
-   launch reads the current buffers and writes the other ones, so the state
-   does not advance.  Three round-robin passes, each candidate's fastest counting
-   (a single pass in a fixed order times the first candidates while the clocks ramp). */
+/* Pick the tile height and prefetch depth with the shortest step for this ensemble: every candidate
+   launch reads the current buffers and writes the other ones, so the state does not advance.  Some
+   launches first, so that the clocks have ramped up; then the heights at a middle depth, and the
+   depths at the best height (each candidate's fastest of two rounds). */
 template <typename real>
 int autotune(phx_ensemble* e, double dt) {
     hipEvent_t e0, e1;
     ENS_HIP(hipEventCreate(&e0));
     ENS_HIP(hipEventCreate(&e1));
-    const int tys[] = {8, 10, 12, 16, 20};
-    float ms_best[5] = {1e30f, 1e30f, 1e30f, 1e30f, 1e30f};
+    const int tys[] = {8, 10, 12, 16, 20, 4};
+    const int pfs[] = {2, 4, 6};
     int rc = PHX_OK;
-    for (int pass = 0; pass < 3 && !rc; pass++) {
-        for (int i = 0; i < 5 && !rc; i++) {
-            rc = build_tables<real>(e, tys[i]);
-            for (int w = 0; w < 2 && !rc; w++) rc = launch_step<real>(e, dt, e->cur);
-            if (!rc && hipEventRecord(e0, e->stream) != hipSuccess) rc = efail(PHX_ERR_HIP, "hipEventRecord");
-            for (int r = 0; r < 5 && !rc; r++) rc = launch_step<real>(e, dt, e->cur);
-            if (!rc && hipEventRecord(e1, e->stream) != hipSuccess) rc = efail(PHX_ERR_HIP, "hipEventRecord");
-            float ms = 0;
-            if (!rc && (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
-                rc = efail(PHX_ERR_HIP, "event timing");
-            if (!rc) ms_best[i] = std::min(ms_best[i], ms);
-        }
-    }
+    auto timed = [&](int ty, int pf, float& best) {
+        if (!rc && e->tables_ty != ty) rc = build_tables<real>(e, ty);
+        e->pf = pf;
+        if (!rc) rc = launch_step<real>(e, dt, e->cur);
+        if (!rc && hipEventRecord(e0, e->stream) != hipSuccess) rc = efail(PHX_ERR_HIP, "hipEventRecord");
+        for (int r = 0; r < 4 && !rc; r++) rc = launch_step<real>(e, dt, e->cur);
+        if (!rc && hipEventRecord(e1, e->stream) != hipSuccess) rc = efail(PHX_ERR_HIP, "hipEventRecord");
+        float ms = 0;
+        if (!rc && (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+            rc = efail(PHX_ERR_HIP, "event timing");
+        if (!rc) best = std::min(best, ms);
+    };
+    float ms[6] = {1e30f, 1e30f, 1e30f, 1e30f, 1e30f, 1e30f}, warm = 1e30f;
+    for (int i = 0; i < 4 && !rc; i++) timed(tys[2], pfs[1], warm);
+    for (int round = 0; round < 2 && !rc; round++)
+        for (int i = 0; i < 6 && !rc; i++) timed(tys[i], pfs[1], ms[i]);
+    const int ty = tys[std::min_element(ms, ms + 6) - ms];
+    float mp[3] = {1e30f, 1e30f, 1e30f};
+    for (int round = 0; round < 2 && !rc; round++)
+        for (int i = 0; i < 3 && !rc; i++) timed(ty, pfs[i], mp[i]);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    e->ty = tys[std::min_element(ms_best, ms_best + 5) - ms_best];
+    e->ty = ty;
+    e->pf = pfs[std::min_element(mp, mp + 3) - mp];
     e->ty_auto = false;
     return PHX_OK;
 }

@@ -109,9 +109,10 @@ struct Rk4BatchArgs {
     int iso; /* every instance has dx == dy (kin_yx == 1): stencil without the y/x ratio */
 };
 
-/* All instances share the feature set (reservoir / pump / potential) and dt. */
+/* All instances share the feature set (reservoir / pump / potential) and dt.  ty: output rows per tile
+   (4, 8, 10, 12, 16, 20), pf: rows loaded ahead (2, or 4 and 6 for the pumped reservoir model with dx == dy) */
 template <typename real>
-hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, bool res, bool pump, bool pot, hipStream_t s);
+hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, int pf, bool res, bool pump, bool pot, hipStream_t s);
 
 /* wavefront tiles of one grid for the fused RK4 kernel with tile height ty */
 __host__ __device__ inline int rk4_tiles(int Nc, int Nr, int ty) { return ((Nc + 55) / 56) * ((Nr + ty - 1) / ty); }
@@ -139,7 +140,7 @@ struct Rk4AdjArgs {
     int ty, nstrips, tiles_per_item, ntiles; /* ty: output rows per wavefront tile */
     size_t item_stride, param_stride;       /* elements; param_stride 0: P, V shared */
     real dt;
-    real pamp[4], vamp_h[4];
+    real vamp_h; /* 1 / hbar: P and V are constant over a step */
     PhxPhys<real> ph;
 };
 
@@ -216,9 +217,12 @@ hipError_t launch_rk4_generic(const RkGenArgs<real>& a, hipStream_t s);
 int rk4_generic_tile_rows(int Nc, int Nr);
 /* adaptive DP45, TE-TM, FP32, tile height 32 (phx_rk_dp45t.hip) */
 hipError_t launch_dp45_tetm_tall(const RkGenArgs<float>& a, int ty, hipStream_t s);
+/* ... the others and the shorter tiles (phx_rk_dp45.hip) */
+template <typename real>
+hipError_t launch_dp45_adaptive(const RkGenArgs<real>& a, int ty, hipStream_t s);
 /* tile height of the adaptive DP45 kernel for a grid: the height among the compiled ones that
-   minimises (wavefront tiles per SIMD, rounded up) x (row evaluations per tile), a VALU-bound
-   model; PHX_GEN_TY fixes it (16 or 32) */
+   minimises (blocks of tiles per CU, rounded up) x (row evaluations per tile), a VALU-bound
+   model; PHX_GEN_TY fixes it (8, 16, 28, 32 or 42) */
 int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr);
 
 /* Staged Runge-Kutta step (phx_staged.hip): one launch per CALCULATE_K, INTERMEDIATE_SUM_K
@@ -275,7 +279,8 @@ struct StagedArgs {
 };
 template <typename real>
 hipError_t launch_staged(const StagedArgs<real>& a, StagedOp op, hipStream_t s);
-/* deterministic reduction of (error, norm) pairs into sums[0..1] (one workgroup, fixed order) */
+/* deterministic reduction of (error, norm) pairs into sums[0..1] (one workgroup, fixed order); sums may be
+   pinned host memory */
 hipError_t launch_reduce_partials(const double* partials, int nwaves, double* sums, hipStream_t s);
 /* blocks of the FINAL launch (partials buffer size = 2 * this) */
 inline size_t staged_final_blocks(int Nc, int Nr) { return (size_t)((Nc + 63) / 64) * (size_t)((Nr + 3) / 4); }
@@ -297,8 +302,8 @@ hipError_t launch_noise_field(typename Vec2<real>::type* xi, int Nc, int Nr, uin
                               hipStream_t s);
 
 /* wavefront tiles of the generic kernel for a grid at tile height ty; the partials buffer of an
-   adaptive tableau holds 2 doubles per tile at the smallest height the launcher uses (16) */
-constexpr int kRkGenMinTileRows = 16;
+   adaptive tableau holds 2 doubles per tile at the smallest height the launchers use (8) */
+constexpr int kRkGenTileRows = 16, kRkGenMinTileRows = 8;
 inline int rk_generic_waves(RkTableau tab, int Nc, int Nr, int ty = kRkGenMinTileRows) {
     const int S = rk_tableau_stages(tab);
     const int outw = 64 - 2 * S;

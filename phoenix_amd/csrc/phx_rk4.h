@@ -209,10 +209,8 @@ __device__ __forceinline__ void rk4_tile(const Rk4Args<real>& a, int strip, int 
 template <typename real, int TY, bool ISO, int PF, bool RES, bool PUMP, bool POT, bool PERY>
 __global__ __launch_bounds__(256) void rk4_scalar_fused(Rk4Args<real> a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int tile = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int strip = tile % a.nstrips;
-    const int band = (tile / a.nstrips) * kWavesPerBlock + wave;
-    if (band >= a.nbands) return;
+    int strip, band;
+    if (!tile_of(xcd_contiguous(blockIdx.x, gridDim.x), wave, a.nstrips, a.nbands, strip, band)) return;
     rk4_tile<real, TY, ISO, PF, RES, PUMP, POT, PERY>(a, strip, band);
 }
 
@@ -245,10 +243,9 @@ template <typename real, int TY, bool ISO, int PF, bool RES, bool PUMP, bool POT
 __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow f) {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int tile = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int strip = tile % a.nstrips;
-    const int band = (tile / a.nstrips) * kWavesPerBlock + wave;
-    if (band >= a.nbands) return; /* no tile: nobody watches this wave's counter */
+    int strip, band;
+    if (!tile_of(xcd_contiguous(blockIdx.x, gridDim.x), wave, a.nstrips, a.nbands, strip, band))
+        return; /* no tile: nobody watches this wave's counter */
     const int me = band * a.nstrips + strip;
     /* lanes 0..24 watch the tiles up to two strips and two bands away that the halo reaches: the next one
        on each side, and the one behind it where the next is a last strip or band of fewer than kHalo cells */
@@ -340,8 +337,7 @@ inline hipError_t launch_ty(const Rk4Args<real>& a0, hipStream_t s) {
     Rk4Args<real> a = a0;
     a.nstrips = (a.Nc + kOutW - 1) / kOutW;
     a.nbands = (a.Nr + TY - 1) / TY;
-    const int bandgroups = (a.nbands + kWavesPerBlock - 1) / kWavesPerBlock;
-    const int nblocks = a.nstrips * bandgroups;
+    const int nblocks = tile_blocks(a.nstrips, a.nbands);
     /* periodic rows: a separate kernel, whose row descriptors are loop invariant (fewer
        scalar registers than the zero-boundary form, which selects an empty descriptor for
        rows outside the grid) */
@@ -404,7 +400,7 @@ inline hipError_t launch_flow_ty(const Rk4Args<real>& a0, const Rk4Flow& f, hipS
     Rk4Args<real> a = a0;
     a.nstrips = (a.Nc + kOutW - 1) / kOutW;
     a.nbands = (a.Nr + TY - 1) / TY;
-    const int nblocks = a.nstrips * ((a.nbands + kWavesPerBlock - 1) / kWavesPerBlock);
+    const int nblocks = tile_blocks(a.nstrips, a.nbands);
     const void* fn = a.periodic_y ? (const void*)&rk4_scalar_flow<real, TY, ISO, PF, RES, PUMP, POT, true, CAMP>
                                   : (const void*)&rk4_scalar_flow<real, TY, ISO, PF, RES, PUMP, POT, false, CAMP>;
     /* every wave must be resident at once: the cooperative launch refuses a grid that is not */
@@ -466,44 +462,47 @@ hipError_t launch_rk4_flow(const Rk4Args<real>& a, const Rk4Tune& t, const Rk4Fl
 }
 
 /* ---------------------------------------------------------------- ensembles */
-template <typename real, int TY, bool ISO, bool RES, bool PUMP, bool POT>
+template <typename real, int TY, bool ISO, int PF, bool RES, bool PUMP, bool POT>
 inline hipError_t launch_batch_ty(const Rk4BatchArgs<real>& b, hipStream_t s) {
     const int nblocks = (b.ntiles + kWavesPerBlock - 1) / kWavesPerBlock;
     if (b.common.periodic_y)
-        hipLaunchKernelGGL((rk4_batched_fused<real, TY, ISO, 2, RES, PUMP, POT, true>), dim3(nblocks),
+        hipLaunchKernelGGL((rk4_batched_fused<real, TY, ISO, PF, RES, PUMP, POT, true>), dim3(nblocks),
                            dim3(kWave * kWavesPerBlock), 0, s, b);
     else
-        hipLaunchKernelGGL((rk4_batched_fused<real, TY, ISO, 2, RES, PUMP, POT, false>), dim3(nblocks),
+        hipLaunchKernelGGL((rk4_batched_fused<real, TY, ISO, PF, RES, PUMP, POT, false>), dim3(nblocks),
                            dim3(kWave * kWavesPerBlock), 0, s, b);
     return hipGetLastError();
 }
 
-template <typename real, bool ISO, bool RES, bool PUMP, bool POT>
+template <typename real, bool ISO, int PF, bool RES, bool PUMP, bool POT>
 inline hipError_t launch_batch_tys(const Rk4BatchArgs<real>& b, int ty, hipStream_t s) {
     switch (ty) {
-        case 4: return launch_batch_ty<real, 4, ISO, RES, PUMP, POT>(b, s);
-        case 8: return launch_batch_ty<real, 8, ISO, RES, PUMP, POT>(b, s);
-        case 10: return launch_batch_ty<real, 10, ISO, RES, PUMP, POT>(b, s);
-        case 16: return launch_batch_ty<real, 16, ISO, RES, PUMP, POT>(b, s);
-        case 20: return launch_batch_ty<real, 20, ISO, RES, PUMP, POT>(b, s);
-        default: return launch_batch_ty<real, 12, ISO, RES, PUMP, POT>(b, s);
+        case 4: return launch_batch_ty<real, 4, ISO, PF, RES, PUMP, POT>(b, s);
+        case 8: return launch_batch_ty<real, 8, ISO, PF, RES, PUMP, POT>(b, s);
+        case 10: return launch_batch_ty<real, 10, ISO, PF, RES, PUMP, POT>(b, s);
+        case 16: return launch_batch_ty<real, 16, ISO, PF, RES, PUMP, POT>(b, s);
+        case 20: return launch_batch_ty<real, 20, ISO, PF, RES, PUMP, POT>(b, s);
+        default: return launch_batch_ty<real, 12, ISO, PF, RES, PUMP, POT>(b, s);
     }
 }
 
 template <typename real, bool RES, bool PUMP, bool POT>
-inline hipError_t launch_batch_flags(const Rk4BatchArgs<real>& b, int ty, hipStream_t s) {
-    return b.iso ? launch_batch_tys<real, true, RES, PUMP, POT>(b, ty, s) : launch_batch_tys<real, false, RES, PUMP, POT>(b, ty, s);
+inline hipError_t launch_batch_flags(const Rk4BatchArgs<real>& b, int ty, int pf, hipStream_t s) {
+    if constexpr (RES && PUMP) {
+        if (b.iso && pf == 4) return launch_batch_tys<real, true, 4, RES, PUMP, POT>(b, ty, s);
+        if (b.iso && pf == 6) return launch_batch_tys<real, true, 6, RES, PUMP, POT>(b, ty, s);
+    }
+    return b.iso ? launch_batch_tys<real, true, 2, RES, PUMP, POT>(b, ty, s) : launch_batch_tys<real, false, 2, RES, PUMP, POT>(b, ty, s);
 }
 
 template <typename real>
-hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, bool res, bool pump, bool pot, hipStream_t s) {
+hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, int pf, bool res, bool pump, bool pot, hipStream_t s) {
     /* (instance sizes are checked when the ensemble is created) */
     if (!b.entries && (size_t)b.common.Nc * (size_t)b.common.Nr * sizeof(typename Vec2<real>::type) > kMaxArrayBytes)
         return hipErrorInvalidValue;
-    if (!res) return pot ? launch_batch_flags<real, false, false, true>(b, ty, s) : launch_batch_flags<real, false, false, false>(b, ty, s);
-    if (pump) return pot ? launch_batch_flags<real, true, true, true>(b, ty, s) : launch_batch_flags<real, true, true, false>(b, ty, s);
-    return pot ? launch_batch_flags<real, true, false, true>(b, ty, s) : launch_batch_flags<real, true, false, false>(b, ty, s);
+    if (!res) return pot ? launch_batch_flags<real, false, false, true>(b, ty, pf, s) : launch_batch_flags<real, false, false, false>(b, ty, pf, s);
+    if (pump) return pot ? launch_batch_flags<real, true, true, true>(b, ty, pf, s) : launch_batch_flags<real, true, true, false>(b, ty, pf, s);
+    return pot ? launch_batch_flags<real, true, false, true>(b, ty, pf, s) : launch_batch_flags<real, true, false, false>(b, ty, pf, s);
 }
-
 
 } // namespace phx

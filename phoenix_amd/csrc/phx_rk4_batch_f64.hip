@@ -1,0 +1,11 @@
+/*
+ * phx_rk4_batch_f64.hip -- FP64 instantiations of the batched RK4 kernel of phx_rk4.h (in translation units of
+ * their own, so that they compile in parallel).
+ */
+#include "phx_rk4.h"
+
+namespace phx {
+
+template hipError_t launch_rk4_batched<double>(const Rk4BatchArgs<double>&, int, int, bool, bool, bool, hipStream_t);
+
+} // namespace phx

@@ -30,7 +30,7 @@ static hipError_t launch_chain_ng(const RkGenArgs<real>& a0, const RkChainArgs<r
     constexpr int outw = kWave - 2 * TabRK4::S;
     a.nstrips = (a.Nc + outw - 1) / outw;
     a.nbands = (a.Nr + TY - 1) / TY;
-    const dim3 grid(a.nstrips * ((a.nbands + kWavesPerBlock - 1) / kWavesPerBlock)), blk(kWave * kWavesPerBlock);
+    const dim3 grid(tile_blocks(a.nstrips, a.nbands)), blk(kWave * kWavesPerBlock);
     if (std::max(std::max(ch.npump, ch.npot), ch.npulse) <= 1)
         hipLaunchKernelGGL((rk_chain_fused<real, TY, TETM, RES, STOCH, 1>), grid, blk, 0, s, a, ch);
     else

@@ -41,7 +41,8 @@ __device__ __forceinline__ double rk_wave_sum(double v) {
     return v;
 }
 
-/* deterministic reduction of the per-wave partials (one workgroup, fixed order) into sums[0..1] */
+/* deterministic reduction of the per-wave partials (one workgroup, fixed order) into sums[0..1], which may be
+   pinned host memory */
 hipError_t launch_reduce_partials(const double* partials, int nwaves, double* sums, hipStream_t s);
 
 /* ---------------------------------------------------------------- kernel */
@@ -64,9 +65,8 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int tile = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int strip = tile % a.nstrips;
-    const int band = (tile / a.nstrips) * kWavesPerBlock + wave;
-    if (band >= a.nbands) return;
+    int strip, band;
+    if (!tile_of(tile, wave, a.nstrips, a.nbands, strip, band)) return;
     const int outw = kWave - 2 * H;
     const int x0 = strip * outw;
     const int y0 = band * TY;
@@ -119,7 +119,7 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
     real fr[NC][G][E], fi[NC][G][E]; /* pulse fields (NG > 0) */
     real Kr[NC][S][E], Ki[NC][S][E], Kn[NC][S][E];
     real Yr[NC][S][E], Yi[NC][S][E], Yn[NC][S][E]; /* Y[s] = input of stage s+1, s = 0..S-2 */
-    real xr[E], xi[E], sg[E];                      /* noise xi and its amplitude sqrt((R n0 + gc)/(4 dV)) */
+    real xr[E], xi[E]; /* noise xi of a row; from stage 1 on xi sqrt((R n0 + gc)/(4 dV)) */
     double err_acc = 0.0, nrm_acc = 0.0;
 
     auto load_row = [&](int r) {
@@ -150,8 +150,6 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
             const v2 z = load_cplx_s<real>(d_xi, vc, 0u);
             xr[r] = z.x;
             xi[r] = z.y;
-            const real nplus = RES ? n0[0][r] : real(0);
-            sg[r] = phx_sqrt((RES ? phx_fma(ph.R, nplus, ph.gamma_c) : ph.gamma_c) / (real(4) * ph.dV));
         }
     };
 
@@ -228,13 +226,19 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
                 /* stochastic corrections of the RHS (kernel_gp_compute.cuh:83-85,106-108):
                    k_psi -= g_c/hbar (-i psi)/dV ; k_n += R n / dV */
                 const real g = ph.gc_h / ph.dV;
-                kr -= g * ci_[k];
-                ki += g * cr_[k];
+                kr = phx_fma(-g, ci_[k], kr);
+                ki = phx_fma(g, cr_[k], ki);
                 if (RES) kn = phx_fma(ph.R / ph.dV, nv, kn);
             }
             Kr[k][s][e] = kr;
             Ki[k][s][e] = ki;
             Kn[k][s][e] = kn;
+        }
+        if (STOCH && s == 0) {
+            /* the row's noise increment, once it is first used (two rows after its loads were issued) */
+            const real sg = phx_sqrt((RES ? phx_fma(ph.R, n0[0][e], ph.gamma_c) : ph.gamma_c) / (real(4) * ph.dV));
+            xr[e] *= sg;
+            xi[e] *= sg;
         }
         /* input of the next stage: Y_s = psi0 + dt sum_{j<=s} a[s+1][j] K_j (+ noise) */
         if (s + 1 < S) {
@@ -263,8 +267,8 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
                 real yr = phx_fma(dtr, sr, phx_fma(-dti, si, p0r[k][e]));
                 real yi = phx_fma(dtr, si, phx_fma(dti, sr, p0i[k][e]));
                 if (STOCH) {
-                    yr = phx_fma(wsum * xr[e], sg[e], yr);
-                    yi = phx_fma(wsum * xi[e], sg[e], yi);
+                    yr = phx_fma(wsum, xr[e], yr);
+                    yi = phx_fma(wsum, xi[e], yi);
                 }
                 Yr[k][s][e] = yr;
                 Yi[k][s][e] = yi;
@@ -301,8 +305,8 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
             real o_r = phx_fma(dtr, sr, phx_fma(-dti, si, p0r[k][e]));
             real o_i = phx_fma(dtr, si, phx_fma(dti, sr, p0i[k][e]));
             if (STOCH) {
-                o_r = phx_fma(bsum * xr[e], sg[e], o_r);
-                o_i = phx_fma(bsum * xi[e], sg[e], o_i);
+                o_r = phx_fma(bsum, xr[e], o_r);
+                o_i = phx_fma(bsum, xi[e], o_i);
             }
             if (k == 0) {
                 out0r = o_r;
@@ -373,8 +377,7 @@ static hipError_t launch_gen(const RkGenArgs<real>& a0, hipStream_t s) {
     const int outw = kWave - 2 * TAB::S;
     a.nstrips = (a.Nc + outw - 1) / outw;
     a.nbands = (a.Nr + TY - 1) / TY;
-    const int bandgroups = (a.nbands + kWavesPerBlock - 1) / kWavesPerBlock;
-    hipLaunchKernelGGL((rk_generic_fused<real, TAB, TY, TETM, RES, STOCH, POT>), dim3(a.nstrips * bandgroups),
+    hipLaunchKernelGGL((rk_generic_fused<real, TAB, TY, TETM, RES, STOCH, POT>), dim3(tile_blocks(a.nstrips, a.nbands)),
                        dim3(kWave * kWavesPerBlock), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !TAB::ERR) return e;
@@ -402,7 +405,7 @@ static hipError_t dispatch_flags(const RkGenArgs<real>& a, hipStream_t s) {
 /* the kernel for one tableau, every feature set, tile height 16 */
 template <typename real, typename TAB>
 hipError_t launch_tab(const RkGenArgs<real>& a, hipStream_t s) {
-    return dispatch_flags<real, TAB, 16>(a, s);
+    return dispatch_flags<real, TAB, kRkGenTileRows>(a, s);
 }
 
 } // namespace phx

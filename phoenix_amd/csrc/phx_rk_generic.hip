@@ -14,17 +14,18 @@
 namespace phx {
 
 /* deterministic reduction of the per-wave partials: one workgroup, fixed order */
-__global__ __launch_bounds__(256) void reduce_partials(const double* __restrict__ partials, int nwaves, double* __restrict__ out) {
-    __shared__ double se[256], sn[256];
+constexpr int kReduceThreads = 1024;
+__global__ __launch_bounds__(kReduceThreads) void reduce_partials(const double* __restrict__ partials, int nwaves, double* __restrict__ out) {
+    __shared__ double se[kReduceThreads], sn[kReduceThreads];
     double e = 0, n = 0;
-    for (int i = threadIdx.x; i < nwaves; i += 256) {
+    for (int i = threadIdx.x; i < nwaves; i += kReduceThreads) {
         e += partials[2 * i];
         n += partials[2 * i + 1];
     }
     se[threadIdx.x] = e;
     sn[threadIdx.x] = n;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
+    for (int w = kReduceThreads / 2; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) {
             se[threadIdx.x] += se[threadIdx.x + w];
             sn[threadIdx.x] += sn[threadIdx.x + w];
@@ -38,7 +39,7 @@ __global__ __launch_bounds__(256) void reduce_partials(const double* __restrict_
 }
 
 hipError_t launch_reduce_partials(const double* partials, int nwaves, double* sums, hipStream_t s) {
-    hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(256), 0, s, partials, nwaves, sums);
+    hipLaunchKernelGGL(reduce_partials, dim3(1), dim3(kReduceThreads), 0, s, partials, nwaves, sums);
     return hipGetLastError();
 }
 
@@ -186,24 +187,24 @@ int rk4_generic_tile_rows(int Nc, int Nr) {
 }
 
 int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr) {
-    if (!(tetm && fp32)) return kRkGenMinTileRows; /* the tall tiles exist for the FP32 spinor kernel */
+    const bool tall = tetm && fp32; /* the tall tiles exist for the FP32 spinor kernel */
     const char* e = std::getenv("PHX_GEN_TY"); /* read at every launch: tests switch it within a process */
     const int env_ty = e ? std::atoi(e) : 0;
-    if (env_ty == 16 || env_ty == 32) return env_ty;
-    const int simds = rk4_simds();
+    if (env_ty == 8 || env_ty == 16 || (tall && (env_ty == 28 || env_ty == 32 || env_ty == 42))) return env_ty;
     /* One wave per SIMD at the kernel's register count (over 256 VGPRs + AGPRs at every height),
-       and about the same VALU work per row evaluation at every height (145-148 instructions): a
-       SIMD's time is its number of tiles (rounded up) times the row evaluations of one tile,
-       S (TY + 2 S) - S (S + 1) for S = 7.  At 2048^2 this predicts 32 rows 1.16x faster than 16
-       (1.21x measured).  Other heights that the model ranks near or above 32 measured slower and
-       are not built: 42 rows (2009 tiles, 2 rounds) 1.24x slower, 28 rows (3034 tiles, 3 full
-       rounds of 238 row evaluations against 3 x 266) 1.19x slower. */
+       and about the same VALU work per row evaluation at every height (135-148 instructions): a
+       grid's time is its blocks in rounds over the CUs (rounded up) times the row evaluations of one
+       tile, S (TY + 2 S) - S (S + 1) for S = 7.  us per attempt, FP32 TE-TM, 8 / 16 / 28 / 32 / 42 rows
+       (the rule's choice in brackets): 2048^2 with noise 365 / 318 / 242 / 266 / [229], without 303 / 265 /
+       202 / 221 / [190]; 1536 x 1200 148 / 141 / 137 / 150 / [103]; 1024^2 95 / 99 / [78] / 85 / 101; 600^2
+       [43] / 56 / 72 / 79 / 95; FP64 1024^2 488 / [482], 300^2 [126] / 171. */
     constexpr int S = 7;
-    int best = kRkGenMinTileRows;
+    int best = kRkGenTileRows;
     long best_cost = -1;
-    for (int ty : {16, 32}) {
-        const long waves = (long)((Nc + 63 - 2 * S) / (64 - 2 * S)) * ((Nr + ty - 1) / ty);
-        const long cost = ((waves + simds - 1) / simds) * (long)(S * (ty + 2 * S) - S * (S + 1));
+    for (int ty : {16, 8, 28, 32, 42}) {
+        if (ty > kRkGenTileRows && !tall) continue;
+        const long blocks = tile_blocks((Nc + 63 - 2 * S) / (64 - 2 * S), (Nr + ty - 1) / ty), cus = rk4_simds() / 4;
+        const long cost = ((blocks + cus - 1) / cus) * (long)(S * (ty + 2 * S) - S * (S + 1));
         if (best_cost < 0 || cost < best_cost) best = ty, best_cost = cost;
     }
     return best;
@@ -217,8 +218,8 @@ hipError_t launch_rk_generic(const RkGenArgs<real>& a, RkTableau tab, hipStream_
         case RkTableau::DP45_ADAPTIVE: {
             const int ty = dp45_adaptive_tile_rows(a.tetm, sizeof(real) == 4, a.Nc, a.Nr);
             if constexpr (sizeof(real) == 4)
-                if (ty != kRkGenMinTileRows && a.tetm) return launch_dp45_tetm_tall(a, ty, s);
-            return launch_tab<real, TabDP45Adaptive>(a, s);
+                if (ty > kRkGenTileRows && a.tetm) return launch_dp45_tetm_tall(a, ty, s);
+            return launch_dp45_adaptive<real>(a, ty, s);
         }
         case RkTableau::NEWTON:
         case RkTableau::MP:

@@ -78,8 +78,8 @@ struct phx_solver {
     double* norm_partials = nullptr; /* imaginary-time normalisation: per-block sums, reduced sums */
     double* norm_sums = nullptr;
     double* partials = nullptr; /* per-wavefront (error, norm) of the adaptive kernel */
-    double* sums = nullptr;     /* reduced (error, norm), device */
-    double* sums_host = nullptr; /* pinned host copy */
+    double* sums_host = nullptr; /* reduced (error, norm), in pinned host memory that the reduction writes */
+    double* sums = nullptr;      /* ... its device address */
     const phx::IteratorInfo* iter = nullptr; /* registry entry of cfg.iterator (nullptr for SSFM) */
     bool ssfm = false;                        /* split-step Fourier iterator */
     /* linear factors along rows (N_r) and columns (N_c): of a half step, and of the two half steps that meet
@@ -140,6 +140,12 @@ int dev_alloc(phx_solver* s, void** p, size_t bytes) {
     PHX_HIP(hipMalloc(p, bytes));
     PHX_HIP(hipMemsetAsync(*p, 0, bytes, s->stream));
     s->allocs.push_back(*p);
+    return PHX_OK;
+}
+
+int sums_alloc(phx_solver* s) {
+    PHX_HIP(hipHostMalloc((void**)&s->sums_host, 2 * sizeof(double), hipHostMallocDefault));
+    PHX_HIP(hipHostGetDevicePointer((void**)&s->sums, s->sums_host, 0));
     return PHX_OK;
 }
 
@@ -206,9 +212,7 @@ int initialize_t(phx_solver* s) {
         const int nw = phx::rk_generic_waves(s->iter->adaptive, c.N_c, c.N_r);
         PHX_HIP(hipMalloc((void**)&s->partials, 2 * sizeof(double) * (size_t)nw));
         s->allocs.push_back(s->partials);
-        PHX_HIP(hipMalloc((void**)&s->sums, 2 * sizeof(double)));
-        s->allocs.push_back(s->sums);
-        PHX_HIP(hipHostMalloc((void**)&s->sums_host, 2 * sizeof(double), hipHostMallocDefault));
+        if (int r = sums_alloc(s)) return r;
     }
     if (const char* e = std::getenv("PHX_MAX_REJECTIONS")) s->max_rejections = std::atoi(e);
     if (c.use_fft_mask && (!phx::fft_supported(c.N_c, sizeof(real)) || !phx::fft_supported(c.N_r, sizeof(real))))
@@ -286,10 +290,8 @@ int initialize_t(phx_solver* s) {
         }
         const size_t nb = phx::staged_final_blocks(c.N_c, c.N_r);
         if (int r = dev_alloc(s, (void**)&s->st_partials, 2 * nb * sizeof(double))) return r;
-        if (!s->sums) {
-            if (int r = dev_alloc(s, (void**)&s->sums, 2 * sizeof(double))) return r;
-            PHX_HIP(hipHostMalloc((void**)&s->sums_host, 2 * sizeof(double), hipHostMallocDefault));
-        }
+        if (!s->sums)
+            if (int r = sums_alloc(s)) return r;
     }
     if (c.imag_time_amplitude != 0.0) {
         if (int r = dev_alloc(s, (void**)&s->norm_partials, 2 * sizeof(double) * phx::imag_norm_blocks(N))) return r;
@@ -953,8 +955,7 @@ int step_body_t(phx_solver* s, double t_pre, double t_adv, bool force_fixed) {
             /* retries see the kernel time already advanced (updateKernelTime in adaptTimeStep, solver.cu:97) */
             const double t_k = rejections == 0 ? t_pre : t_adv;
             if (int r = rk_attempt<real>(s, s->iter->adaptive, t_k, s->dt)) return r;
-            PHX_HIP(hipMemcpyAsync(s->sums_host, s->sums, 2 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-            PHX_HIP(hipStreamSynchronize(s->stream));
+            PHX_HIP(hipStreamSynchronize(s->stream)); /* the reduction wrote its sums to pinned memory */
             double new_dt = 0, final_error = 0;
             const bool accept = adapt_dt(s->sums_host[0], s->sums_host[1], c.tolerance, s->dt, c.dt_min, c.dt_max,
                                          s->iter->power, &new_dt, &final_error);
