@@ -68,15 +68,21 @@ hipError_t launch_rk4_scalar(const Rk4Args<real>& a, const Rk4Tune& t, hipStream
 /* Many RK4 steps in one launch (rk4_scalar_flow): one step counter per wavefront tile in
    device memory (kFlowCounterStride ints apart), all equal to `base` when the launch starts
    and base + steps after it;
-   *error is set (and the state undefined) if a tile waited more than spin_limit polls for
+   the error word is set (and the state undefined) if a tile waited more than spin_limit polls for
    a neighbour.  Tiles: nstrips x nbands = ceil(Nc / 56) x ceil(Nr / ty). */
 constexpr int kFlowCounterStride = 32; /* ints: one 128-byte line per tile counter */
+enum { kFlowAll = 1, kFlowTickets = 2 }; /* values of the gate */
+/* Rk4Flow::words, kFlowCounterStride ints each: the error word; the next ticket, the blocks that have left and the
+   gate (who steps what), 0 between launches; then for each block its word, base + 1 once all blocks are resident */
+enum { kFlowError = 0, kFlowTicket, kFlowLeft, kFlowGate, kFlowGo };
 struct Rk4Flow {
     int* counters; /* tile t's counter at counters[t * kFlowCounterStride] */
-    int* error;
+    int* words;
     int base;
     int steps;
     int spin_limit;
+    int gate_limit; /* polls until a block gives up waiting for all others to be resident; < 0: tickets only */
+    int chunks;     /* blocks of four tiles a step (set by the launcher) */
 };
 template <typename real>
 hipError_t launch_rk4_flow(const Rk4Args<real>& a, const Rk4Tune& t, const Rk4Flow& f, hipStream_t s);

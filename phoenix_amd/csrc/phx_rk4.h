@@ -217,74 +217,200 @@ __global__ __launch_bounds__(256) void rk4_scalar_fused(Rk4Args<real> a) {
 /* Tile d (-2 .. 2) places away along one axis of n tiles of w cells (the last: the rest of N): its index, and
    `ok` cleared where it does not exist or the kHalo cells next to tile i do not reach it. */
 __device__ __forceinline__ int flow_reach(int i, int d, int n, int w, int N, bool periodic, bool& ok) {
-    int j = i + d;
-    if (j < 0 || j >= n) {
-        if (!periodic) ok = false;
-        j = (j + 2 * n) % n;
-    }
+    /* into 0 .. n - 1 for |d| <= 2 and n >= 1, without a division */
+    auto turned = [n](int j) {
+        j = j < 0 ? j + n : j >= n ? j - n : j;
+        return j < 0 ? j + n : j >= n ? j - n : j;
+    };
+    if (!periodic && (i + d < 0 || i + d >= n)) ok = false;
+    const int j = turned(i + d);
     if (d == 2 || d == -2) { /* cells of the tile in between */
-        const int m = (i + d / 2 + n) % n;
+        const int m = turned(i + (d > 0 ? 1 : -1));
         if ((m == n - 1 ? N - m * w : w) >= kHalo) ok = false;
     }
     return j;
 }
 
-/* Many steps in one launch, one resident wavefront per tile.  Before step k a tile waits
-   until the tiles whose cells its 4-cell halo covers (eight of them, more next to a narrow
-   last strip or band) have finished step k-1 (their step counters reach base + k): their outputs of step k-1 are its inputs, and their reads
-   of step k-1, which covered its cells in the buffer it is about to overwrite, are done.
+/* The tile whose counter this lane watches for tile (strip, band), -1: none.  Lanes 0..24 stand for the tiles up to
+   two strips and two bands away: the tile itself (kOwnLane), the next one on each side, and the one behind it where
+   the next is a last strip or band of fewer than kHalo cells. */
+constexpr int kOwnLane = 12;
+__device__ __forceinline__ int flow_watch(int strip, int band, int nstrips, int nbands, int TY, int Nc, int Nr, bool px, bool py) {
+    const int lane = threadIdx.x & (kWave - 1);
+    if (lane >= 25) return -1;
+    bool ok = true;
+    const int db = (lane * 13) >> 6; /* lane / 5 */
+    const int ns = flow_reach(strip, lane - 5 * db - 2, nstrips, kOutW, Nc, px, ok);
+    const int nb = flow_reach(band, db - 2, nbands, TY, Nr, py, ok);
+    return ok ? nb * nstrips + ns : -1;
+}
+/* Waits until the watched counters are at `need`; false: not within spin_limit polls. */
+__device__ __forceinline__ bool flow_wait(const int* theirs, int need, int spin_limit) {
+    int polls = 0;
+    bool ready = theirs == nullptr;
+    for (;;) {
+        if (!ready) ready = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= need;
+        if (__builtin_amdgcn_ballot_w64(!ready) == 0) break;
+        if (++polls > spin_limit) return false;
+        __builtin_amdgcn_s_sleep(4);
+    }
+    asm volatile("" ::: "memory");
+    return true;
+}
+
+/* Many steps in one launch.  Before step k a tile waits until it and the tiles whose cells its 4-cell halo
+   covers (eight of them, more next to a narrow last strip or band) have finished step k-1 (their step counters
+   reach base + k): their outputs of step k-1 are its inputs, and their reads of step k-1, which covered its
+   cells in the buffer it is about to overwrite, are done.
+   Who steps which tiles is settled while the kernel runs, so that it ends however few of its blocks are
+   resident, beside any other kernel and without a cooperative launch.  Ticket t stands for chunk t % chunks
+   (four tiles, tile_of) of step t / chunks; a block's first ticket gives it a chunk of step 0.
+   - If each of the first `chunks` tickets went to another block, all blocks are resident.  The block that drew
+     the last one says so (gate 0 -> kFlowAll, and a word for each block), and from step 1 on a block keeps one
+     chunk for all steps, next to those of its XCD (by ticket instead: 383 instead of 367 us), each wave for itself.
+   - A block that has waited gate_limit polls for that, after its step 0, closes the gate (0 -> kFlowTickets; the two writes
+     exclude each other) and from then on blocks take one ticket after the other.  A tile waits only for lower
+     tickets, and a ticket that has been taken is held by a resident block that finishes its lower ones first,
+     so the lowest unfinished ticket can always run.  Each step's order of chunks is turned by one row of
+     chunks against the step before, so that on a periodic grid the first chunks of a step wait for the first
+     ones of the step before and not for its last.
+   us per run of 50 steps, one handle alone / three in turn, and as a cooperative launch of one block a chunk:
+   1024^2 FP32 349 / 310 and 360 / 354, FP64 507 / 518 and 514 / 513, 600^2 FP32 217 / 128 and 234 / 227, FP64
+   284 / 201 and 278 / 272; tickets only: 1024^2 406 / 309, 551 / 519.  The cooperative launch also left a hardware
+   queue behind that slowed the launches of other handles (three of 150x116, 10 steps each: 97 instead of 23 us).
    psi and n go through device-scope loads and stores (no stale line of another XCD's
    write is used); a counter moves only after all stores of the step have completed.  Each
    counter has a 128-byte line of its own: packed 32 to a line, the polls of neighbouring
    tiles contended for the same lines and a step took 21 instead of 8 us at 1024^2.  A
-   wait longer than spin_limit polls sets *error and ends the wave (its neighbours then
-   time out too, so every wave exits); the state is then undefined. */
+   wait longer than spin_limit polls sets *error and ends the block (its neighbours then
+   time out too, so every block exits); the state is then undefined. */
 template <typename real, int TY, bool ISO, int PF, bool RES, bool PUMP, bool POT, bool PERY, bool CAMP = false>
 __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow f) {
+    /* The numbers that steer the tiles live in LDS: held in scalar registers across a tile's rows they push the
+       tile's own constants out of them.  The pointers do not: accesses through a pointer from LDS are flat ones,
+       and every wait for a row's loads then waits for all of them (FP64 600^2, 50 steps: 294 instead of 284 us). */
+    __shared__ struct {
+        int base, steps, spin_limit, gate_limit, chunks;
+    } sf;
+    __shared__ struct {
+        int chunk, step;
+    } sh[2]; /* by turns: written before the barrier that starts the turn in which they are read */
+    __shared__ int sh_late[2]; /* likewise; never cleared */
+    __shared__ int sh_go, sh_first, sh_turn, sh_gate; /* of thread 0: first ticket of the step, its turn; kFlowAll or kFlowTickets */
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    int strip, band;
-    if (!tile_of(xcd_contiguous(blockIdx.x, gridDim.x), wave, a.nstrips, a.nbands, strip, band))
-        return; /* no tile: nobody watches this wave's counter */
-    const int me = band * a.nstrips + strip;
-    /* lanes 0..24 watch the tiles up to two strips and two bands away that the halo reaches: the next one
-       on each side, and the one behind it where the next is a last strip or band of fewer than kHalo cells */
-    int watch = -1;
-    if (lane < 25) {
-        const int ds = lane % 5 - 2, db = lane / 5 - 2;
-        bool ok = lane != 12;
-        const int ns = flow_reach(strip, ds, a.nstrips, kOutW, a.Nc, a.periodic_x, ok);
-        const int nb = flow_reach(band, db, a.nbands, TY, a.Nr, PERY, ok);
-        if (ok) watch = nb * a.nstrips + ns;
-    }
-    int* const mine = f.counters + (size_t)me * kFlowCounterStride;
-    int* const theirs = watch < 0 ? nullptr : f.counters + (size_t)watch * kFlowCounterStride;
-    Rk4Args<real> s = a;
-    for (int k = 0; k < f.steps; k++) {
-        if (k > 0) {
-            const int need = f.base + k;
-            int polls = 0;
-            bool ready = theirs == nullptr;
-            for (;;) {
-                if (!ready) ready = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= need;
-                if (__builtin_amdgcn_ballot_w64(!ready) == 0) break;
-                if (++polls > f.spin_limit) {
-                    if (lane == 0) __hip_atomic_store(f.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    return;
-                }
-                __builtin_amdgcn_s_sleep(4);
-            }
-            asm volatile("" ::: "memory");
+    auto word = [&](int i) { return f.words + (size_t)i * kFlowCounterStride; };
+    auto draw = [&]() { return __hip_atomic_fetch_add(word(kFlowTicket), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    auto shut = [&]() { /* closes the gate unless it is open for all; what it is then */
+        int open = 0;
+        return __hip_atomic_compare_exchange_strong(word(kFlowGate), &open, kFlowTickets, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                   ? kFlowTickets
+                   : open;
+    };
+    auto give = [&](int par, int t) { /* ticket t: its chunk and step */
+        int first = sh_first, turn = sh_turn, k = sh[par ^ 1].step;
+        while (t - first >= sf.chunks) {
+            first += sf.chunks;
+            k++;
+            turn += a.nstrips;
+            if (turn >= sf.chunks) turn %= sf.chunks;
         }
-        const bool even = (k & 1) == 0;
-        s.psi_in = even ? a.psi_in : a.psi_out;
-        s.psi_out = even ? (typename Vec2<real>::type*)a.psi_out : (typename Vec2<real>::type*)a.psi_in;
-        s.n_in = even ? a.n_in : a.n_out;
-        s.n_out = even ? a.n_out : (real*)a.n_in;
-        rk4_tile<real, TY, ISO, PF, RES, PUMP, POT, PERY, kDeviceScope, kDeviceScope, CAMP>(s, strip, band);
-        /* all of this step's stores have completed before the counter moves */
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (lane == 0) __hip_atomic_store(mine, f.base + k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh_first = first;
+        sh_turn = turn;
+        const int c = t - first + turn;
+        sh[par].chunk = c >= sf.chunks ? c - sf.chunks : c;
+        sh[par].step = k;
+    };
+    if (threadIdx.x == 0) {
+        sf = {f.base, f.steps, f.spin_limit, f.gate_limit, f.chunks};
+        sh_first = sh_turn = sh_go = 0;
+        sh[1].step = 0;
+        const int t = draw();
+        give(0, t);
+        sh_late[0] = sh_late[1] = 0;
+        int gate = 0; /* not settled */
+        if (t >= f.chunks) {
+            gate = kFlowTickets;
+        } else if (f.gate_limit < 0) {
+            gate = shut();
+        } else if (t == f.chunks - 1) {
+            int open = 0;
+            if (!__hip_atomic_compare_exchange_strong(word(kFlowGate), &open, kFlowAll, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                gate = kFlowTickets;
+            else
+                sh_go = 1;
+        }
+        sh_gate = gate;
+    }
+    __syncthreads();
+    int gate = __builtin_amdgcn_readfirstlane(sh_gate);
+    if (sh_go)
+        for (int i = threadIdx.x; i < sf.chunks; i += blockDim.x)
+            __hip_atomic_store(word(kFlowGo + i), sf.base + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int par = 0;; par ^= 1) {
+        int k = __builtin_amdgcn_readfirstlane(sh[par].step);
+        if (k >= sf.steps || sh_late[par]) break;
+        /* the next ticket is taken ahead, so that its latency passes during this chunk */
+        int next = 0;
+        if (gate == kFlowTickets && threadIdx.x == 0) next = draw();
+        int strip, band;
+        bool late = false;
+        if (tile_of(__builtin_amdgcn_readfirstlane(sh[par].chunk), wave, a.nstrips, a.nbands, strip, band)) {
+            int* const mine = f.counters + (size_t)(band * a.nstrips + strip) * kFlowCounterStride;
+            const int watch = flow_watch(strip, band, a.nstrips, a.nbands, TY, a.Nc, a.Nr, a.periodic_x, PERY);
+            const int* theirs = watch < 0 ? nullptr : f.counters + (size_t)watch * kFlowCounterStride;
+            do { /* the step of a ticket, or all those left of a chunk that this block keeps */
+                if (k > 0 && !flow_wait(theirs, sf.base + k, sf.spin_limit)) {
+                    if (lane == 0) __hip_atomic_store(word(kFlowError), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    late = true;
+                    break;
+                }
+                const bool even = (k & 1) == 0;
+                Rk4Args<real> s = a;
+                s.psi_in = even ? a.psi_in : a.psi_out;
+                s.psi_out = even ? (typename Vec2<real>::type*)a.psi_out : (typename Vec2<real>::type*)a.psi_in;
+                s.n_in = even ? a.n_in : a.n_out;
+                s.n_out = even ? a.n_out : (real*)a.n_in;
+                rk4_tile<real, TY, ISO, PF, RES, PUMP, POT, PERY, kDeviceScope, kDeviceScope, CAMP>(s, strip, band);
+                /* all of this step's stores have completed before the counter moves */
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                k++;
+                if (lane == kOwnLane) theirs = nullptr; /* a kept chunk's own last step is behind it */
+                if (lane == 0) __hip_atomic_store(mine, sf.base + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } while (gate == kFlowAll && k < sf.steps);
+        }
+        if (gate == kFlowAll) break;
+        if (threadIdx.x == 0) {
+            if (gate == 0) { /* step 0 of the first ticket is done: are all blocks resident? */
+                const int* const go = word(kFlowGo + sh[par].chunk);
+                int polls = 0, settled = kFlowAll;
+                while (__hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != sf.base + 1) {
+                    if (++polls > sf.gate_limit) {
+                        settled = shut();
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(4);
+                }
+                sh_gate = settled;
+                if (settled == kFlowTickets) next = draw();
+            }
+            if (sh_gate == kFlowTickets) {
+                give(par ^ 1, next);
+            } else {
+                sh[par ^ 1].chunk = xcd_contiguous(blockIdx.x, gridDim.x);
+                sh[par ^ 1].step = 1;
+            }
+        }
+        if (late && lane == 0) sh_late[par ^ 1] = 1;
+        __syncthreads();
+        gate = __builtin_amdgcn_readfirstlane(sh_gate);
+    }
+    /* the last block to leave puts the words of this launch back for the next one */
+    __syncthreads();
+    if (threadIdx.x == 0 && __hip_atomic_fetch_add(word(kFlowLeft), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1) {
+        __hip_atomic_store(word(kFlowTicket), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(word(kFlowGate), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(word(kFlowLeft), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -400,19 +526,21 @@ inline hipError_t launch_flow_ty(const Rk4Args<real>& a0, const Rk4Flow& f, hipS
     Rk4Args<real> a = a0;
     a.nstrips = (a.Nc + kOutW - 1) / kOutW;
     a.nbands = (a.Nr + TY - 1) / TY;
-    const int nblocks = tile_blocks(a.nstrips, a.nbands);
-    const void* fn = a.periodic_y ? (const void*)&rk4_scalar_flow<real, TY, ISO, PF, RES, PUMP, POT, true, CAMP>
-                                  : (const void*)&rk4_scalar_flow<real, TY, ISO, PF, RES, PUMP, POT, false, CAMP>;
-    /* every wave must be resident at once: the cooperative launch refuses a grid that is not */
+    const auto fn = a.periodic_y ? &rk4_scalar_flow<real, TY, ISO, PF, RES, PUMP, POT, true, CAMP>
+                                 : &rk4_scalar_flow<real, TY, ISO, PF, RES, PUMP, POT, false, CAMP>;
     int per_cu = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kWave * kWavesPerBlock, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, kWave * kWavesPerBlock, 0) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return hipErrorNotSupported;
-    if ((long)per_cu * cus < nblocks) return hipErrorCooperativeLaunchTooLarge;
+    /* more blocks than the device holds at once would always go ticket by ticket, which is slower than launches
+       (2048^2, 20 steps: FP32 504 and 433 us, FP64 831 and 790 us) */
+    if (tile_blocks(a.nstrips, a.nbands) > (long)per_cu * cus) return hipErrorNotSupported;
     if (!f.counters) return hipSuccess; /* dry run: the kernel takes this grid */
     Rk4Flow fl = f;
-    void* args[] = {&a, &fl};
-    return hipLaunchCooperativeKernel(fn, dim3(nblocks), dim3(kWave * kWavesPerBlock), args, 0, s);
+    fl.chunks = tile_blocks(a.nstrips, a.nbands);
+    if ((int64_t)fl.chunks * f.steps >= (1 << 30)) return hipErrorNotSupported; /* tickets are ints */
+    hipLaunchKernelGGL(fn, dim3(fl.chunks), dim3(kWave * kWavesPerBlock), 0, s, a, fl);
+    return hipGetLastError();
 }
 
 template <typename real, bool ISO, int PF, bool RES, bool PUMP, bool POT, bool CAMP = false>
@@ -446,9 +574,8 @@ inline hipError_t launch_flow_flags(const Rk4Args<real>& a, const Rk4Tune& t, co
 }
 
 /* f.steps RK4 steps from a.psi_in / a.n_in; an even count leaves the result there, an odd
-   one in a.psi_out / a.n_out.  Errors: hipErrorNotSupported for a shape or tile height the
-   kernel does not take, hipErrorCooperativeLaunchTooLarge when its waves cannot all be
-   resident; the caller then steps launch by launch.  f.counters == nullptr: only check. */
+   one in a.psi_out / a.n_out.  Error: hipErrorNotSupported for a shape or tile height the
+   kernel does not take and for a grid whose blocks the device cannot hold at once; the caller then steps launch by launch.  f.counters == nullptr: only check. */
 template <typename real>
 hipError_t launch_rk4_flow(const Rk4Args<real>& a, const Rk4Tune& t, const Rk4Flow& f, hipStream_t s) {
     if ((size_t)a.Nc * (size_t)a.Nr * sizeof(typename Vec2<real>::type) > kMaxArrayBytes) return hipErrorInvalidValue;

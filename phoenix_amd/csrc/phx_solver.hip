@@ -104,9 +104,9 @@ struct phx_solver {
     bool graph_off = false;
     int64_t direct_steps = 0; /* steps of such runs launched one by one so far */
     /* the same runs as one launch of rk4_scalar_flow: per-tile step counters (all equal to
-       flow_base between launches) and the kernel's error word */
+       flow_base between launches) and Rk4Flow::words */
     int* flow_counters = nullptr;
-    int* flow_error = nullptr;
+    int* flow_words = nullptr;
     int flow_base = 0;
     int64_t flow_steps = 0, flow_launches = 0;
     bool flow_off = false;
@@ -1017,8 +1017,9 @@ int iterate(phx_solver* s, bool force_fixed) {
 constexpr int kGraphSteps = 50, kGraphMinSteps = 10;
 constexpr int64_t kGraphAfter = 400;
 
-/* One launch of rk4_scalar_flow for `steps` (even) steps of the same run; returns 1 when the
-   kernel cannot take this grid or launch shape (the caller falls back to the graph). */
+/* Polls of rk4_scalar_flow: for all blocks to be resident, after a block's first chunk (they start within a few us
+   unless another kernel is in their way; 8, 32 and 300 made no difference), and for a neighbour. */
+constexpr int kFlowGateLimit = 32;
 constexpr int kFlowSpinLimit = 1 << 21; /* polls of about 1 us: a wait of ~2 s ends the launch */
 
 /* Kernel arguments of a fixed RK4 step of the scalar model from psi/n `in` to `out`, with the
@@ -1049,13 +1050,11 @@ phx::Rk4Args<real> rk4_args(phx_solver* s, void* psi_in, void* n_in, void* psi_o
 }
 
 /* Whether a run of n steps goes to the multi-step kernel.  PHX_RK4_FLOW=0: never, 1: from 2 steps on.
-   Otherwise from 10 steps on, on grids whose 4-row tiles fill the SIMDs.  A cooperative launch costs about
-   15 us before its first step and no two of them run at once on a device, so short runs and small grids
-   are launched step by step (from a graph once they repeat), which leaves room for the kernels of other
-   handles.  us per run, one handle alone / three in turn, launches and multi-step (FP64 unless noted):
-   256^2 5 steps 32 / 25 and 43 / 34, 50 steps 199 / 95 and 212 / 208; 400^2 5 steps 37 / 27 and 45 / 36,
-   50 steps 252 / 137 and 234 / 226; 640^2 5 steps 48 / 24 and 50 / 43, 50 steps 349 / 269 and 288 / 307;
-   1024^2 10 steps 140 / 102 and 126 / 127, 50 steps 643 / 514 and 525 / 587, FP32 439 / 326 and 369 / 390. */
+   Otherwise from 10 steps on, on grids whose 4-row tiles fill the SIMDs.  Short runs and small grids are launched
+   step by step (from a graph once they repeat): their kernels leave room for those of other handles.  us per run,
+   one handle alone / three in turn, launches and multi-step: 600^2 FP32 50 steps 262 / 130 and 217 / 128, FP64
+   328 / 206 and 284 / 201; 1024^2 10 steps FP32 87 / 54 and 78 / 65, FP64 133 / 95 and 109 / 107; 50 steps FP32
+   415 / 266 and 349 / 310, FP64 636 / 474 and 507 / 518. */
 constexpr int64_t kFlowMinSteps = 10, kFlowMaxSteps = 500;
 
 bool flow_wanted(phx_solver* s, int64_t n) {
@@ -1072,17 +1071,19 @@ int flow_ready(phx_solver* s) {
     const size_t counters = (size_t)((c.N_c + 55) / 56) * (size_t)((c.N_r + 3) / 4) * phx::kFlowCounterStride;
     if (!s->flow_counters) {
         const phx::Rk4Args<real> a = rk4_args<real>(s, s->psi[0][s->cur], s->n[0][s->cur], s->psi[0][s->cur ^ 1], s->n[0][s->cur ^ 1]);
-        if (phx::launch_rk4_flow<real>(a, s->flow_tune, phx::Rk4Flow{nullptr, nullptr, 0, 2, 0}, s->stream) != hipSuccess) {
+        if (phx::launch_rk4_flow<real>(a, s->flow_tune, phx::Rk4Flow{.steps = 2}, s->stream) != hipSuccess) {
             (void)hipGetLastError();
             s->flow_off = true;
             return 1;
         }
         if (int r = dev_alloc(s, (void**)&s->flow_counters, counters * sizeof(int))) return r; /* any tile height >= 4 */
-        if (int r = dev_alloc(s, (void**)&s->flow_error, sizeof(int))) return r;
+        if (int r = dev_alloc(s, (void**)&s->flow_words, (phx::kFlowGo * phx::kFlowCounterStride + counters) * sizeof(int))) return r;
         s->flow_base = 0;
     }
     if (s->flow_base > (1 << 30)) { /* keep the counters far from overflow */
         PHX_HIP(hipMemsetAsync(s->flow_counters, 0, counters * sizeof(int), s->stream));
+        PHX_HIP(hipMemsetAsync(s->flow_words + phx::kFlowCounterStride, 0,
+                               ((phx::kFlowGo - 1) * phx::kFlowCounterStride + counters) * sizeof(int), s->stream));
         s->flow_base = 0;
     }
     return PHX_OK;
@@ -1095,7 +1096,9 @@ hipError_t flow_launch(phx_solver* s, const phx::Rk4Tune& tune, void* psi_in, vo
     int spin_limit = kFlowSpinLimit;
     if (const char* e = std::getenv("PHX_FLOW_SPIN_LIMIT")) spin_limit = std::atoi(e); /* tests of the time-out path */
     const phx::Rk4Args<real> a = rk4_args<real>(s, psi_in, n_in, psi_out, n_out);
-    const phx::Rk4Flow f{s->flow_counters, s->flow_error, s->flow_base, steps, spin_limit};
+    int gate_limit = kFlowGateLimit;
+    if (const char* e = std::getenv("PHX_FLOW_GATE_LIMIT")) gate_limit = std::atoi(e); /* tests of the ticket path */
+    const phx::Rk4Flow f{s->flow_counters, s->flow_words, s->flow_base, steps, spin_limit, gate_limit, 0};
     const hipError_t e = phx::launch_rk4_flow<real>(a, tune, f, s->stream);
     if (e == hipSuccess) {
         s->flow_base += steps;
@@ -1107,6 +1110,12 @@ hipError_t flow_launch(phx_solver* s, const phx::Rk4Tune& tune, void* psi_in, vo
 
 template <typename real>
 int flow_block_t(phx_solver* s, int steps) {
+    /* a launch counts from flow_base, so a captured one must not be replayed */
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return 1;
+    }
     if (int r = flow_ready<real>(s)) return r;
     if (flow_launch<real>(s, s->flow_tune, s->psi[0][s->cur], s->n[0][s->cur], s->psi[0][s->cur ^ 1], s->n[0][s->cur ^ 1], steps) !=
         hipSuccess) {
@@ -1205,12 +1214,12 @@ int autotune_flow(phx_solver* s) {
 /* The error word of rk4_scalar_flow, read after the stream has drained.  After a time-out the
    counters no longer match flow_base: the multi-step launch stays off for this handle. */
 int flow_check(phx_solver* s) {
-    if (!s->flow_error) return PHX_OK;
+    if (!s->flow_words) return PHX_OK;
     int err = 0;
-    PHX_HIP(hipMemcpy(&err, s->flow_error, sizeof(int), hipMemcpyDeviceToHost));
+    PHX_HIP(hipMemcpy(&err, s->flow_words, sizeof(int), hipMemcpyDeviceToHost));
     if (err) {
         s->flow_off = true;
-        PHX_HIP(hipMemset(s->flow_error, 0, sizeof(int))); /* reported once */
+        PHX_HIP(hipMemset(s->flow_words, 0, sizeof(int))); /* reported once */
         return fail(PHX_ERR_HIP, "multi-step RK4 launch: a tile waited too long for its neighbours; the state is undefined");
     }
     return PHX_OK;
