@@ -289,7 +289,7 @@ int phx_ensemble_get_field(phx_ensemble* e, int inst, int field, void* host, siz
 int phx_ensemble_device_ptr(phx_ensemble* e, int inst, int field, void** dptr);
 
 /* Output rows per wavefront tile of the batched kernel: 8, 10, 12, 16 or 20.
-   Without this call the first step times every height and keeps the fastest. */
+   Without this call the first step picks it by the number of tiles. */
 int phx_ensemble_set_tile_rows(phx_ensemble* e, int ty);
 
 /* n_steps RK4 steps of every instance.  graph_steps >= 2 captures that many

@@ -383,7 +383,7 @@ struct phx_adjoint {
     const void* P = nullptr; /* parameters of the last forward call (caller-owned) */
     const void* V = nullptr;
     bool have_forward = false;
-    int ty_fwd = 12, pf_fwd = 2, ty_adj = 32;
+    int ty_fwd = 12, ty_adj = 32;
     bool tuned = false;
     hipStream_t own = nullptr, stream = nullptr;
 
@@ -444,7 +444,7 @@ int fwd_step(phx_adjoint* a, const void* psi_in, const void* n_in, void* psi_out
     }
     c.ph = adj_phys<real>(a);
     b.iso = c.ph.kin_yx == real(1);
-    ADJ_HIP(phx::launch_rk4_batched<real>(b, ty, a->pf_fwd, a->res, a->pump, a->pot, st ? st : a->stream));
+    ADJ_HIP(phx::launch_rk4_batched<real>(b, ty, a->res, a->pump, a->pot, st ? st : a->stream));
     return PHX_OK;
 }
 
@@ -520,37 +520,29 @@ int autotune(phx_adjoint* a) {
         return PHX_OK;
     };
     const int fwd_tys[] = {8, 10, 12, 16, 20, 4};
-    const int fwd_pfs[] = {2, 4, 6};
     const int adj_tys[] = {16, 20, 24, 28, 32, 40, 48, 56, 64, 80};
-    float fwd_ms[6], pf_ms[3], adj_ms[10];
+    float fwd_ms[6], adj_ms[10];
     for (float& m : fwd_ms) m = 1e30f;
-    for (float& m : pf_ms) m = 1e30f;
     for (float& m : adj_ms) m = 1e30f;
     int rc = PHX_OK;
-    auto time_fwd = [&](int ty, int pf, float& best) {
-        float ms = 0;
-        a->pf_fwd = pf;
-        rc = timeit([&] { return fwd_step<real>(a, a->state_psi(a->ckpt_at(0)), a->state_n(a->ckpt_at(0)), a->state_psi(a->lam[1]),
-                                                a->state_n(a->lam[1]), ty); },
-                    ms);
-        if (!rc) best = std::min(best, ms);
-    };
     for (int pass = 0; pass < 3 && !rc; pass++) {
-        for (int i = 0; i < 6 && !rc; i++) time_fwd(fwd_tys[i], 4, fwd_ms[i]);
+        for (int i = 0; i < 6 && !rc; i++) {
+            float ms = 0;
+            rc = timeit([&] { return fwd_step<real>(a, a->state_psi(a->ckpt_at(0)), a->state_n(a->ckpt_at(0)), a->state_psi(a->lam[1]),
+                                                    a->state_n(a->lam[1]), fwd_tys[i]); },
+                        ms);
+            if (!rc) fwd_ms[i] = std::min(fwd_ms[i], ms);
+        }
         for (int i = 0; i < 10 && !rc; i++) {
             float ms = 0;
             rc = timeit([&] { return adj_step<real>(a, a->ckpt_at(0), 0, adj_tys[i]); }, ms);
             if (!rc) adj_ms[i] = std::min(adj_ms[i], ms);
         }
     }
-    const int ty_fwd = fwd_tys[std::min_element(fwd_ms, fwd_ms + 6) - fwd_ms];
-    for (int pass = 0; pass < 2; pass++) /* the forward kernel's prefetch depth at its best height */
-        for (int i = 0; i < 3 && !rc; i++) time_fwd(ty_fwd, fwd_pfs[i], pf_ms[i]);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    a->ty_fwd = ty_fwd;
-    a->pf_fwd = fwd_pfs[std::min_element(pf_ms, pf_ms + 3) - pf_ms];
+    a->ty_fwd = fwd_tys[std::min_element(fwd_ms, fwd_ms + 6) - fwd_ms];
     a->ty_adj = adj_tys[std::min_element(adj_ms, adj_ms + 10) - adj_ms];
     a->tuned = true;
     return PHX_OK;

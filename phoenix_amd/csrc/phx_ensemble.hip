@@ -48,8 +48,8 @@ struct phx_ensemble {
     /* per instance: offsets (bytes) of psi[2], n[2], pump, pot in the pool */
     std::vector<size_t> off_psi[2], off_n[2], off_pump, off_pot;
     int cur = 0;
-    int ty = 12, pf = 2; /* tile height, rows loaded ahead */
-    bool ty_auto = true; /* picked by timing at the first step */
+    int ty = 12;
+    bool ty_auto = true; /* tile height picked by rule_tile_rows at the first step */
     /* device tables for the two buffer parities and the tile list */
     void* entries[2] = {nullptr, nullptr};
     int* tile_inst = nullptr;
@@ -154,55 +154,35 @@ int launch_step(phx_ensemble* e, double dt, int parity) {
         b.common.vamp_h[k] = (real)e->ph.one_over_h_bar_s;
     }
     b.common.ph = phys_of<real>(e, 0);
-    ENS_HIP(phx::launch_rk4_batched<real>(b, e->tables_ty, e->pf, e->res, e->pump, e->pot, e->stream));
+    ENS_HIP(phx::launch_rk4_batched<real>(b, e->tables_ty, e->res, e->pump, e->pot, e->stream));
     return PHX_OK;
 }
 
-/* Pick the tile height and prefetch depth with the shortest step for this ensemble: every candidate
-   launch reads the current buffers and writes the other ones, so the state does not advance.  Some
-   launches first, so that the clocks have ramped up; then the heights at a middle depth, and the
-   depths at the best height (each candidate's fastest of two rounds). */
-template <typename real>
-int autotune(phx_ensemble* e, double dt) {
-    hipEvent_t e0, e1;
-    ENS_HIP(hipEventCreate(&e0));
-    ENS_HIP(hipEventCreate(&e1));
-    const int tys[] = {8, 10, 12, 16, 20, 4};
-    const int pfs[] = {2, 4, 6};
-    int rc = PHX_OK;
-    auto timed = [&](int ty, int pf, float& best) {
-        if (!rc && e->tables_ty != ty) rc = build_tables<real>(e, ty);
-        e->pf = pf;
-        if (!rc) rc = launch_step<real>(e, dt, e->cur);
-        if (!rc && hipEventRecord(e0, e->stream) != hipSuccess) rc = efail(PHX_ERR_HIP, "hipEventRecord");
-        for (int r = 0; r < 4 && !rc; r++) rc = launch_step<real>(e, dt, e->cur);
-        if (!rc && hipEventRecord(e1, e->stream) != hipSuccess) rc = efail(PHX_ERR_HIP, "hipEventRecord");
-        float ms = 0;
-        if (!rc && (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
-            rc = efail(PHX_ERR_HIP, "event timing");
-        if (!rc) best = std::min(best, ms);
+/* Tile height of an ensemble by its tiles over all instances, as rk4_default_tune picks it for one grid, but
+   20 rows where many rounds of tiles run: us per step at 4 / 8 / 10 / 12 / 16 / 20 rows (the rule's choice
+   in brackets), sides from {128 .. 512}: 0.33 M cells FP32 5.3 / [5.2] / 5.6 / 6.1 / 7.1 / 8.0; 0.57 M 6.9 /
+   6.9 / 7.6 / [6.5] / 7.4 / 8.4; 1.0 M 9.8 / 9.1 / [8.2] / 8.9 / 10.2 / 9.1, FP64 15.9 / 14.3 / 12.7 / 13.2 /
+   14.7 / [12.4]; 1.9 M 17.2 / 13.5 / 13.2 / 14.5 / 14.3 / [12.8]; 3.6 M 25.9 / 21.6 / 21.2 / 21.1 / 21.4 /
+   [20.6], FP64 44.1 / 36.3 / 35.2 / 33.9 / 34.9 / [34.8].  (Timing the heights on the first step cost 105
+   launches and six table builds, so that the first step took 5.8 instead of 1.4 ms, and picked within 3 % of
+   this.)  Loading 4 or 6 rows ahead instead of 2 moved no size by more than 2 %. */
+int rule_tile_rows(const phx_ensemble* e) {
+    auto tiles = [&](int ty) {
+        long n = 0;
+        for (int i = 0; i < e->n; i++) n += phx::rk4_tiles(e->Nc[i], e->Nr[i], ty);
+        return n;
     };
-    float ms[6] = {1e30f, 1e30f, 1e30f, 1e30f, 1e30f, 1e30f}, warm = 1e30f;
-    for (int i = 0; i < 4 && !rc; i++) timed(tys[2], pfs[1], warm);
-    for (int round = 0; round < 2 && !rc; round++)
-        for (int i = 0; i < 6 && !rc; i++) timed(tys[i], pfs[1], ms[i]);
-    const int ty = tys[std::min_element(ms, ms + 6) - ms];
-    float mp[3] = {1e30f, 1e30f, 1e30f};
-    for (int round = 0; round < 2 && !rc; round++)
-        for (int i = 0; i < 3 && !rc; i++) timed(ty, pfs[i], mp[i]);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (rc) return rc;
-    e->ty = ty;
-    e->pf = pfs[std::min_element(mp, mp + 3) - mp];
-    e->ty_auto = false;
-    return PHX_OK;
+    for (int ty : {4, 8, 12})
+        if (tiles(ty) <= phx::rk4_simds()) return ty;
+    return e->precision == PHX_FP32 && tiles(10) <= 2 * phx::rk4_simds() ? 10 : 20;
 }
 
 template <typename real>
 int step_t(phx_ensemble* e, double dt, int64_t n_steps, int graph_steps) {
-    if (e->ty_auto && n_steps > 0)
-        if (int r = autotune<real>(e, dt)) return r;
+    if (e->ty_auto && n_steps > 0) {
+        e->ty = rule_tile_rows(e);
+        e->ty_auto = false;
+    }
     if (e->tables_ty != e->ty)
         if (int r = build_tables<real>(e, e->ty)) return r;
     int64_t done = 0;

@@ -116,9 +116,9 @@ struct Rk4BatchArgs {
 };
 
 /* All instances share the feature set (reservoir / pump / potential) and dt.  ty: output rows per tile
-   (4, 8, 10, 12, 16, 20), pf: rows loaded ahead (2, or 4 and 6 for the pumped reservoir model with dx == dy) */
+   (4, 8, 10, 12, 16, 20) */
 template <typename real>
-hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, int pf, bool res, bool pump, bool pot, hipStream_t s);
+hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, bool res, bool pump, bool pot, hipStream_t s);
 
 /* wavefront tiles of one grid for the fused RK4 kernel with tile height ty */
 __host__ __device__ inline int rk4_tiles(int Nc, int Nr, int ty) { return ((Nc + 55) / 56) * ((Nr + ty - 1) / ty); }

@@ -614,22 +614,18 @@ inline hipError_t launch_batch_tys(const Rk4BatchArgs<real>& b, int ty, hipStrea
 }
 
 template <typename real, bool RES, bool PUMP, bool POT>
-inline hipError_t launch_batch_flags(const Rk4BatchArgs<real>& b, int ty, int pf, hipStream_t s) {
-    if constexpr (RES && PUMP) {
-        if (b.iso && pf == 4) return launch_batch_tys<real, true, 4, RES, PUMP, POT>(b, ty, s);
-        if (b.iso && pf == 6) return launch_batch_tys<real, true, 6, RES, PUMP, POT>(b, ty, s);
-    }
+inline hipError_t launch_batch_flags(const Rk4BatchArgs<real>& b, int ty, hipStream_t s) {
     return b.iso ? launch_batch_tys<real, true, 2, RES, PUMP, POT>(b, ty, s) : launch_batch_tys<real, false, 2, RES, PUMP, POT>(b, ty, s);
 }
 
 template <typename real>
-hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, int pf, bool res, bool pump, bool pot, hipStream_t s) {
+hipError_t launch_rk4_batched(const Rk4BatchArgs<real>& b, int ty, bool res, bool pump, bool pot, hipStream_t s) {
     /* (instance sizes are checked when the ensemble is created) */
     if (!b.entries && (size_t)b.common.Nc * (size_t)b.common.Nr * sizeof(typename Vec2<real>::type) > kMaxArrayBytes)
         return hipErrorInvalidValue;
-    if (!res) return pot ? launch_batch_flags<real, false, false, true>(b, ty, pf, s) : launch_batch_flags<real, false, false, false>(b, ty, pf, s);
-    if (pump) return pot ? launch_batch_flags<real, true, true, true>(b, ty, pf, s) : launch_batch_flags<real, true, true, false>(b, ty, pf, s);
-    return pot ? launch_batch_flags<real, true, false, true>(b, ty, pf, s) : launch_batch_flags<real, true, false, false>(b, ty, pf, s);
+    if (!res) return pot ? launch_batch_flags<real, false, false, true>(b, ty, s) : launch_batch_flags<real, false, false, false>(b, ty, s);
+    if (pump) return pot ? launch_batch_flags<real, true, true, true>(b, ty, s) : launch_batch_flags<real, true, true, false>(b, ty, s);
+    return pot ? launch_batch_flags<real, true, false, true>(b, ty, s) : launch_batch_flags<real, true, false, false>(b, ty, s);
 }
 
 } // namespace phx

@@ -6,6 +6,6 @@
 
 namespace phx {
 
-template hipError_t launch_rk4_batched<float>(const Rk4BatchArgs<float>&, int, int, bool, bool, bool, hipStream_t);
+template hipError_t launch_rk4_batched<float>(const Rk4BatchArgs<float>&, int, bool, bool, bool, hipStream_t);
 
 } // namespace phx

@@ -6,6 +6,6 @@
 
 namespace phx {
 
-template hipError_t launch_rk4_batched<double>(const Rk4BatchArgs<double>&, int, int, bool, bool, bool, hipStream_t);
+template hipError_t launch_rk4_batched<double>(const Rk4BatchArgs<double>&, int, bool, bool, bool, hipStream_t);
 
 } // namespace phx
