@@ -202,7 +202,7 @@ int phx_get_info(phx_solver* s, phx_info* info);
 /* Use an external HIP stream (hipStream_t passed as void*) for all work of this
    handle; NULL restores the handle's own stream (so the null stream itself cannot be set: a
    caller whose work runs on it orders a stream of its own with events).  The same holds for
-   phx_ensemble_set_stream and phx_adjoint_set_stream. */
+   phx_ensemble_set_stream; phx_adjoint_set_stream also takes PHX_NULL_STREAM. */
 int phx_set_stream(phx_solver* s, void* stream);
 
 /* Wait for all device work of the handle. */
@@ -333,8 +333,9 @@ int phx_adjoint_forward(phx_adjoint* a, const void* psi0, const void* n0, const 
 int phx_adjoint_backward(phx_adjoint* a, const void* g_psi_T, const void* g_n_T, void* g_pump, void* g_pot, void* g_psi0,
                          void* g_n0);
 
-/* Run on a caller-owned hipStream_t (NULL: the handle's own stream).  The backward's recompute
-   stream waits for this stream's earlier work. */
+/* Run on a caller-owned hipStream_t (NULL: the handle's own stream; PHX_NULL_STREAM: the device's null
+   stream).  The backward's recompute stream waits for this stream's earlier work. */
+#define PHX_NULL_STREAM ((void*)1)
 int phx_adjoint_set_stream(phx_adjoint* a, void* stream);
 int phx_adjoint_sync(phx_adjoint* a);
 void phx_adjoint_destroy(phx_adjoint* a);

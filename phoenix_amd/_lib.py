@@ -37,6 +37,7 @@ EXPORTED = [
     "phx_step_at", "phx_rk4_scalar_device_noalloc",
 ]
 PHX_ENS_RESERVOIR, PHX_ENS_PUMP, PHX_ENS_POTENTIAL = 1, 2, 4
+PHX_NULL_STREAM = 1
 def stream_arg(stream_ptr: Optional[int]):
     """hipStream_t for the set_stream entry points, whose NULL selects the handle's own stream.
     None -> the handle's own stream.  A handle of 0 (torch's default stream) is refused: it would
@@ -382,6 +383,10 @@ class Adjoint:
 
     def set_stream(self, stream_ptr: Optional[int]):
         check(lib().phx_adjoint_set_stream(self._h, stream_arg(stream_ptr)))
+
+    def set_null_stream(self):
+        """Run on the device's null stream (torch's default stream)."""
+        check(lib().phx_adjoint_set_stream(self._h, PHX_NULL_STREAM))
 
     def sync(self):
         check(lib().phx_adjoint_sync(self._h))

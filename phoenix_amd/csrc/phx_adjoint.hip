@@ -678,7 +678,8 @@ int phx_adjoint_create(phx_adjoint** out, int precision, const phx_physics* ph, 
                              hipMalloc(&a->seg[1], (a->K - 1) * a->sbytes) == hipSuccess));
     ok = ok && hipMalloc(&a->lam[0], a->sbytes) == hipSuccess && hipMalloc(&a->lam[1], a->sbytes) == hipSuccess;
     ok = ok && hipMalloc(&a->gp, rb) == hipSuccess && hipMalloc(&a->gv, rb) == hipSuccess;
-    ok = ok && hipStreamCreate(&a->own) == hipSuccess && hipStreamCreate(&a->aux) == hipSuccess;
+    /* aux is ordered by events alone: with the null stream as the main one it must not wait for every launch there */
+    ok = ok && hipStreamCreate(&a->own) == hipSuccess && hipStreamCreateWithFlags(&a->aux, hipStreamNonBlocking) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&a->ev_start, hipEventDisableTiming) == hipSuccess;
     a->ev_rec.assign(a->nseg, nullptr);
     a->ev_adj.assign(a->nseg, nullptr);
@@ -714,7 +715,7 @@ int phx_adjoint_backward(phx_adjoint* a, const void* g_psi_T, const void* g_n_T,
 
 int phx_adjoint_set_stream(phx_adjoint* a, void* stream) {
     if (!a) return afail(PHX_ERR_INVALID, "null handle");
-    a->stream = stream ? (hipStream_t)stream : a->own;
+    a->stream = stream == PHX_NULL_STREAM ? (hipStream_t) nullptr : stream ? (hipStream_t)stream : a->own;
     return PHX_OK;
 }
 
