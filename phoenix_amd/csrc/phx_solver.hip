@@ -1050,16 +1050,17 @@ phx::Rk4Args<real> rk4_args(phx_solver* s, void* psi_in, void* n_in, void* psi_o
 }
 
 /* Whether a run of n steps goes to the multi-step kernel.  PHX_RK4_FLOW=0: never, 1: from 2 steps on.
-   Otherwise from 10 steps on, on grids whose 4-row tiles fill the SIMDs.  Short runs and small grids are launched
+   Otherwise from 10 steps on, on grids of one and a half 4-row tiles a SIMD.  Short runs and small grids are launched
    step by step (from a graph once they repeat): their kernels leave room for those of other handles.  us per run,
    one handle alone / three in turn, launches and multi-step: 600^2 FP32 50 steps 262 / 130 and 217 / 128, FP64
    328 / 206 and 284 / 201; 1024^2 10 steps FP32 87 / 54 and 78 / 65, FP64 133 / 95 and 109 / 107; 50 steps FP32
-   415 / 266 and 349 / 310, FP64 636 / 474 and 507 / 518. */
+   415 / 266 and 349 / 310, FP64 636 / 474 and 507 / 518; below the line 512^2 FP32 with a potential, 68 steps:
+   365 / 175 and 362 / 185 to 271. */
 constexpr int64_t kFlowMinSteps = 10, kFlowMaxSteps = 500;
 
 bool flow_wanted(phx_solver* s, int64_t n) {
     if (const char* e = std::getenv("PHX_RK4_FLOW")) return std::atoi(e) != 0 && n >= 2;
-    return n >= kFlowMinSteps && phx::rk4_tiles(s->cfg.N_c, s->cfg.N_r, 4) > phx::rk4_simds();
+    return n >= kFlowMinSteps && 2 * phx::rk4_tiles(s->cfg.N_c, s->cfg.N_r, 4) > 3 * phx::rk4_simds();
 }
 
 /* Counters of the multi-step kernel, allocated on first use once the kernel is known to take
@@ -1201,6 +1202,15 @@ int autotune_flow(phx_solver* s) {
     int best = -1;
     for (int cand = 0; cand < nty * npf; cand++)
         if (ms[cand] < 1e29f && (best < 0 || ms[cand] < ms[best])) best = cand;
+    /* of heights within 3 % of the fastest the tallest: it reads the fewest halo rows again, which counts beside other
+       handles (1024^2 FP64, 50 steps and a filter: 10 rows 571 us alone and 605 with three in turn, 20 rows 562 and 520) */
+    if (best >= 0) {
+        const float within = 1.03f * ms[best];
+        for (int cand = 0; cand < nty * npf; cand++) {
+            const int ty = tys[cand % nty], best_ty = tys[best % nty];
+            if (ms[cand] <= within && (ty > best_ty || (ty == best_ty && ms[cand] < ms[best]))) best = cand;
+        }
+    }
     if (best < 0) {
         s->flow_off = true;
         return PHX_OK;
