@@ -251,7 +251,7 @@ def time_batched(instances: int, steps: int, seed: int = 99, graph_steps: int = 
         seq.append((int(N), t[0], t[1], t[2], torch.empty_like(t[0]), torch.empty_like(t[1])))
     cells = int(sum(int(N) ** 2 for N in sides))
     torch.cuda.synchronize()
-    # warm-up: autotune of the tile height and graph capture, without advancing the timed state twice
+    # warm-up: tile tables and graph capture, without advancing the timed state twice
     ens.step(dt, graph_steps, graph_steps=graph_steps)
     ens.step(dt, graph_steps, graph_steps=graph_steps)
     ens.sync()
