@@ -1300,6 +1300,7 @@ int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     }
     if (graphs && s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream && s->graph_parity == s->cur && s->graph_steps <= m) {
         PHX_HIP(hipGraphLaunch(s->graph, s->stream));
+        s->direct_steps = 0; /* the rest of a run that the graph serves is no reason to capture a shorter one */
         return took(advance_steps(s, s->graph_steps, t_stop, t, fc));
     }
     /* (a run that starts in the other buffer than the captured one is launched too, not captured anew) */
