@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "phx_row_wrap.h"
+
 namespace phx {
 
 constexpr int kWave = 64;
@@ -54,29 +56,6 @@ __device__ __forceinline__ bool tile_of(int block, int wave, int nstrips, int nb
     strip = t / rem;
     band = groups * kWavesPerBlock + t % rem;
     return true;
-}
-
-/* Periodic row wrap without branches, so that a fully unrolled row loop stays one
-   basic block (a branch there splits it, and DPP moves then no longer fold into the
-   adds that consume them).  x mod Nr for x = g + bias >= 0 is x - Nr * q with
-   q = mulhi(x, ceil(2^32 / Nr)), exact whenever x * Nr < 2^32; g >= -halo, and
-   bias = Nr (Nr >= halo) or Nr * halo keeps x below 3 Nr + the tile height. */
-struct RowWrap {
-    uint32_t nr, magic, bias;
-};
-__device__ __forceinline__ RowWrap make_row_wrap(int Nr, int halo) {
-    RowWrap w;
-    w.nr = (uint32_t)Nr;
-    w.magic = 0xFFFFFFFFu / (uint32_t)Nr + 1u; /* ceil(2^32 / Nr) for Nr >= 2 */
-    w.bias = Nr >= halo ? (uint32_t)Nr : (uint32_t)(Nr * halo);
-    return w;
-}
-/* Row of tile row g: wrapped into [0, Nr) (exact modulo for periodic grids; for a
-   zero boundary `in` says whether g lies in the grid, the wrapped row is then unused). */
-__device__ __forceinline__ uint32_t tile_row(int g, const RowWrap& w, int periodic, bool& in) {
-    in = periodic || (g >= 0 && g < (int)w.nr);
-    const uint32_t x = (uint32_t)g + w.bias;
-    return x - __umulhi(x, w.magic) * w.nr;
 }
 
 template <int CTRL>
