@@ -125,6 +125,9 @@ int build_tables(phx_ensemble* e, int ty) {
     }
     /* launches still queued on the stream read the old tables: let them finish first */
     if (e->stream) ENS_HIP(hipStreamSynchronize(e->stream));
+    /* and a captured run holds their addresses */
+    if (e->graph) ENS_HIP(hipGraphExecDestroy(e->graph));
+    e->graph = nullptr;
     for (int par = 0; par < 2; par++) {
         if (e->entries[par]) ENS_HIP(hipFree(e->entries[par]));
         ENS_HIP(hipMalloc(&e->entries[par], ent[par].size() * sizeof(ent[par][0])));
