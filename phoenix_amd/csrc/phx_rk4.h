@@ -296,7 +296,8 @@ __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow 
         int chunk, step;
     } sh[2]; /* by turns: written before the barrier that starts the turn in which they are read */
     __shared__ int sh_late[2]; /* likewise; never cleared */
-    __shared__ int sh_go, sh_first, sh_turn, sh_gate; /* of thread 0: first ticket of the step, its turn; kFlowAll or kFlowTickets */
+    __shared__ int sh_gate[2]; /* likewise: 0 (not settled), kFlowAll or kFlowTickets */
+    __shared__ int sh_go, sh_first, sh_turn; /* of thread 0: first ticket of the step, its turn */
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     auto word = [&](int i) { return f.words + (size_t)i * kFlowCounterStride; };
@@ -340,10 +341,10 @@ __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow 
             else
                 sh_go = 1;
         }
-        sh_gate = gate;
+        sh_gate[0] = gate;
     }
     __syncthreads();
-    int gate = __builtin_amdgcn_readfirstlane(sh_gate);
+    int gate = __builtin_amdgcn_readfirstlane(sh_gate[0]);
     if (sh_go)
         for (int i = threadIdx.x; i < sf.chunks; i += blockDim.x)
             __hip_atomic_store(word(kFlowGo + i), sf.base + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -381,9 +382,11 @@ __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow 
         }
         if (gate == kFlowAll) break;
         if (threadIdx.x == 0) {
+            int settled = gate;
             if (gate == 0) { /* step 0 of the first ticket is done: are all blocks resident? */
                 const int* const go = word(kFlowGo + sh[par].chunk);
-                int polls = 0, settled = kFlowAll;
+                int polls = 0;
+                settled = kFlowAll;
                 while (__hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != sf.base + 1) {
                     if (++polls > sf.gate_limit) {
                         settled = shut();
@@ -391,10 +394,10 @@ __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow 
                     }
                     __builtin_amdgcn_s_sleep(4);
                 }
-                sh_gate = settled;
                 if (settled == kFlowTickets) next = draw();
             }
-            if (sh_gate == kFlowTickets) {
+            sh_gate[par ^ 1] = settled;
+            if (settled == kFlowTickets) {
                 give(par ^ 1, next);
             } else {
                 sh[par ^ 1].chunk = xcd_contiguous(blockIdx.x, gridDim.x);
@@ -403,7 +406,7 @@ __global__ __launch_bounds__(256) void rk4_scalar_flow(Rk4Args<real> a, Rk4Flow 
         }
         if (late && lane == 0) sh_late[par ^ 1] = 1;
         __syncthreads();
-        gate = __builtin_amdgcn_readfirstlane(sh_gate);
+        gate = __builtin_amdgcn_readfirstlane(sh_gate[par ^ 1]);
     }
     /* the last block to leave puts the words of this launch back for the next one */
     __syncthreads();
