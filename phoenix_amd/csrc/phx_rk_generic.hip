@@ -197,12 +197,15 @@ int dp45_adaptive_tile_rows(bool tetm, bool fp32, int Nc, int Nr) {
        tile, S (TY + 2 S) - S (S + 1) for S = 7.  us per attempt, FP32 TE-TM, 8 / 16 / 28 / 32 / 42 rows
        (the rule's choice in brackets): 2048^2 with noise 365 / 318 / 242 / 266 / [229], without 303 / 265 /
        202 / 221 / [190]; 1536 x 1200 148 / 141 / 137 / 150 / [103]; 1024^2 95 / 99 / [78] / 85 / 101; 600^2
-       [43] / 56 / 72 / 79 / 95; FP64 1024^2 488 / [482], 300^2 [126] / 171. */
+       [43] / 56 / 72 / 79 / 95; FP64 1024^2 [488] / 482, 300^2 [126] / 171. */
     constexpr int S = 7;
     int best = kRkGenTileRows;
     long best_cost = -1;
     for (int ty : {16, 8, 28, 32, 42}) {
         if (ty > kRkGenTileRows && !tall) continue;
+        /* the 42-row tiles address ten rows further past the grid's end than the 32-row ones (launch_gen): a
+           grid of nearly 2 GiB a field stays with those */
+        if (ty > 32 && (size_t)Nc * (size_t)(Nr + ty + S) * sizeof(float2) > kMaxArrayBytes) continue;
         const long blocks = tile_blocks((Nc + 63 - 2 * S) / (64 - 2 * S), (Nr + ty - 1) / ty), cus = rk4_simds() / 4;
         const long cost = ((blocks + cus - 1) / cus) * (long)(S * (ty + 2 * S) - S * (S + 1));
         if (best_cost < 0 || cost < best_cost) best = ty, best_cost = cost;
