@@ -90,6 +90,8 @@ typedef struct {
     int32_t complex_reservoir;  /* 1: the reservoir fields are complex ({re, im} per cell: PHX_N_PLUS /
                                    PHX_N_MINUS take 2 N_c N_r reals), as the reference's n becomes under
                                    --imagTime with a reservoir or a complex temporal pump envelope */
+    int32_t graph_replays;      /* replays of captured runs of single-step launches so far (in what was padding:
+                                   the struct keeps its size) */
 } phx_info;
 
 /* Parse PHOENIX flags (argv[0] is the program name and is skipped), including

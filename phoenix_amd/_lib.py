@@ -67,7 +67,7 @@ class PhxInfo(C.Structure):
         ("fft_every", C.c_double), ("tolerance", C.c_double), ("dt_min", C.c_double), ("dt_max", C.c_double),
         ("iteration", C.c_int64), ("rejected", C.c_int64), ("tile_rows", C.c_int32), ("prefetch_rows", C.c_int32),
         ("staged", C.c_int32), ("multi_step_steps", C.c_int64), ("multi_step_launches", C.c_int64),
-        ("complex_reservoir", C.c_int32),
+        ("complex_reservoir", C.c_int32), ("graph_replays", C.c_int32),
     ]
 
     def as_dict(self):

@@ -102,7 +102,9 @@ struct phx_solver {
     double graph_dt = 0;
     hipStream_t graph_stream = nullptr;
     bool graph_off = false;
-    int64_t direct_steps = 0; /* steps of such runs launched one by one so far */
+    int64_t direct_steps = 0; /* steps of such runs launched one by one since the last replay or capture */
+    int64_t short_steps = 0;  /* steps replayed since the capture that a longer graph would have served */
+    int64_t graph_replays = 0;
     /* the same runs as one launch of rk4_scalar_flow: per-tile step counters (all equal to
        flow_base between launches) and Rk4Flow::words */
     int* flow_counters = nullptr;
@@ -1272,9 +1274,16 @@ int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     if (m < 2) return PHX_OK;
     const char* ge = std::getenv("PHX_GRAPH"); /* PHX_GRAPH=0: launch by launch */
     const bool graphs = !s->graph_off && !(ge && std::atoi(ge) == 0);
-    const bool same = s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream;
-    if (graphs && s->direct_steps >= kGraphAfter && m >= kGraphMinSteps && !(same && s->graph_steps <= m)) {
-        const int cur = s->cur, steps = (int)std::min<int64_t>(m, kGraphSteps) & ~1;
+    const int steps = (int)std::min<int64_t>(m, kGraphSteps) & ~1; /* of a graph for this run */
+    auto serves = [&] {
+        return s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream && s->graph_parity == s->cur && s->graph_steps <= m;
+    };
+    /* a new graph once the runs that none serves, or that one serves with fewer steps than they could take at a
+       time, have come to kGraphAfter steps */
+    if (graphs && m >= kGraphMinSteps &&
+        (serves() ? s->graph_steps < steps && s->short_steps >= kGraphAfter : s->direct_steps >= kGraphAfter)) {
+        s->short_steps = 0;
+        const int cur = s->cur;
         s->direct_steps = 0;
         if (s->graph) PHX_HIP(hipGraphExecDestroy(s->graph));
         s->graph = nullptr;
@@ -1298,12 +1307,13 @@ int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
             s->graph_steps = steps;
         }
     }
-    if (graphs && s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream && s->graph_parity == s->cur && s->graph_steps <= m) {
+    if (graphs && serves()) {
         PHX_HIP(hipGraphLaunch(s->graph, s->stream));
+        s->graph_replays++;
         s->direct_steps = 0; /* the rest of a run that the graph serves is no reason to capture a shorter one */
+        if (s->graph_steps < steps) s->short_steps += s->graph_steps;
         return took(advance_steps(s, s->graph_steps, t_stop, t, fc));
     }
-    /* (a run that starts in the other buffer than the captured one is launched too, not captured anew) */
     for (int64_t k = 0; k < m; k++)
         if (int r = rk4_launch<real>(s, s->t, s->dt)) return r;
     s->direct_steps += m;
@@ -1654,6 +1664,7 @@ int phx_get_info(phx_solver* s, phx_info* info) {
     info->staged = s->staged;
     info->multi_step_steps = s->flow_steps;
     info->multi_step_launches = s->flow_launches;
+    info->graph_replays = (int32_t)std::min<int64_t>(s->graph_replays, INT32_MAX);
     info->complex_reservoir = s->cfg.complex_reservoir;
     return PHX_OK;
 }
