@@ -57,6 +57,14 @@ struct Rk4Tune {
     int ty = 16, ew = 1, pf = 2;
 };
 
+/* whether a caller is capturing the stream */
+inline bool stream_capturing(hipStream_t s) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
 /* SIMDs of the device (four a CU) */
 int rk4_simds();
 /* tile height of an untimed launch (phx_rk_generic.hip) */

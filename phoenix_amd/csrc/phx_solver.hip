@@ -1114,11 +1114,7 @@ hipError_t flow_launch(phx_solver* s, const phx::Rk4Tune& tune, void* psi_in, vo
 template <typename real>
 int flow_block_t(phx_solver* s, int steps) {
     /* a launch counts from flow_base, so a captured one must not be replayed */
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return 1;
-    }
+    if (phx::stream_capturing(s->stream)) return 1;
     if (int r = flow_ready<real>(s)) return r;
     if (flow_launch<real>(s, s->flow_tune, s->psi[0][s->cur], s->n[0][s->cur], s->psi[0][s->cur ^ 1], s->n[0][s->cur ^ 1], steps) !=
         hipSuccess) {
@@ -1273,7 +1269,8 @@ int block_t(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) {
     }
     if (m < 2) return PHX_OK;
     const char* ge = std::getenv("PHX_GRAPH"); /* PHX_GRAPH=0: launch by launch */
-    const bool graphs = !s->graph_off && !(ge && std::atoi(ge) == 0);
+    /* nor into a caller's capture: a replay there runs at once and is not recorded */
+    const bool graphs = !s->graph_off && !(ge && std::atoi(ge) == 0) && !phx::stream_capturing(s->stream);
     const int steps = (int)std::min<int64_t>(m, kGraphSteps) & ~1; /* of a graph for this run */
     auto serves = [&] {
         return s->graph && s->graph_dt == s->dt && s->graph_stream == s->stream && s->graph_parity == s->cur && s->graph_steps <= m;

@@ -100,3 +100,33 @@ def test_runs_cut_by_the_filter(prec):
     check(state(a), state(b))
     a.close()
     b.close()
+
+
+def test_capture_by_the_caller():
+    """a caller captures phx_step on its own stream while the handle holds a graph: the launches are recorded"""
+    import torch
+    stream = torch.cuda.Stream()
+    a, b = start("fp32"), start("fp32")
+    a.set_stream(stream.cuda_stream)
+    for s in (a, b):
+        for _ in range(50):
+            s.step(10)
+    a.sync()
+    assert a.info["graph_replays"] > 0
+    replays = a.info["graph_replays"]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        assert a.step(20) == 20
+    assert a.info["graph_replays"] == replays
+    for k in range(4):
+        print(f"[graph runs] replay {k}", flush=True)
+        with torch.cuda.stream(stream):
+            g.replay()
+        stream.synchronize()
+        b.step(20)
+        assert np.array_equal(a.get("psi_plus"), b.get("psi_plus")) and np.array_equal(a.get("n_plus"), b.get("n_plus"))
+    a.step(3)
+    b.step(3)
+    assert np.array_equal(a.get("psi_plus"), b.get("psi_plus"))
+    a.close()
+    b.close()
