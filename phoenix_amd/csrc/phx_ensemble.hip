@@ -190,7 +190,8 @@ int step_t(phx_ensemble* e, double dt, int64_t n_steps, int graph_steps) {
         if (int r = build_tables<real>(e, e->ty)) return r;
     int64_t done = 0;
     graph_steps &= ~1; /* even: the buffers return to the same parity */
-    bool replay = graph_steps >= 2 && n_steps >= graph_steps;
+    /* (into a caller's capture go the launches: a replay there runs at once and is not recorded) */
+    bool replay = graph_steps >= 2 && n_steps >= graph_steps && !phx::stream_capturing(e->stream);
     /* the captured launches hard-wire the buffer parity they start from */
     if (replay && (!e->graph || e->graph_steps != graph_steps || e->graph_dt != dt || e->graph_ty != e->ty ||
                    e->graph_parity != e->cur)) {

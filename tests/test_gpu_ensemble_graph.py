@@ -25,3 +25,33 @@ def test_tile_height_there_and_back(prec, between):
         assert np.array_equal(a.get(i, "n_plus"), b.get(i, "n_plus"))
     a.close()
     b.close()
+
+
+def test_capture_by_the_caller():
+    """a caller captures Ensemble.step on its own stream while the ensemble holds a graph for that call"""
+    import torch
+    print("[ensemble graph] captured by the caller", flush=True)
+    dt, stream = 0.02, torch.cuda.Stream()
+    a, *_ = make_ensemble("fp32")
+    b, *_ = make_ensemble("fp32")
+    a.set_stream(stream.cuda_stream)
+    for e in (a, b):
+        e.step(dt, 12, graph_steps=6)
+    a.sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        a.step(dt, 6, graph_steps=6)
+    for k in range(4):
+        print(f"  replay {k}", flush=True)
+        with torch.cuda.stream(stream):
+            g.replay()
+        stream.synchronize()
+        b.step(dt, 6)
+        for i in range(len(SIZES)):
+            assert np.array_equal(a.get(i, "psi_plus"), b.get(i, "psi_plus"))
+            assert np.array_equal(a.get(i, "n_plus"), b.get(i, "n_plus"))
+    a.step(dt, 12, graph_steps=6)
+    b.step(dt, 12)
+    assert np.array_equal(a.get(0, "psi_plus"), b.get(0, "psi_plus"))
+    a.close()
+    b.close()
