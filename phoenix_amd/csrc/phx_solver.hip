@@ -650,7 +650,8 @@ int rk_attempt(phx_solver* s, phx::RkTableau tab, double t_k, double dt) {
 template <typename real>
 int fft_filter_t(phx_solver* s) {
     auto& c = s->cfg;
-    if (!s->fft_c.table || !s->fft_r.table) return fail(PHX_ERR_STATE, "no FFT mask in this configuration");
+    /* (SSFM and spectra for output have the transforms without a mask) */
+    if (!s->fft_c.table || !s->fft_r.table || !s->mask[0]) return fail(PHX_ERR_STATE, "no FFT mask in this configuration");
     using v2 = typename phx::Vec2<real>::type;
     for (int k = 0; k < (c.tetm ? 2 : 1); k++)
         PHX_HIP(phx::launch_fft_filter<real>((v2*)s->psi[k][s->cur], s->fft_c, s->fft_r, (const real*)s->mask[k], s->stream,
