@@ -856,6 +856,12 @@ int ssfm_block(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) 
     return PHX_OK;
 }
 
+/* Whether a tile height is worth timing on a grid: 2- and 4-row tiles evaluate 4.1 and 2.5 times the rows that they
+   write (16 rows: 1.4) and pay only where the tiles run in a round or two.  The first step with every height timed,
+   and with these two left out beyond: 2048^2 FP32 27 and 19 ms, 4096^2 115 and 80, FP64 46 / 32, 217 / 150; no grid of
+   600^2 to 1100^2 picked either. */
+bool tall_enough(const phx_solver* s, int ty) { return ty > 4 || phx::rk4_tiles(s->cfg.N_c, s->cfg.N_r, ty) <= 2 * phx::rk4_simds(); }
+
 /* Autotuner of the fused RK4 launch shape: time each candidate tile height on this
    grid (writing into the spare buffers, so the state is untouched) and keep the
    fastest.  Results are cached per (precision, grid, feature set) for the process.
@@ -889,6 +895,7 @@ int autotune_rk4(phx_solver* s) {
             phx::Rk4Tune t = s->tune;
             t.ty = cands[cand % ncand];
             t.pf = pfs[cand / ncand];
+            if (!tall_enough(s, t.ty)) continue;
             const phx::Rk4Tune keep = s->tune;
             s->tune = t;
             int rc = PHX_OK;
@@ -1182,6 +1189,7 @@ int autotune_flow(phx_solver* s) {
             phx::Rk4Tune t = one_step;
             t.ty = tys[cand % nty];
             t.pf = pfs[cand / nty];
+            if (!tall_enough(s, t.ty)) continue;
             if (hipEventRecord(e0, s->stream) != hipSuccess) rc = fail(PHX_ERR_HIP, "hipEventRecord");
             if (!rc && flow_launch<real>(s, t, psi2, n2, tmp_psi, tmp_n, kFlowTuneSteps) != hipSuccess) continue;
             float m = 0;
