@@ -862,23 +862,39 @@ int ssfm_block(phx_solver* s, int64_t max_steps, double t_stop, int64_t* taken) 
    600^2 to 1100^2 picked either. */
 bool tall_enough(const phx_solver* s, int ty) { return ty > 4 || phx::rk4_tiles(s->cfg.N_c, s->cfg.N_r, ty) <= 2 * phx::rk4_simds(); }
 
+/* Launch shapes found in this process, by configuration; handles on several threads share them. */
+class TuneCache {
+    std::mutex mu;
+    std::map<std::string, phx::Rk4Tune> shapes;
+
+public:
+    bool find(const std::string& key, phx::Rk4Tune& t) {
+        std::lock_guard<std::mutex> lock(mu);
+        const auto it = shapes.find(key);
+        if (it == shapes.end()) return false;
+        t = it->second;
+        return true;
+    }
+    void put(const std::string& key, const phx::Rk4Tune& t) {
+        std::lock_guard<std::mutex> lock(mu);
+        shapes[key] = t;
+    }
+};
+
 /* Autotuner of the fused RK4 launch shape: time each candidate tile height on this
    grid (writing into the spare buffers, so the state is untouched) and keep the
    fastest.  Results are cached per (precision, grid, feature set) for the process.
    PHX_RK4_TY fixes the shape; PHX_AUTOTUNE=0 keeps the default. */
 template <typename real>
 int autotune_rk4(phx_solver* s) {
-    static std::map<std::string, phx::Rk4Tune> cache;
+    static TuneCache cache;
     auto& c = s->cfg;
     if (std::getenv("PHX_RK4_TY")) return PHX_OK;
     if (const char* e = std::getenv("PHX_AUTOTUNE"))
         if (std::atoi(e) == 0) return PHX_OK;
     const std::string key = std::to_string(sizeof(real)) + ":" + std::to_string(c.N_c) + "x" + std::to_string(c.N_r) + ":" +
                             std::to_string(c.use_reservoir) + std::to_string(c.use_pumps) + std::to_string(c.use_potentials);
-    if (auto it = cache.find(key); it != cache.end()) {
-        s->tune = it->second;
-        return PHX_OK;
-    }
+    if (cache.find(key, s->tune)) return PHX_OK;
     hipEvent_t e0, e1;
     PHX_HIP(hipEventCreate(&e0));
     PHX_HIP(hipEventCreate(&e1));
@@ -921,7 +937,7 @@ int autotune_rk4(phx_solver* s) {
     PHX_HIP(hipEventDestroy(e0));
     PHX_HIP(hipEventDestroy(e1));
     s->tune = best_t;
-    cache[key] = best_t;
+    cache.put(key, best_t);
     return PHX_OK;
 }
 
@@ -1142,7 +1158,7 @@ constexpr int kFlowTuneSteps = 40;
 
 template <typename real>
 int autotune_flow(phx_solver* s) {
-    static std::map<std::string, phx::Rk4Tune> cache;
+    static TuneCache cache;
     auto& c = s->cfg;
     s->flow_tune = s->tune;
     if (std::getenv("PHX_RK4_TY")) return PHX_OK;
@@ -1156,10 +1172,7 @@ int autotune_flow(phx_solver* s) {
     const std::string key = std::to_string(sizeof(real)) + ":" + std::to_string(c.N_c) + "x" + std::to_string(c.N_r) + ":" +
                             std::to_string(c.use_reservoir) + std::to_string(c.use_pumps) + std::to_string(c.use_potentials) +
                             std::to_string(c.periodic_x) + std::to_string(c.periodic_y);
-    if (auto it = cache.find(key); it != cache.end()) {
-        s->flow_tune = it->second;
-        return PHX_OK;
-    }
+    if (cache.find(key, s->flow_tune)) return PHX_OK;
     const phx::Rk4Tune one_step = s->tune;
     s->flow_tune.ty = 10; /* a shape the kernel has, for the availability check */
     s->flow_tune.pf = 2;
@@ -1224,7 +1237,7 @@ int autotune_flow(phx_solver* s) {
     }
     s->flow_tune.ty = tys[best % nty];
     s->flow_tune.pf = pfs[best / nty];
-    cache[key] = s->flow_tune;
+    cache.put(key, s->flow_tune);
     return PHX_OK;
 }
 
