@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
     const bool gp_on = RES && a.g_pump, gv_on = a.g_pot != nullptr;
     const rsrc_t d_gp = row_rsrc(gp_on ? a.g_pump + so : nullptr, gp_on ? all_r : 0u);
     const rsrc_t d_gv = row_rsrc(gv_on ? a.g_pot + so : nullptr, gv_on ? all_r : 0u);
-    const RowWrap wrap = make_row_wrap(Nr, kAdjHalo);
+    RowWalk walk = make_row_walk(y0 - kAdjHalo, 1, Nr, kAdjHalo, a.periodic_y);
 
     PhxPhys<real> ph = a.ph;
     ph.mhalf_gamma_c = in_vgpr(ph.mhalf_gamma_c);
@@ -131,9 +131,8 @@ __global__ __launch_bounds__(256) void rk4_adjoint_fused(Rk4AdjArgs<real> a) {
     }
 
     auto load_row = [&](int r, int sl) {
-        bool in;
-        const uint32_t grow = tile_row(y0 - kAdjHalo + r, wrap, a.periodic_y, in); /* wave-uniform */
-        in = in && r < E;                                                         /* rows past the tile read as zero */
+        const bool in = next_row(walk) && r < E; /* rows past the tile read as zero */
+        const uint32_t grow = walk.row;          /* wave-uniform */
         const uint32_t vc = in ? off_c + grow * row_c : kOutOfRange;
         const uint32_t vr = in ? off_r + grow * row_r : kOutOfRange;
         const v2 x = load_cplx<real>(d_x, vc);

@@ -81,13 +81,13 @@ __device__ __forceinline__ void rk4_tile(const Rk4Args<real>& a, int strip, int 
     const rsrc_t w_psi = row_rsrc(a.psi_out, all_c), w_n = row_rsrc(a.n_out, all_r);
     /* the same arrays with no records: output rows past the grid end store through them (dropped) */
     const rsrc_t w_psi_none = row_rsrc(a.psi_out, 0u), w_n_none = row_rsrc(a.n_out, 0u);
-    const RowWrap wrap = make_row_wrap(Nr, kHalo);
     /* tile row r is grid row row0 + rdir * r.  With alt_rows, odd bands stream bottom to top: the 8
        halo rows that two vertically adjacent tiles share are then read by both at the same end of
        their sweeps, close in time, so the second read finds them in L2.  North and south only swap
        places in a sum, so every cell's result is the same either way. */
     const bool up = a.alt_rows && (band & 1);
     const int row0 = up ? y0 + TY + kHalo - 1 : y0 - kHalo, rdir = up ? -1 : 1;
+    RowWalk walk = make_row_walk(row0, rdir, Nr, kHalo, PERY);
 
     constexpr int E = TY + 2 * kHalo;
     real p0r[E], p0i[E], n0[E], pp[E], vv[E];
@@ -105,8 +105,8 @@ __device__ __forceinline__ void rk4_tile(const Rk4Args<real>& a, int strip, int 
     const real kin_x = ph.kin_x, kin_yx = ph.kin_yx;
 
     auto load_row = [&](int r) {
-        bool in;
-        const uint32_t grow = tile_row(row0 + rdir * r, wrap, PERY, in); /* wave-uniform */
+        const bool in = next_row(walk) || PERY;
+        const uint32_t grow = in ? walk.row : 0u; /* wave-uniform */
         const uint32_t sc = grow * row_c, sr = grow * row_r;
         const uint32_t nc = in ? all_c : 0u, nr = in ? all_r : 0u;
         const auto x = load_cplx_s<real, CP>(row_rsrc(a.psi_in, nc), off_c, sc);

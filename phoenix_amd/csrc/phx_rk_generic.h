@@ -92,7 +92,7 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
     rsrc_t d_psi[NC], d_n[NC], d_p[NC], d_v[NC], o_psi[NC], o_n[NC];
     rsrc_t d_f[NC];
     const rsrc_t d_xi = row_rsrc(a.noise, STOCH ? all_c : 0u);
-    const RowWrap wrap = make_row_wrap(Nr, H);
+    RowWalk walk = make_row_walk(y0 - H, 1, Nr, H, a.periodic_y);
 #pragma unroll
     for (int k = 0; k < NC; k++) {
         d_psi[k] = row_rsrc(a.psi_in[k], all_c);
@@ -123,8 +123,8 @@ __device__ __forceinline__ void rk_generic_tile(const RkGenArgs<real>& a, const 
     double err_acc = 0.0, nrm_acc = 0.0;
 
     auto load_row = [&](int r) {
-        bool in;
-        const uint32_t grow = tile_row(y0 - H + r, wrap, a.periodic_y, in); /* wave-uniform */
+        const bool in = next_row(walk);
+        const uint32_t grow = walk.row; /* wave-uniform */
         const uint32_t vc = in ? off_c + grow * row_c : kOutOfRange;
         const uint32_t vr = in ? off_r + grow * row_r : kOutOfRange;
 #pragma unroll

@@ -1,6 +1,6 @@
 /*
- * phx_row_wrap.h -- periodic row index of the streaming kernels, in plain C++ so that it compiles for the
- * host too.
+ * phx_row_wrap.h -- grid rows of a tile's rows in the streaming kernels, in plain C++ so that it compiles for
+ * the host too.
  */
 #pragma once
 #include <stdint.h>
@@ -13,30 +13,33 @@
 
 namespace phx {
 
-/* Periodic row wrap without branches, so that a fully unrolled row loop stays one
-   basic block (a branch there splits it, and DPP moves then no longer fold into the
-   adds that consume them).  With x = g + bias >= 0 and magic = floor((2^32 - 1) / Nr),
-   mulhi(x, magic) is x / Nr or one less for every x < 2^32 and Nr >= 1 (magic is short of 2^32 / Nr by
-   at most one, so the product by at most x / 2^32 < 1), hence one conditional subtraction;
-   g >= -halo, and bias = Nr (Nr >= halo) or Nr * halo keeps x from going negative. */
-struct RowWrap {
-    uint32_t nr, magic, bias;
+/* Walk over the grid rows of consecutive tile rows, upwards (dir 1) or downwards (dir -1), without branches, so that
+   a fully unrolled row loop stays one basic block (a branch there splits it, and DPP moves then no longer fold into
+   the adds that consume them): one add, one compare and one select a row.  A periodic axis turns at its end, whatever
+   its length; beyond a zero boundary the row is out of range (next_row says so) and counts on.  (A quotient by a
+   reciprocal took four scalar operations a row and was wrong for one row and for more than 37837; six made it exact.
+   us per pass with four, six and the walk: FP64 512 x 512 with a pulse, 10 steps, 44.6 / 46.4 / 44.3; FP64 spinor DP45 of
+   134 x 134 1675 / 1740 / 1672; FP32 adjoint of 12 x 185 x 153 1235 / 1246 / 1206.) */
+struct RowWalk {
+    uint32_t row, step, stop, turn, nr;
 };
-PHX_HD RowWrap make_row_wrap(int Nr, int halo) {
-    RowWrap w;
+/* from tile row `first` >= -halo on: next_row moves there first */
+PHX_HD RowWalk make_row_walk(int first, int dir, int Nr, int halo, bool periodic) {
+    RowWalk w;
     w.nr = (uint32_t)Nr;
-    w.magic = 0xFFFFFFFFu / (uint32_t)Nr;
-    w.bias = Nr >= halo ? (uint32_t)Nr : (uint32_t)(Nr * halo);
+    w.step = (uint32_t)dir;
+    const uint32_t before = (uint32_t)(first - dir);
+    const uint32_t bias = Nr > halo ? w.nr : w.nr * (uint32_t)(halo + 1); /* a multiple of Nr past halo */
+    w.row = periodic ? (before + bias) % w.nr : before;
+    w.stop = periodic ? (dir > 0 ? w.nr : 0xFFFFFFFFu) : 0x80000000u; /* the last: never reached */
+    w.turn = dir > 0 ? 0u : w.nr - 1u;
     return w;
 }
-/* Row of tile row g: wrapped into [0, Nr) (for a zero boundary `in` says whether g lies in the grid, the
-   wrapped row is then unused). */
-PHX_HD uint32_t tile_row(int g, const RowWrap& w, int periodic, bool& in) {
-    in = periodic || (g >= 0 && g < (int)w.nr);
-    const uint32_t x = (uint32_t)g + w.bias;
-    const uint32_t r = x - (uint32_t)(((uint64_t)x * w.magic) >> 32) * w.nr; /* in [0, 2 Nr) */
-    const uint32_t less = r - w.nr;                                          /* past every r where r < Nr */
-    return r < less ? r : less;
+/* the next row; whether it lies in the grid */
+PHX_HD bool next_row(RowWalk& w) {
+    const uint32_t t = w.row + w.step;
+    w.row = t == w.stop ? w.turn : t;
+    return w.row < w.nr;
 }
 
 } // namespace phx
