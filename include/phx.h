@@ -84,8 +84,9 @@ typedef struct {
                                    stage by stage with the K's in HBM, or, for RK4 under sources of at most two
                                    temporal groups, by the fused chain kernel */
     int64_t multi_step_steps;   /* fixed RK4 steps taken by the multi-step kernel (phx_step and
-                                   phx_run_interval run constant-source stretches that way, up to 500 steps
-                                   per launch; PHX_RK4_FLOW=0: never) */
+                                   phx_run_interval run constant-source stretches of 10 steps and more that
+                                   way on grids from about 600 x 600 to where its blocks no longer fit the device
+                                   at once, up to 500 steps per launch; PHX_RK4_FLOW=0: never) */
     int64_t multi_step_launches; /* its launches */
     int32_t complex_reservoir;  /* 1: the reservoir fields are complex ({re, im} per cell: PHX_N_PLUS /
                                    PHX_N_MINUS take 2 N_c N_r reals), as the reference's n becomes under
@@ -109,11 +110,13 @@ int phx_initialize(phx_solver* s);
 
 /* Run up to n_steps iterate() calls; stops early when t >= t_max.
    *n_done receives the number of accepted steps taken.  Stretches of fixed RK4 steps of the
-   scalar model with constant sources (no filter application or t_max inside) go to the device
-   as one launch of up to 500 steps in which every tile waits for its neighbours (bitwise the
-   same result as step by step); should
-   such a wait ever exceed ~2 s, the next phx_sync / phx_get_field returns PHX_ERR_HIP and the
-   state is undefined.  PHX_RK4_FLOW=0 launches step by step instead.
+   scalar model with constant sources (no filter application or t_max inside) of 10 steps and more
+   go to the device as one launch of up to 500 steps in which every tile waits for its neighbours
+   (bitwise the same result as step by step) on grids from about 600 x 600 to where that kernel's
+   blocks no longer fit the device at once; should such a wait ever exceed ~2 s, the next phx_sync /
+   phx_get_field returns PHX_ERR_HIP and the state is undefined.  Shorter stretches and other grids are
+   launched step by step, and replayed from a captured graph once they repeat.  PHX_RK4_FLOW=0 launches
+   step by step everywhere.
    Replaces: Solver::iterate (solver.cu:22-70) in the main loop (main.cu:80-117). */
 int phx_step(phx_solver* s, int64_t n_steps, int64_t* n_done);
 
@@ -291,7 +294,8 @@ int phx_ensemble_get_field(phx_ensemble* e, int inst, int field, void* host, siz
 int phx_ensemble_device_ptr(phx_ensemble* e, int inst, int field, void** dptr);
 
 /* Output rows per wavefront tile of the batched kernel: 8, 10, 12, 16 or 20.
-   Without this call the first step picks it by the number of tiles. */
+   Without this call the first step picks it by the number of tiles (small ensembles: 4 rows, which
+   cannot be asked for). */
 int phx_ensemble_set_tile_rows(phx_ensemble* e, int ty);
 
 /* n_steps RK4 steps of every instance.  graph_steps >= 2 captures that many

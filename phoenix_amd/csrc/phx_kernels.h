@@ -51,8 +51,8 @@ inline int rk4_alt_rows() {
 
 /* Launch shape of the fused RK4 kernel.
    ty: output rows per wavefront tile (2, 4, 8, 10, 12, 16, 20, 24);
-   ew, pf: kept for the tuning interface; the kernel uses DPP wave shifts for
-   east/west and loads rows 2 ahead of first use. */
+   pf: rows loaded ahead of first use (2; 3, 4, 6 and 8 exist for the pumped reservoir model with dx == dy);
+   ew: kept for the tuning interface (the kernel uses DPP wave shifts for east/west). */
 struct Rk4Tune {
     int ty = 16, ew = 1, pf = 2;
 };
@@ -229,7 +229,7 @@ hipError_t launch_rk_tab6f(const RkGenArgs<real>& a, RkTableau tab, hipStream_t 
 template <typename real>
 hipError_t launch_rk4_generic(const RkGenArgs<real>& a, hipStream_t s);
 int rk4_generic_tile_rows(int Nc, int Nr);
-/* adaptive DP45, TE-TM, FP32, tile height 32 (phx_rk_dp45t.hip) */
+/* adaptive DP45, TE-TM, FP32, tile heights 28, 32 and 42 (phx_rk_dp45t.hip) */
 hipError_t launch_dp45_tetm_tall(const RkGenArgs<float>& a, int ty, hipStream_t s);
 /* ... the others and the shorter tiles (phx_rk_dp45.hip) */
 template <typename real>

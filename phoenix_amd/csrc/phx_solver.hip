@@ -1080,8 +1080,15 @@ phx::Rk4Args<real> rk4_args(phx_solver* s, void* psi_in, void* n_in, void* psi_o
    step by step (from a graph once they repeat): their kernels leave room for those of other handles.  us per run,
    one handle alone / three in turn, launches and multi-step: 600^2 FP32 50 steps 262 / 130 and 217 / 128, FP64
    328 / 206 and 284 / 201; 1024^2 10 steps FP32 87 / 54 and 78 / 65, FP64 133 / 95 and 109 / 107; 50 steps FP32
-   415 / 266 and 349 / 310, FP64 636 / 474 and 507 / 518; below the line 512^2 FP32 with a potential, 68 steps:
-   365 / 175 and 362 / 185 to 271. */
+   415 / 266 and 349 / 310, FP64 636 / 474 and 507 / 518.  Below the line, 50 steps (launches: in a handle's first 400
+   steps, and from its graph afterwards; the cooperative form that the multi-step kernel had before took 241 / 223 and
+   285 / 260 at 400^2):
+     400^2 FP32   271 / 133, 214 / 89    multi-step 196 / 92      FP64 300 / 145, 256 / 123    255 / 131
+     512^2 FP32   302 / 143, 255 / 115              231 / 114     FP64 345 / 197, 319 / 169    287 / 145
+     512^2 + V    320 / 143, 278 / 126              254 / 128          360 / 213, 330 / 182    333 / 161
+   A handle alone pays for the launches until its graph is there, 6 to 17 % of a run against the cooperative form; with
+   others, and at 400^2 alone from the graph, runs are shorter than they were.  The multi-step kernel without its
+   cooperative start would pay at 512^2 too; 256^2 FP64 is 199 / 86 from the graph and 241 / 104. */
 constexpr int64_t kFlowMinSteps = 10, kFlowMaxSteps = 500;
 
 bool flow_wanted(phx_solver* s, int64_t n) {
