@@ -11,41 +11,53 @@
 namespace phx {
 
 /* ------------------------------------------------------------------ transforms in registers */
-/* cos and sin of 2 pi k / R at compile time: Taylor series after reduction to |x| <= pi / 4 */
-inline constexpr double kPi = 3.14159265358979323846264338327950288;
-constexpr double taylor_sin(double x) {
-    double t = x, s = 0;
-    for (int n = 1; n < 24; n += 2) {
-        s += t;
-        t *= -x * x / ((n + 1) * (n + 2));
-    }
-    return s;
-}
-constexpr double taylor_cos(double x) {
-    double t = 1, s = 0;
-    for (int n = 0; n < 24; n += 2) {
-        s += t;
-        t *= -x * x / ((n + 1) * (n + 2));
-    }
-    return s;
-}
-/* cos(2 pi k / R) for 0 <= k: eighths of a turn, exact reduction in integers */
-constexpr double cos_turn(int k, int R) {
+/* cos and sin of 2 pi k / R to more digits than a double holds, k / R in lowest terms below one half; the compiler
+   rounds them once (a Taylor series in double was off by up to 1.6 units: the rotations by an eighth of a turn shrank
+   what they turned by 0.8 units of 2^-53, and with it a split-step run) */
+inline constexpr struct {
+    int k, R;
+    double c, s;
+} kTurns[] = {
+    {1, 3, -0.500000000000000000000, 0.866025403784438646764},  {1, 5, 0.309016994374947424102, 0.951056516295153572116},
+    {2, 5, -0.809016994374947424102, 0.587785252292473129169},  {1, 7, 0.623489801858733530525, 0.781831482468029808708},
+    {2, 7, -0.222520933956314404289, 0.974927912181823607018},  {3, 7, -0.900968867902419126236, 0.433883739117558120476},
+    {1, 8, 0.707106781186547524401, 0.707106781186547524401},   {3, 8, -0.707106781186547524401, 0.707106781186547524401},
+    {1, 9, 0.766044443118978035202, 0.642787609686539326323},   {2, 9, 0.173648177666930348852, 0.984807753012208059367},
+    {4, 9, -0.939692620785908384054, 0.342020143325668733044},  {1, 10, 0.809016994374947424102, 0.587785252292473129169},
+    {3, 10, -0.309016994374947424102, 0.951056516295153572116}, {1, 11, 0.841253532831181168862, 0.540640817455597582108},
+    {2, 11, 0.415415013001886425529, 0.909631995354518371412},  {3, 11, -0.142314838273285140444, 0.989821441880932732376},
+    {4, 11, -0.654860733945285064057, 0.755749574354258283774}, {5, 11, -0.959492973614497389890, 0.281732556841429697711},
+    {1, 13, 0.885456025653209895900, 0.464723172043768545656},  {2, 13, 0.568064746731155802512, 0.822983865893656394580},
+    {3, 13, 0.120536680255323053349, 0.992708874098053992801},  {4, 13, -0.354604887042535625970, 0.935016242685414823440},
+    {5, 13, -0.748510748171101098635, 0.663122658240795202377}, {6, 13, -0.970941817426052027157, 0.239315664287557767149},
+    {1, 16, 0.923879532511286756128, 0.382683432365089771728},  {3, 16, 0.382683432365089771728, 0.923879532511286756128},
+    {5, 16, -0.382683432365089771728, 0.923879532511286756128}, {7, 16, -0.923879532511286756128, 0.382683432365089771728},
+};
+struct Turn {
+    double c, s;
+};
+/* of k Rths of a turn, R one of the radices */
+constexpr Turn turn(int k, int R) {
     k %= R;
-    if (2 * k > R) k = R - k;                        /* cos is even: k / R <= 1/2 */
-    if (4 * k > R) return -cos_turn(R - 2 * k, 2 * R); /* cos(pi - x) = -cos x */
-    if (8 * k > R) return taylor_sin(kPi * (R - 4 * k) / (2.0 * R)); /* sin(pi/2 - x) */
-    return taylor_cos(2.0 * kPi * k / R);
+    if (k == 0) return {1.0, 0.0};
+    if (2 * k == R) return {-1.0, 0.0};
+    if (2 * k > R) {
+        const Turn t = turn(R - k, R);
+        return {t.c, -t.s};
+    }
+    if (4 * k == R) return {0.0, 1.0};
+    for (const auto& t : kTurns)
+        if (k * t.R == t.k * R) return {t.c, t.s};
+    return {0.0, 0.0}; /* not reached */
 }
-constexpr double sin_turn(int k, int R) { return cos_turn(4 * k + 3 * R, 4 * R); } /* sin x = cos(x - pi/2) */
 
 template <int R>
 struct Roots {
     double c[R] = {}, s[R] = {};
     constexpr Roots() {
         for (int k = 0; k < R; k++) {
-            c[k] = cos_turn(k, R);
-            s[k] = sin_turn(k, R);
+            c[k] = turn(k, R).c;
+            s[k] = turn(k, R).s;
         }
     }
 };

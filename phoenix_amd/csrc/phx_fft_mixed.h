@@ -45,7 +45,12 @@ struct FftAxis {
 bool fft_mixed_supported(int N, size_t real_size);
 /* plan of an axis (no device work) and the table it needs, in double precision */
 FftAxis fft_axis(int N);
-std::vector<std::complex<double>> fft_axis_table(const FftAxis& a);
+std::vector<std::complex<double>> fft_axis_table(const FftAxis& a, size_t real_size);
+/* What a transform forth and back along an axis multiplies amplitudes by, because the constants of its passes are
+   rounded (0.4 units of the roundoff a transform and more, always the same): 1 for lengths whose table makes up for it
+   (Bluestein's) and for powers of two, which other kernels take.  Rows run the radices in one order, columns turn them
+   round for the way back. */
+double fft_axis_gain(const FftAxis& a, bool columns, size_t real_size);
 
 enum { kFftFilter = 0, kFftPropagate = 1, kFftForward = 2 };
 

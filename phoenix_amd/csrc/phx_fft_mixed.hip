@@ -20,6 +20,7 @@
  */
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "phx_fft_engine.h"
 
@@ -213,23 +214,119 @@ std::complex<real> root(long long k, long long n) {
 
 /* Bluestein's tables are made in the host's long double (64-bit mantissa on x86) and rounded once: the chirp's
    transform in double was off by several units, as much as the FP64 transform itself (a filter of 138 x 158,
-   relative L2 in units of 2^-53: 12.0 with tables from double, 5.9; direct sums 11.2) */
+   relative L2 in units of 2^-53: 12.0 with tables from double, 5.9 so, 4.3 with hat made up for the gain below and the
+   butterflies' constants rounded once; direct sums 11.2) */
 using cld = std::complex<long double>;
 std::complex<double> rounded(cld z) { return {(double)z.real(), (double)z.imag()}; }
 
-/* forward DFT of every step-th value from x, by decimation in time over the prime factors of the length n;
-   w holds the roots of the whole transform, of n * step points */
-std::vector<cld> host_fft(const cld* x, size_t n, size_t step, const std::vector<cld>& w) {
-    if (n == 1) return {x[0]};
-    size_t p = 2;
-    while (n % p) p++;
-    const size_t m = n / p;
-    std::vector<cld> out(n);
-    for (size_t j = 0; j < p; j++) {
-        const auto sub = host_fft(x + j * step, m, step * p, w);
-        for (size_t k = 0; k < n; k++) out[k] += w[j * k % n * step] * sub[k % m];
-    }
+/* ---- the transforms on the host, in long double, with the constants rounded to `real` (long double: exact) */
+struct Lc {
+    long double r, i;
+};
+inline Lc operator*(Lc a, Lc b) { return {a.r * b.r - a.i * b.i, a.r * b.i + a.i * b.r}; } /* (std::complex looks for NaN) */
+inline Lc conj(Lc a) { return {a.r, -a.i}; }
+using Lcs = std::vector<Lc>;
+
+template <typename real>
+Lc to_real(cld z) {
+    if constexpr (std::is_same<real, long double>::value) return {z.real(), z.imag()};
+    return {(long double)(real)(double)z.real(), (long double)(real)(double)z.imag()};
+}
+template <typename real>
+Lcs to_real(const std::vector<cld>& v) {
+    Lcs out;
+    for (const cld& z : v) out.push_back(to_real<real>(z));
     return out;
+}
+template <typename real>
+struct HostConstants {
+    Lc w[17][16]; /* e^{-2 pi i k / R} */
+    HostConstants() {
+        for (int R : kRadices)
+            for (int k = 0; k < R; k++) {
+                const Turn t = turn(k, R);
+                w[R][k] = std::is_same<real, long double>::value ? to_real<real>(root<long double>(k, R)) : Lc{(real)t.c, -(long double)(real)t.s};
+            }
+    }
+};
+
+/* dft() of phx_fft_engine.h: R values `step` apart, in place */
+template <typename real>
+void host_dft(const HostConstants<real>& h, int R, Lc* x, int step) {
+    const int R1 = R == 4 ? R : first_factor(R), R2 = R / R1;
+    Lc y[16];
+    if (R1 == R) {
+        for (int j = 0; j < R; j++) {
+            Lc t{0, 0};
+            for (int k = 0; k < R; k++) {
+                const Lc z = x[k * step] * h.w[R][j * k % R];
+                t = {t.r + z.r, t.i + z.i};
+            }
+            y[j] = t;
+        }
+        for (int j = 0; j < R; j++) x[j * step] = y[j];
+        return;
+    }
+    for (int n2 = 0; n2 < R2; n2++) { /* the values R2 n1 + n2, then their transform k1 there */
+        host_dft(h, R1, x + n2 * step, R2 * step);
+        for (int k1 = 1; k1 < R1; k1++) x[(R2 * k1 + n2) * step] = x[(R2 * k1 + n2) * step] * h.w[R][n2 * k1 % R];
+    }
+    for (int k1 = 0; k1 < R1; k1++) {
+        host_dft(h, R2, x + R2 * k1 * step, step);
+        for (int k2 = 0; k2 < R2; k2++) y[k1 + R1 * k2] = x[(R2 * k1 + k2) * step];
+    }
+    for (int k = 0; k < R; k++) x[k * step] = y[k];
+}
+/* transform(); w: the roots of len points, rounded */
+template <typename real>
+Lcs host_transform(const HostConstants<real>& h, const FftPlan& p, Lcs x, const Lcs& w) {
+    Lcs y(p.len);
+    for (int i = 0; i < p.passes; i++) {
+        const int R = p.radix[i], s = p.s[i], nb = p.len / R;
+        const bool last = i == p.passes - 1;
+        for (int b = 0; b < nb; b++) {
+            const int pp = b / s, q = b - pp * s;
+            Lc t[16];
+            for (int j = 0; j < R; j++) t[j] = x[b + j * nb];
+            host_dft(h, R, t, 1);
+            for (int j = 0; j < R; j++) y[q + s * (R * pp + j)] = last ? t[j] : t[j] * w[j * pp * s];
+        }
+        std::swap(x, y);
+    }
+    return x;
+}
+/* Bluestein's transform of N values from its tables; the sign of the second transform is turned by conjugation */
+template <typename real>
+Lcs host_bluestein(const HostConstants<real>& h, const FftAxis& a, const Lcs& x, const Lcs& w, const Lcs& chirp, const Lcs& hat) {
+    Lcs y(a.M, Lc{0, 0});
+    for (int j = 0; j < a.N; j++) y[j] = x[j] * chirp[j];
+    y = host_transform(h, a.fwd, y, w);
+    for (int k = 0; k < a.M; k++) y[k] = conj(y[k] * hat[k]);
+    y = host_transform(h, a.inv, y, w);
+    y.resize(a.N);
+    for (int j = 0; j < a.N; j++) y[j] = conj(y[j]) * chirp[j];
+    return y;
+}
+/* mean gain of `rounded` against `exact`, two linear maps of n values, over 512 or more fixed pseudo-random ones: known
+   to a few hundredths of what the rounding of one constant does */
+template <class F, class G>
+long double mean_gain(int n, F rounded, G exact) {
+    uint32_t state = 12345;
+    auto next = [&] {
+        state = state * 1664525u + 1013904223u;
+        return (long double)(int32_t)state / 2147483648.0L;
+    };
+    long double num = 0, den = 0;
+    for (int done = 0; done < 512; done += n) {
+        Lcs x(n);
+        for (Lc& z : x) {
+            z.r = next();
+            z.i = next();
+        }
+        const Lcs r = rounded(x), e = exact(x);
+        for (int k = 0; k < n; k++) num += e[k].r * r[k].r + e[k].i * r[k].i, den += e[k].r * e[k].r + e[k].i * e[k].i;
+    }
+    return num / den;
 }
 
 /* the next power of two from 2 N - 1, or the length 2^a 3^b 5^c below it with the least cost where that
@@ -268,20 +365,63 @@ FftAxis fft_axis(int N) {
     return a;
 }
 
-std::vector<std::complex<double>> fft_axis_table(const FftAxis& a) {
+template <typename real>
+static std::vector<std::complex<double>> axis_table(const FftAxis& a) {
     std::vector<std::complex<double>> t;
     for (int k = 0; k < a.N; k++) t.push_back(root<double>(k, a.N));
-    if (!a.M) return t;
-    std::vector<cld> w(a.M), b(a.M);
-    for (int k = 0; k < a.M; k++) t.push_back(rounded(w[k] = root<long double>(k, a.M)));
+    if (!a.M || !a.fwd.passes) return t;
+    const HostConstants<real> h;
+    const HostConstants<long double> he;
+    std::vector<cld> w(a.M), chirp(a.N);
+    for (int k = 0; k < a.M; k++) w[k] = root<long double>(k, a.M);
+    const Lcs we = to_real<long double>(w), wr = to_real<real>(w);
+    Lcs b(a.M, Lc{0, 0});
     for (long long j = 0; j < a.N; j++) {
-        const cld c = root<long double>(j * j % (2 * a.N), 2 * a.N);
-        t.push_back(rounded(c));
-        b[j] = std::conj(c);
-        if (j) b[a.M - j] = std::conj(c);
+        const cld c = chirp[j] = root<long double>(j * j % (2 * a.N), 2 * a.N);
+        b[j] = conj(to_real<long double>(c));
+        if (j) b[a.M - j] = b[j];
     }
-    for (const auto& z : host_fft(b.data(), a.M, 1, w)) t.push_back(rounded(z / (long double)a.M));
+    const Lcs hate = [&] {
+        Lcs y = host_transform(he, a.fwd, b, we);
+        for (Lc& z : y) z = {z.r / a.M, z.i / a.M};
+        return y;
+    }();
+    std::vector<cld> hat;
+    for (const Lc& z : hate) hat.emplace_back(z.r, z.i);
+    /* the rounded constants of the two transforms shrink or stretch what passes through by 0.4 to 1 units, the same way
+       every time: hat makes up for it (a split-step run of 106 x 106 FP32 lost 2.5 units of amplitude a step, 76 x 76
+       3.2, direct sums less than 0.5; now 0.03 and -0.7) */
+    const Lcs cr = to_real<real>(chirp), hr = to_real<real>(hat), ce = to_real<long double>(chirp);
+    const long double gain = mean_gain(
+        a.N, [&](const Lcs& x) { return host_bluestein(h, a, x, wr, cr, hr); }, [&](const Lcs& x) { return host_bluestein(he, a, x, we, ce, hate); });
+    for (const auto& z : w) t.push_back(rounded(z));
+    for (const auto& z : chirp) t.push_back(rounded(z));
+    for (const auto& z : hat) t.push_back(rounded(z / gain));
     return t;
+}
+
+std::vector<std::complex<double>> fft_axis_table(const FftAxis& a, size_t real_size) {
+    return real_size == sizeof(float) ? axis_table<float>(a) : axis_table<double>(a);
+}
+
+template <typename real>
+static long double plan_gain(const FftPlan& p) {
+    const HostConstants<real> h;
+    const HostConstants<long double> he;
+    Lcs we, wr;
+    for (int k = 0; k < p.len; k++) {
+        const std::complex<double> z = root<double>(k, p.len); /* as the table holds it */
+        we.push_back(to_real<long double>(root<long double>(k, p.len)));
+        wr.push_back(to_real<real>(cld(z.real(), z.imag())));
+    }
+    return mean_gain(
+        p.len, [&](const Lcs& x) { return host_transform(h, p, x, wr); }, [&](const Lcs& x) { return host_transform(he, p, x, we); });
+}
+
+double fft_axis_gain(const FftAxis& a, bool columns, size_t real_size) {
+    if (a.M || !a.fwd.passes || largest_prime(a.N) <= 2) return 1.0;
+    auto gain = [&](const FftPlan& p) { return real_size == sizeof(float) ? plan_gain<float>(p) : plan_gain<double>(p); };
+    return (double)(gain(a.fwd) * gain(columns ? a.inv : a.fwd));
 }
 
 template <typename real>

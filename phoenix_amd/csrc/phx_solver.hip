@@ -87,6 +87,7 @@ struct phx_solver {
     void* ssfm_rowf[2] = {nullptr, nullptr};
     void* ssfm_colf[2] = {nullptr, nullptr};
     double ssfm_dt = -1.0;                    /* dt the factors were made for */
+    double ssfm_gain = 1.0;                   /* fft_axis_gain of both axes, which the factors undo */
     int max_rejections = 10000;
     double last_error = 0; /* E of the last adaptive attempt */
     /* time bookkeeping in the build's precision (system_parameters.hpp:33) */
@@ -306,12 +307,14 @@ int initialize_t(phx_solver* s) {
         }
     }
     if (c.use_fft_mask || s->ssfm || s->spec[0]) {
+        std::vector<std::complex<double>> table;
         for (phx::FftAxis* ax : {&s->fft_c, &s->fft_r}) {
             *ax = phx::fft_axis(ax == &s->fft_c ? c.N_c : c.N_r);
-            const auto table = phx::fft_axis_table(*ax);
+            if (ax == &s->fft_c || c.N_r != c.N_c) table = phx::fft_axis_table(*ax, sizeof(real));
             if (int r = dev_alloc(s, &ax->table, 2 * table.size() * sizeof(real))) return r;
             if (int r = upload_complex<real>(s, ax->table, table)) return r;
         }
+        if (s->ssfm) s->ssfm_gain = phx::fft_axis_gain(s->fft_c, false, sizeof(real)) * phx::fft_axis_gain(s->fft_r, true, sizeof(real));
     }
 
     /* initial states (solver_initialization.cu:55-98) */
@@ -696,7 +699,7 @@ int ssfm_tables(phx_solver* s) {
         std::vector<std::complex<double>> rowf(c.N_r), colf(c.N_c);
         for (int r = 0; r < c.N_r; r++) {
             const double ky = 2.0 * 3.1415926535 * (double)(r <= c.N_r / 2 ? r : r - c.N_r) / c.L_y;
-            rowf[r] = std::polar(1.0, (w + 1) * (-lin * ky * ky * dt / 2.0)) / ((double)c.N_c * (double)c.N_r);
+            rowf[r] = std::polar(1.0, (w + 1) * (-lin * ky * ky * dt / 2.0)) / ((double)c.N_c * (double)c.N_r * s->ssfm_gain);
         }
         for (int col = 0; col < c.N_c; col++) {
             const double kx = 2.0 * 3.1415926535 * (double)(col <= c.N_c / 2 ? col : col - c.N_c) / c.L_x;
