@@ -20,7 +20,6 @@
  */
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 #include "phx_fft_engine.h"
 
@@ -206,60 +205,59 @@ FftPlan make_plan(int len, const int* radix, int passes) {
     return p;
 }
 
-/* e^{-2 pi i k / n}, k reduced exactly */
-template <typename real>
-std::complex<real> root(long long k, long long n) {
-    return std::polar((real)1, (real)-2 * (real)3.14159265358979323846264338327950288L * (real)(k % n) / (real)n);
-}
-
-/* Bluestein's tables are made in the host's long double (64-bit mantissa on x86) and rounded once: the chirp's
-   transform in double was off by several units, as much as the FP64 transform itself (a filter of 138 x 158,
-   relative L2 in units of 2^-53: 12.0 with tables from double, 5.9 so, 4.3 with hat made up for the gain below and the
-   butterflies' constants rounded once; direct sums 11.2) */
-using cld = std::complex<long double>;
-std::complex<double> rounded(cld z) { return {(double)z.real(), (double)z.imag()}; }
-
-/* ---- the transforms on the host, in long double, with the constants rounded to `real` (long double: exact) */
-struct Lc {
-    long double r, i;
+/* ---- tables, and the transforms on the host, in arithmetic of type T: double for FP32, long double (64-bit mantissa
+   on x86) for FP64, so that rounding to the kernels' precision is the only error that counts */
+template <class T>
+struct Hc {
+    T r, i;
 };
-inline Lc operator*(Lc a, Lc b) { return {a.r * b.r - a.i * b.i, a.r * b.i + a.i * b.r}; } /* (std::complex looks for NaN) */
-inline Lc conj(Lc a) { return {a.r, -a.i}; }
-using Lcs = std::vector<Lc>;
+template <class T>
+inline Hc<T> operator*(Hc<T> a, Hc<T> b) { return {a.r * b.r - a.i * b.i, a.r * b.i + a.i * b.r}; } /* (std::complex looks for NaN) */
+template <class T>
+inline Hc<T> conj(Hc<T> a) { return {a.r, -a.i}; }
+template <class T>
+using Hcs = std::vector<Hc<T>>;
 
-template <typename real>
-Lc to_real(cld z) {
-    if constexpr (std::is_same<real, long double>::value) return {z.real(), z.imag()};
-    return {(long double)(real)(double)z.real(), (long double)(real)(double)z.imag()};
+/* e^{-2 pi i k / n}, k reduced exactly */
+template <class T>
+Hc<T> root(long long k, long long n) {
+    const std::complex<T> z = std::polar((T)1, (T)-2 * (T)3.14159265358979323846264338327950288L * (T)(k % n) / (T)n);
+    return {z.real(), z.imag()};
 }
-template <typename real>
-Lcs to_real(const std::vector<cld>& v) {
-    Lcs out;
-    for (const cld& z : v) out.push_back(to_real<real>(z));
-    return out;
+template <class T>
+Hc<T> rounded(Hc<T> z, size_t real_size) { /* to the kernels' precision */
+    if (real_size == sizeof(float)) return {(T)(float)z.r, (T)(float)z.i};
+    return {(T)(double)z.r, (T)(double)z.i};
 }
-template <typename real>
+template <class T>
+Hcs<T> rounded(Hcs<T> v, size_t real_size) {
+    for (Hc<T>& z : v) z = rounded(z, real_size);
+    return v;
+}
+
+/* the constants of the butterflies: exact (real_size 0) or as the kernels have them */
+template <class T>
 struct HostConstants {
-    Lc w[17][16]; /* e^{-2 pi i k / R} */
-    HostConstants() {
+    Hc<T> w[17][16]; /* e^{-2 pi i k / R} */
+    explicit HostConstants(size_t real_size) {
         for (int R : kRadices)
             for (int k = 0; k < R; k++) {
                 const Turn t = turn(k, R);
-                w[R][k] = std::is_same<real, long double>::value ? to_real<real>(root<long double>(k, R)) : Lc{(real)t.c, -(long double)(real)t.s};
+                w[R][k] = real_size ? rounded(Hc<T>{(T)t.c, (T)-t.s}, real_size) : root<T>(k, R);
             }
     }
 };
 
 /* dft() of phx_fft_engine.h: R values `step` apart, in place */
-template <typename real>
-void host_dft(const HostConstants<real>& h, int R, Lc* x, int step) {
+template <class T>
+void host_dft(const HostConstants<T>& h, int R, Hc<T>* x, int step) {
     const int R1 = R == 4 ? R : first_factor(R), R2 = R / R1;
-    Lc y[16];
+    Hc<T> y[16];
     if (R1 == R) {
         for (int j = 0; j < R; j++) {
-            Lc t{0, 0};
+            Hc<T> t{0, 0};
             for (int k = 0; k < R; k++) {
-                const Lc z = x[k * step] * h.w[R][j * k % R];
+                const Hc<T> z = x[k * step] * h.w[R][j * k % R];
                 t = {t.r + z.r, t.i + z.i};
             }
             y[j] = t;
@@ -277,16 +275,16 @@ void host_dft(const HostConstants<real>& h, int R, Lc* x, int step) {
     }
     for (int k = 0; k < R; k++) x[k * step] = y[k];
 }
-/* transform(); w: the roots of len points, rounded */
-template <typename real>
-Lcs host_transform(const HostConstants<real>& h, const FftPlan& p, Lcs x, const Lcs& w) {
-    Lcs y(p.len);
+/* transform(); w: the roots of len points */
+template <class T>
+Hcs<T> host_transform(const HostConstants<T>& h, const FftPlan& p, Hcs<T> x, const Hcs<T>& w) {
+    Hcs<T> y(p.len);
     for (int i = 0; i < p.passes; i++) {
         const int R = p.radix[i], s = p.s[i], nb = p.len / R;
         const bool last = i == p.passes - 1;
         for (int b = 0; b < nb; b++) {
             const int pp = b / s, q = b - pp * s;
-            Lc t[16];
+            Hc<T> t[16];
             for (int j = 0; j < R; j++) t[j] = x[b + j * nb];
             host_dft(h, R, t, 1);
             for (int j = 0; j < R; j++) y[q + s * (R * pp + j)] = last ? t[j] : t[j] * w[j * pp * s];
@@ -296,9 +294,9 @@ Lcs host_transform(const HostConstants<real>& h, const FftPlan& p, Lcs x, const 
     return x;
 }
 /* Bluestein's transform of N values from its tables; the sign of the second transform is turned by conjugation */
-template <typename real>
-Lcs host_bluestein(const HostConstants<real>& h, const FftAxis& a, const Lcs& x, const Lcs& w, const Lcs& chirp, const Lcs& hat) {
-    Lcs y(a.M, Lc{0, 0});
+template <class T>
+Hcs<T> host_bluestein(const HostConstants<T>& h, const FftAxis& a, const Hcs<T>& x, const Hcs<T>& w, const Hcs<T>& chirp, const Hcs<T>& hat) {
+    Hcs<T> y(a.M, Hc<T>{0, 0});
     for (int j = 0; j < a.N; j++) y[j] = x[j] * chirp[j];
     y = host_transform(h, a.fwd, y, w);
     for (int k = 0; k < a.M; k++) y[k] = conj(y[k] * hat[k]);
@@ -307,23 +305,23 @@ Lcs host_bluestein(const HostConstants<real>& h, const FftAxis& a, const Lcs& x,
     for (int j = 0; j < a.N; j++) y[j] = conj(y[j]) * chirp[j];
     return y;
 }
-/* mean gain of `rounded` against `exact`, two linear maps of n values, over 512 or more fixed pseudo-random ones: known
+/* mean gain of `kernel` against `exact`, two linear maps of n values, over 512 or more fixed pseudo-random ones: known
    to a few hundredths of what the rounding of one constant does */
-template <class F, class G>
-long double mean_gain(int n, F rounded, G exact) {
+template <class T, class F, class G>
+T mean_gain(int n, F kernel, G exact) {
     uint32_t state = 12345;
     auto next = [&] {
         state = state * 1664525u + 1013904223u;
-        return (long double)(int32_t)state / 2147483648.0L;
+        return (T)(int32_t)state / (T)2147483648.0;
     };
-    long double num = 0, den = 0;
+    T num = 0, den = 0;
     for (int done = 0; done < 512; done += n) {
-        Lcs x(n);
-        for (Lc& z : x) {
+        Hcs<T> x(n);
+        for (Hc<T>& z : x) {
             z.r = next();
             z.i = next();
         }
-        const Lcs r = rounded(x), e = exact(x);
+        const Hcs<T> r = kernel(x), e = exact(x);
         for (int k = 0; k < n; k++) num += e[k].r * r[k].r + e[k].i * r[k].i, den += e[k].r * e[k].r + e[k].i * e[k].i;
     }
     return num / den;
@@ -365,63 +363,60 @@ FftAxis fft_axis(int N) {
     return a;
 }
 
-template <typename real>
-static std::vector<std::complex<double>> axis_table(const FftAxis& a) {
+/* Bluestein's tables are rounded once: the chirp's transform in double was off by several units, as much as the FP64
+   transform itself (a filter of 138 x 158, relative L2 in units of 2^-53: 12.0 with tables from double, 5.9 so, 4.3
+   with hat made up for the gain below and the butterflies' constants rounded once; direct sums 11.2) */
+template <class T>
+static std::vector<std::complex<double>> axis_table(const FftAxis& a, size_t real_size) {
     std::vector<std::complex<double>> t;
-    for (int k = 0; k < a.N; k++) t.push_back(root<double>(k, a.N));
+    auto put = [&](auto z) { t.emplace_back((double)z.r, (double)z.i); };
+    for (int k = 0; k < a.N; k++) put(root<double>(k, a.N));
     if (!a.M || !a.fwd.passes) return t;
-    const HostConstants<real> h;
-    const HostConstants<long double> he;
-    std::vector<cld> w(a.M), chirp(a.N);
-    for (int k = 0; k < a.M; k++) w[k] = root<long double>(k, a.M);
-    const Lcs we = to_real<long double>(w), wr = to_real<real>(w);
-    Lcs b(a.M, Lc{0, 0});
+    const HostConstants<T> exact(0), kernel(real_size);
+    Hcs<T> w(a.M), chirp(a.N), b(a.M, Hc<T>{0, 0});
+    for (int k = 0; k < a.M; k++) w[k] = root<T>(k, a.M);
     for (long long j = 0; j < a.N; j++) {
-        const cld c = chirp[j] = root<long double>(j * j % (2 * a.N), 2 * a.N);
-        b[j] = conj(to_real<long double>(c));
+        chirp[j] = root<T>(j * j % (2 * a.N), 2 * a.N);
+        b[j] = conj(chirp[j]);
         if (j) b[a.M - j] = b[j];
     }
-    const Lcs hate = [&] {
-        Lcs y = host_transform(he, a.fwd, b, we);
-        for (Lc& z : y) z = {z.r / a.M, z.i / a.M};
-        return y;
-    }();
-    std::vector<cld> hat;
-    for (const Lc& z : hate) hat.emplace_back(z.r, z.i);
+    Hcs<T> hat = host_transform(exact, a.fwd, b, w);
+    for (Hc<T>& z : hat) z = {z.r / a.M, z.i / a.M};
     /* the rounded constants of the two transforms shrink or stretch what passes through by 0.4 to 1 units, the same way
        every time: hat makes up for it (a split-step run of 106 x 106 FP32 lost 2.5 units of amplitude a step, 76 x 76
        3.2, direct sums less than 0.5; now 0.03 and -0.7) */
-    const Lcs cr = to_real<real>(chirp), hr = to_real<real>(hat), ce = to_real<long double>(chirp);
-    const long double gain = mean_gain(
-        a.N, [&](const Lcs& x) { return host_bluestein(h, a, x, wr, cr, hr); }, [&](const Lcs& x) { return host_bluestein(he, a, x, we, ce, hate); });
-    for (const auto& z : w) t.push_back(rounded(z));
-    for (const auto& z : chirp) t.push_back(rounded(z));
-    for (const auto& z : hat) t.push_back(rounded(z / gain));
+    const Hcs<T> wr = rounded(w, real_size), cr = rounded(chirp, real_size), hr = rounded(hat, real_size);
+    const T gain = mean_gain<T>(
+        a.N, [&](const Hcs<T>& x) { return host_bluestein(kernel, a, x, wr, cr, hr); },
+        [&](const Hcs<T>& x) { return host_bluestein(exact, a, x, w, chirp, hat); });
+    for (const auto& z : w) put(z);
+    for (const auto& z : chirp) put(z);
+    for (const auto& z : hat) put(Hc<T>{z.r / gain, z.i / gain});
     return t;
 }
 
 std::vector<std::complex<double>> fft_axis_table(const FftAxis& a, size_t real_size) {
-    return real_size == sizeof(float) ? axis_table<float>(a) : axis_table<double>(a);
+    return real_size == sizeof(float) ? axis_table<double>(a, real_size) : axis_table<long double>(a, real_size);
 }
 
-template <typename real>
-static long double plan_gain(const FftPlan& p) {
-    const HostConstants<real> h;
-    const HostConstants<long double> he;
-    Lcs we, wr;
+template <class T>
+static double plan_gain(const FftPlan& p, size_t real_size) {
+    const HostConstants<T> exact(0), kernel(real_size);
+    Hcs<T> w, wr;
     for (int k = 0; k < p.len; k++) {
-        const std::complex<double> z = root<double>(k, p.len); /* as the table holds it */
-        we.push_back(to_real<long double>(root<long double>(k, p.len)));
-        wr.push_back(to_real<real>(cld(z.real(), z.imag())));
+        const Hc<double> z = root<double>(k, p.len); /* as the table holds it */
+        w.push_back(root<T>(k, p.len));
+        wr.push_back(rounded(Hc<T>{(T)z.r, (T)z.i}, real_size));
     }
-    return mean_gain(
-        p.len, [&](const Lcs& x) { return host_transform(h, p, x, wr); }, [&](const Lcs& x) { return host_transform(he, p, x, we); });
+    return (double)mean_gain<T>(
+        p.len, [&](const Hcs<T>& x) { return host_transform(kernel, p, x, wr); }, [&](const Hcs<T>& x) { return host_transform(exact, p, x, w); });
 }
 
 double fft_axis_gain(const FftAxis& a, bool columns, size_t real_size) {
     if (a.M || !a.fwd.passes || largest_prime(a.N) <= 2) return 1.0;
-    auto gain = [&](const FftPlan& p) { return real_size == sizeof(float) ? plan_gain<float>(p) : plan_gain<double>(p); };
-    return (double)(gain(a.fwd) * gain(columns ? a.inv : a.fwd));
+    auto gain = [&](const FftPlan& p) { return real_size == sizeof(float) ? plan_gain<double>(p, real_size) : plan_gain<long double>(p, real_size); };
+    const double g = gain(a.fwd);
+    return g * (columns ? gain(a.inv) : g);
 }
 
 template <typename real>
